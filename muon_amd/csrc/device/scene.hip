@@ -11,6 +11,7 @@
 
 #include "../common/vecmath.h"
 #include "bvh_device.h"
+#include "exact_div.h"
 #include "runtime.h"
 #include "wide_bvh.h"
 
@@ -356,6 +357,9 @@ extern "C" int muonx_scene_create(muonx_ctx *ctx, const muonx_scene_desc *din, m
   v.leaf_counts = leaf_counts ? 1u : 0u;
   v.root_leaf = root_leaf ? 1u : 0u;
   v.linear = (d->acceleration == 0 && root_leaf) ? 1u : 0u;
+  v.plain_planes = 1u;
+  for (size_t i = 0; i < size_t(nn) * 6; ++i)
+    if (!CoordinateOk(d->node_bounds[i])) v.plain_planes = 0u;
   v.light_prims = s->light_prims.as<uint32_t>();
   v.cull_mis = cull_mis ? 1u : 0u;
   {

@@ -512,7 +512,7 @@ __global__ void __launch_bounds__(kEngBlock) __attribute__((amdgpu_waves_per_eu(
   LaneTrace<WIDTH, false, COUNT> lt;
   DevSceneView sv;
   TraceCounters c;
-  WaveFetch wf(n);
+  WaveFetch<> wf(n);
   uint32_t i = 0, prim_rays = 0, sec_rays = 0;
   bool have = false, drained = false;
   while (true) {
@@ -566,7 +566,7 @@ __global__ void __launch_bounds__(kEngBlock) __attribute__((amdgpu_waves_per_eu(
   LaneTrace<WIDTH, true, COUNT> lt;
   DevSceneView sv;
   TraceCounters c;
-  WaveFetch wf(n);
+  WaveFetch<> wf(n);
   uint32_t sl = 0, traced = 0;
   bool have = false, drained = false;
   while (true) {
@@ -607,7 +607,7 @@ __global__ void __launch_bounds__(kEngBlock) __attribute__((amdgpu_waves_per_eu(
   LaneTrace<WIDTH, false, COUNT> lt;
   DevSceneView sv;
   TraceCounters c;
-  WaveFetch wf(n);
+  WaveFetch<> wf(n);
   uint32_t i = 0, traced = 0;
   bool have = false, drained = false;
   while (true) {
@@ -1077,7 +1077,7 @@ int Engine::AddScene(muonx_scene *scene, uint32_t *slot) {
     max_wstack_ = wstack;
     TraverseCfg cfg;
     const int rc = PlanTraverseInto(tuning_, num_cus_, max_depth_, max_wstack_, uint64_t(capacity_) * kmax_,
-                                    kEngBlock, spill_, cfg, false);
+                                    kEngBlock, spill_, cfg);
     if (rc != MUONX_OK) return rc;
     cfg_ = cfg;
   }

@@ -1,0 +1,210 @@
+// The exact traversal (the reference's node visits, box_hit_exact) as
+// resumable walks of a wavefront's lanes: what the exact queries and the
+// deterministic integrators run.
+#ifndef MUONX_DEVICE_EXACT_TRACE_H_
+#define MUONX_DEVICE_EXACT_TRACE_H_
+
+#include "trace.h"
+#include "wave.h"
+
+namespace muonx {
+
+// Stack of an exact walk: the newest kExactRing entries in LDS (lane
+// columns, conflict free), older ones in the lane's private memory. An exact
+// walk holds at most the binary tree's depth minus one entries, which
+// `private_old` (CAP - kExactRing entries) is sized for.
+constexpr int kExactRing = 8;
+template <int CAP>
+struct ExactStack {
+  static constexpr int kOld = CAP - kExactRing;
+  uint2 *base, *old;
+  int stride, sp = 0;
+  __device__ __forceinline__ ExactStack(uint2 *lds, int s, uint2 *private_old) : base(lds), old(private_old), stride(s) {}
+  __device__ __forceinline__ void reset() { sp = 0; }
+  __device__ __forceinline__ bool empty() const { return sp == 0; }
+  __device__ __forceinline__ void push(uint2 v) {
+    uint2 *slot = base + (sp & (kExactRing - 1)) * stride;
+    if (sp >= kExactRing) {
+      if (sp >= CAP) return;  // sized from the BVH depth: never taken
+      old[sp - kExactRing] = *slot;
+    }
+    *slot = v;
+    ++sp;
+  }
+  __device__ __forceinline__ uint2 pop() {
+    --sp;
+    uint2 *slot = base + (sp & (kExactRing - 1)) * stride;
+    const uint2 v = *slot;
+    if (sp >= kExactRing) *slot = old[sp - kExactRing];
+    return v;
+  }
+};
+
+// Which queries a walk answers: Intersect, HasIntersection, or either, as
+// start() is told.
+constexpr int kWalkClosest = 0, kWalkAny = 1, kWalkEither = 2;
+
+// One lane's walk. COUNT counts the reference's tests (TraceCounters).
+template <bool COUNT, int KIND>
+struct ExactWalk {
+  TraceRay r;
+  float best;
+  int32_t hit;   // leaf-order primitive or -1
+  uint32_t ref;  // the node or leaf to visit next
+  ObjCache oc;
+  bool plain, any_hit;
+
+  __device__ __forceinline__ bool any() const { return KIND == kWalkEither ? any_hit : KIND == kWalkAny; }
+  __device__ __forceinline__ bool at_leaf() const { return (ref & kLeafBit) != 0u; }
+  // Linear::HasIntersection counts nothing (muon/acceleration.cc:33-45).
+  __device__ __forceinline__ bool counts(const DevSceneView &s) const { return COUNT && !(s.linear && any()); }
+
+  // False when the walk is over at once (counting: the ray misses the root's box).
+  template <class Stack>
+  __device__ __forceinline__ bool start(const DevSceneView &s, const TraceRay &ray, float tmax, bool any_query,
+                                        Stack &st, TraceCounters &cnt) {
+    r = ray;
+    best = tmax;
+    hit = -1;
+    ref = 0;
+    oc.tid = -1;
+    any_hit = any_query;
+    plain = plain_ray(s, ray);
+    st.reset();
+    if (!counts(s)) return true;
+    const float4 *np = s.nodes;
+    if (s.linear) {
+      // Linear::Intersect tests every primitive and no bounds
+      // (muon/acceleration.cc:14-31): the one leaf is node 0's first child
+      ref = __float_as_uint(ldg(np + 3).x);
+      return true;
+    }
+    // The reference tests the root's box first (muon/acceleration.cc:92-99);
+    // here it is the union of node 0's child boxes. A ray that misses it
+    // misses every box below, so stopping changes no result. A root that is
+    // a leaf sits in node 0's first child (the second is a sentinel).
+    const float4 n0 = ldg(np), n1 = ldg(np + 1), n2 = ldg(np + 2);
+    float lo;
+    cnt.btests++;
+    if (!box_hit_exact(r, plain, fminf(n0.x, n1.x), fmaxf(n0.y, n1.y), fminf(n0.z, n1.z), fmaxf(n0.w, n1.w),
+                       fminf(n2.x, n2.z), fmaxf(n2.y, n2.w), best, lo))
+      return false;
+    cnt.bhits++;
+    if (s.root_leaf) ref = __float_as_uint(ldg(np + 3).x);
+    return true;
+  }
+
+  // The next stack entry whose box starts before `best`; false when there is
+  // none. Counting, every popped far child is the reference's bounds test at
+  // its pop.
+  template <class Stack>
+  __device__ __forceinline__ bool pop(const DevSceneView &s, Stack &st, TraceCounters &cnt) {
+    const bool count = counts(s);
+    while (!st.empty()) {
+      const uint2 e = st.pop();
+      if (count) cnt.btests++;
+      if (__uint_as_float(e.y) < best) {
+        if (count) cnt.bhits++;
+        ref = e.x;
+        return true;
+      }
+    }
+    return false;
+  }
+
+  // Visits the internal node `ref`, near child (reference order:
+  // children[dir[axis] < 0], muon/acceleration.cc:134-138) first; false when
+  // the walk is over.
+  template <class Stack>
+  __device__ __forceinline__ bool node(const DevSceneView &s, Stack &st, TraceCounters &cnt) {
+    const float4 *np = s.nodes + 4 * size_t(ref);
+    const float4 n0 = ldg(np), n1 = ldg(np + 1), n2 = ldg(np + 2);
+    const int4 n3 = ldg(reinterpret_cast<const int4 *>(np + 3));
+    const bool count = counts(s);
+    if (COUNT) cnt.nodes++;
+    float lo0, lo1;
+    const bool h0 = box_hit_exact(r, plain, n0.x, n0.y, n0.z, n0.w, n2.x, n2.y, best, lo0);
+    const bool h1 = box_hit_exact(r, plain, n1.x, n1.y, n1.z, n1.w, n2.z, n2.w, best, lo1);
+    const uint32_t axis = (uint32_t(n3.z) >> 29) & 3u;
+    const bool swap = (r.dneg >> axis) & 1u;  // near child is children[1]
+    const uint32_t near_ref = swap ? uint32_t(n3.y) : uint32_t(n3.x);
+    const uint32_t far_ref = swap ? uint32_t(n3.x) : uint32_t(n3.y);
+    const bool hn = swap ? h1 : h0;
+    const bool hf = swap ? h0 : h1;
+    const float lof = swap ? lo0 : lo1;
+    if (count) {
+      // The reference (muon/acceleration.cc:137,197) always pushes the far
+      // child and tests its box only when it pops it, which an any-hit query
+      // that stops at its first hit (:182-183) never does. So with the near
+      // box hit the far child is pushed too, with an infinite key when its
+      // box was missed here, and its test is counted at its pop; with the
+      // near box missed the far one is popped at once.
+      cnt.btests += hn ? 1u : 2u;
+      cnt.bhits += uint32_t(hn || hf);
+    }
+    if (hn) {
+      if (count || hf) st.push(make_uint2(far_ref, hf ? __float_as_uint(lof) : 0x7f800000u));
+      ref = near_ref;
+      return true;
+    }
+    if (hf) {
+      ref = far_ref;
+      return true;
+    }
+    return pop(s, st, cnt);
+  }
+
+  // Tests the primitives of the leaf `ref`; false when the walk is over.
+  template <class Stack>
+  __device__ __forceinline__ bool leaf(const DevSceneView &s, Stack &st, TraceCounters &cnt) {
+    const bool count = counts(s);
+    for (uint32_t i = ref & ~kLeafBit;; ++i) {
+      float dist;
+      uint32_t flags;
+      const bool ph = prim_hit(s, i, r, oc, dist, flags);
+      const bool closer = ph && dist > 0.0f && dist < best;
+      if (count) {
+        cnt.prims++;
+        // an object hit is Primitive::Intersect's (closest hit) or
+        // HasIntersection's (any hit: also 0 < dist < tmax), muon/objects.cc:9-17
+        if (any() ? closer : ph) cnt.ohits++;
+      }
+      if (closer) {
+        best = dist;
+        hit = int32_t(i);
+        if (any()) return false;
+      }
+      if (flags & 1u) break;
+    }
+    return pop(s, st, cnt);
+  }
+};
+
+// Advances the wavefront's walks (the lanes with `walking`) until at least
+// `stop` of its lanes have none, at least one step. Lanes step through
+// internal nodes together while at least kWalkNodeLanes of them (or all
+// that walk) are at one; then those at a leaf test its primitives. Every lane
+// makes its own walk's steps in order, whatever the others do. All 64 lanes
+// call it. With 8, 16, 24 and 32 node lanes 300,007 rays on the level-6
+// icosphere take 257 / 260 / 266 / 279 us, 200,000 any-hit rays on 5000
+// spheres 129 / 124 / 127 / 127 us.
+constexpr int kWalkNodeLanes = 16;
+template <class Walk, class Stack>
+__device__ __forceinline__ void run_walks(const DevSceneView &s, Walk &w, bool &walking, Stack &st,
+                                          TraceCounters &cnt, int stop) {
+  uint64_t active = __builtin_amdgcn_ballot_w64(walking);
+  do {
+    uint64_t nodes = __builtin_amdgcn_ballot_w64(walking && !w.at_leaf());
+    while (nodes && (__popcll(nodes) >= kWalkNodeLanes || nodes == active)) {
+      if (walking && !w.at_leaf()) walking = w.node(s, st, cnt);
+      active = __builtin_amdgcn_ballot_w64(walking);
+      nodes = __builtin_amdgcn_ballot_w64(walking && !w.at_leaf());
+    }
+    if (walking && w.at_leaf()) walking = w.leaf(s, st, cnt);
+    active = __builtin_amdgcn_ballot_w64(walking);
+  } while (active && 64 - __popcll(active) < stop);
+}
+
+}  // namespace muonx
+
+#endif

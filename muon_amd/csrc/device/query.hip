@@ -1,5 +1,6 @@
 // Batched closest-hit / any-hit queries over device-resident rays
 // (muonx_intersect_closest / muonx_intersect_any).
+#include "exact_trace.h"
 #include "query.h"
 #include "runtime.h"
 #include "trace.h"
@@ -11,7 +12,20 @@
 
 namespace muonx {
 
-template <int KIND, bool WW, int WIDTH, bool ANY, bool COUNT, bool EXACT>
+constexpr uint32_t kWavesPerBlock = kQueryBlock / 64;
+// chunks of at most 128 rays: 2^24 closest-hit rays over the level-7
+// icosphere trace in 3.245 ms against 3.285 ms with 256 (and 3.41 ms with
+// 512, 3.45 ms with 64); the engine's kernels keep 256, with which the
+// path-traced render of the same scene is 4 % faster than with 128
+constexpr uint32_t kQueryChunk = 128;
+
+// Blocks for n rays: no more than the wavefronts that get a first chunk.
+static uint32_t QueryGrid(uint32_t n, uint32_t max_blocks) {
+  const uint32_t chunk = ClaimChunk(n, max_blocks * kWavesPerBlock, kQueryChunk, true);
+  return std::max(1u, std::min(max_blocks, (n / chunk + kWavesPerBlock) / kWavesPerBlock));
+}
+
+template <int KIND, bool WW, int WIDTH, bool ANY, bool COUNT>
 __global__ void __launch_bounds__(kQueryBlock) k_query(DevSceneView s, StackArgs sa, const float *__restrict__ ro,
                                                        const float *__restrict__ rd, const float *__restrict__ tmax,
                                                        uint32_t n, int32_t *__restrict__ prim_out,
@@ -25,9 +39,7 @@ __global__ void __launch_bounds__(kQueryBlock) k_query(DevSceneView s, StackArgs
     float best = tmax ? tmax[i] : __builtin_inff();
     const TraceRay r = make_ray(o, d);
     auto st = make_stack<KIND>(lds, kQueryBlock, sa);
-    int32_t p;
-    if constexpr (EXACT) p = trace_bvh_s<ANY, COUNT, true, false>(s, r, best, st, cnt);
-    else p = trace_fast<WIDTH, ANY, COUNT, WW>(s, r, best, st, cnt);
+    const int32_t p = trace_fast<WIDTH, ANY, COUNT, WW>(s, r, best, st, cnt);
     if (ANY) {
       occ_out[i] = p >= 0 ? 1 : 0;
     } else {
@@ -64,11 +76,7 @@ __global__ void __launch_bounds__(kQueryBlock) __attribute__((amdgpu_waves_per_e
   auto st = make_stack<KIND>(lds, kQueryBlock, sa);
   LaneTrace<WIDTH, ANY, COUNT> lt;
   uint32_t idx = 0;
-  // chunks of at most 128 rays: 2^24 closest-hit rays over the level-7
-  // icosphere trace in 3.245 ms against 3.285 ms with 256 (and 3.41 ms with
-  // 512, 3.45 ms with 64); the engine's kernels keep 256, with which the
-  // path-traced render of the same scene is 4 % faster than with 128
-  WaveFetch wf(n, 128);
+  WaveFetch<> wf(n, kQueryChunk);
   bool have = false, drained = false;
   while (true) {
     const bool need = !have && !drained;
@@ -111,6 +119,63 @@ __global__ void __launch_bounds__(kQueryBlock) __attribute__((amdgpu_waves_per_e
   }
 }
 
+// Exact mode: the walks of a wavefront's lanes, each lane taking the next
+// unclaimed ray once kExactRefill of them are idle. Bound by instruction
+// issue (lanes 27-31 % used, 200 wavefront instructions per ray). Against one
+// ray per lane and grid step, a node or a leaf step per iteration and the
+// whole stack in LDS (three wavefronts per SIMD, now seven): 300,007
+// incoherent rays on the level-6 icosphere 361 -> 259 us, 10^6 on 10,000
+// spheres 1154 -> 391 us together with the reciprocal quotients. Refilling
+// at 16, 32 or 48 idle lanes measured the same.
+constexpr int kExactRefill = 32;
+template <int CAP, bool ANY, bool COUNT>
+__global__ void __launch_bounds__(kQueryBlock)
+    k_query_exact(DevSceneView s, const float *__restrict__ ro, const float *__restrict__ rd,
+                  const float *__restrict__ tmax, uint32_t n, int32_t *__restrict__ prim_out,
+                  float *__restrict__ t_out, uint8_t *__restrict__ occ_out, unsigned long long *__restrict__ counters,
+                  uint32_t *next) {
+  __shared__ uint2 lds[kExactRing * kQueryBlock];
+  uint2 old[ExactStack<CAP>::kOld];
+  ExactStack<CAP> st(lds + threadIdx.x, kQueryBlock, old);
+  ExactWalk<COUNT, ANY ? kWalkAny : kWalkClosest> w;
+  TraceCounters cnt;
+  WaveFetch<true> wf(n, kQueryChunk);
+  uint32_t idx = 0;
+  bool walking = false, have = false, drained = false;
+  while (true) {
+    const uint64_t needm = __builtin_amdgcn_ballot_w64(!have && !drained);
+    if (needm) {
+      const uint32_t k = wf.claim(needm, next);
+      if (!have && !drained) {
+        if (k < n) {
+          idx = k;
+          have = true;
+          const V3 o{ro[3 * k], ro[3 * k + 1], ro[3 * k + 2]};
+          const V3 d{rd[3 * k], rd[3 * k + 1], rd[3 * k + 2]};
+          walking = w.start(s, make_ray(o, d), tmax ? tmax[k] : __builtin_inff(), ANY, st, cnt);
+        } else {
+          drained = true;
+        }
+      }
+    }
+    if (__builtin_amdgcn_ballot_w64(have) == 0) break;
+    run_walks(s, w, walking, st, cnt, __builtin_amdgcn_ballot_w64(drained) ? 65 : kExactRefill);
+    if (have && !walking) {
+      have = false;
+      if (ANY) {
+        occ_out[idx] = w.hit >= 0 ? 1 : 0;
+      } else {
+        prim_out[idx] = w.hit >= 0 ? s.prim_id[w.hit] : -1;
+        if (t_out) t_out[idx] = w.hit >= 0 ? w.best : 0.0f;
+      }
+    }
+  }
+  if (COUNT) {
+    wave_count(cnt.nodes, &counters[0]);
+    wave_count(cnt.prims, &counters[1]);
+  }
+}
+
 namespace {
 template <bool ANY, bool COUNT>
 struct QueryDynLaunch {
@@ -133,7 +198,7 @@ struct QueryDynLaunch {
   }
 };
 
-template <bool ANY, bool COUNT, bool EXACT>
+template <bool ANY, bool COUNT>
 struct QueryLaunch {
   const TraverseCfg &cfg;
   const DevSceneView &s;
@@ -147,7 +212,7 @@ struct QueryLaunch {
   template <int KIND, bool WW, int WIDTH>
   void run() const {
     const StackArgs sa{cfg.spill, cfg.gcap};
-    hipLaunchKernelGGL((k_query<KIND, WW, WIDTH, ANY, COUNT, EXACT>), dim3(cfg.grid), dim3(kQueryBlock), 0, stream,
+    hipLaunchKernelGGL((k_query<KIND, WW, WIDTH, ANY, COUNT>), dim3(cfg.grid), dim3(kQueryBlock), 0, stream,
                        s, sa, ro, rd, tmax, n, prim, t, occ, counters);
   }
 };
@@ -191,6 +256,72 @@ int InitStaticScratch(int device) {
   return MUONX_OK;
 }
 
+// The claim counter of the per-lane fetch kernels, cleared on `stream`: in
+// the static scratch with `noalloc` (by a kernel rather than a memset node),
+// else in the context, ordered after its previous user like the spill region.
+static int ClearClaims(muonx_ctx *ctx, hipStream_t stream, bool noalloc, void *scratch_base, uint32_t **next) {
+  if (noalloc) {
+    *next = static_cast<uint32_t *>(scratch_base);
+    hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(1), 0, stream, *next);
+    return MUONX_OK;
+  }
+  MX_HIP(ctx->fetch_ctr.Reserve(sizeof(uint32_t)));
+  if (!ctx->spill_done) MX_HIP(hipEventCreateWithFlags(&ctx->spill_done, hipEventDisableTiming));
+  MX_HIP(hipStreamWaitEvent(stream, ctx->spill_done, 0));
+  MX_HIP(hipMemsetAsync(ctx->fetch_ctr.ptr, 0, sizeof(uint32_t), stream));
+  *next = ctx->fetch_ctr.as<uint32_t>();
+  return MUONX_OK;
+}
+
+// Exact mode: stacks in LDS and private memory, so the claim counter is the
+// only scratch, and a batch that the wavefronts' first chunks cover needs
+// none. 6, 8, 12 or 16 blocks per CU: 308 / 301 / 260 / 260 us for 300,007
+// rays on the level-6 icosphere.
+constexpr int kExactBlocksPerCu = 12;
+constexpr uint32_t kExactPart = 1u << 30;  // rays per launch: 3 * index stays below 2^32
+static int LaunchExactQuery(muonx_ctx *ctx, const DevSceneView &s, bool any, const float *ro, const float *rd,
+                            const float *tmax, uint32_t n, int32_t *prim, float *t, uint8_t *occ,
+                            unsigned long long *counters, hipStream_t stream, bool noalloc, void *scratch_base) {
+  if (s.bvh_depth > 96) {
+    SetError("BVH depth " + std::to_string(s.bvh_depth) + " exceeds the exact-mode traversal stack (96)");
+    return MUONX_ERR_CAPACITY;
+  }
+  for (uint32_t at = 0; at < n; at += std::min(n - at, kExactPart)) {
+    const uint32_t m = std::min(n - at, kExactPart);
+    const uint64_t cus = uint64_t(ctx->num_cus > 0 ? ctx->num_cus : 256);
+    const uint32_t grid = QueryGrid(m, uint32_t(cus) * kExactBlocksPerCu);
+    uint32_t *next = nullptr;
+    const bool claims = !CoveredByFirstChunks(m, grid * kWavesPerBlock, kQueryChunk);
+    if (claims) {
+      const int rc = ClearClaims(ctx, stream, noalloc, scratch_base, &next);
+      if (rc != MUONX_OK) return rc;
+    }
+    const float *o = ro + 3 * size_t(at), *d = rd + 3 * size_t(at), *tm = tmax ? tmax + at : nullptr;
+    int32_t *po = prim ? prim + at : nullptr;
+    float *to = t ? t + at : nullptr;
+    uint8_t *oo = occ ? occ + at : nullptr;
+#define MX_QX(CAP, A, C) \
+  hipLaunchKernelGGL((k_query_exact<CAP, A, C>), dim3(grid), dim3(kQueryBlock), 0, stream, s, o, d, tm, m, po, to, oo, \
+                     counters, next)
+#define MX_QXC(A, C) \
+  if (s.bvh_depth <= 24) MX_QX(24, A, C); \
+  else if (s.bvh_depth <= 48) MX_QX(48, A, C); \
+  else MX_QX(96, A, C)
+    if (any) {
+      MX_QXC(true, false);
+    } else if (counters) {
+      MX_QXC(false, true);
+    } else {
+      MX_QXC(false, false);
+    }
+#undef MX_QXC
+#undef MX_QX
+    MX_HIP(hipGetLastError());
+    if (claims && !noalloc) MX_HIP(hipEventRecord(ctx->spill_done, stream));
+  }
+  return MUONX_OK;
+}
+
 // Launches the query kernels. With `noalloc` the spill region and the claim
 // counter come from the static scratch (the grid is capped so that the spill
 // fits), the counter is cleared by a kernel rather than a memset node, and
@@ -208,7 +339,10 @@ int LaunchQuery(muonx_ctx *ctx, const DevSceneView &s, bool any, bool exact, con
       SetError("muonx_intersect_noalloc: no static scratch address for device " + std::to_string(ctx->device));
       return MUONX_ERR_STATE;
     }
-    rc = PlanTraverseShape(ctx->tuning, ctx->num_cus, s.bvh_depth, s.wstack, n, kQueryBlock, cfg, exact);
+  }
+  if (exact) return LaunchExactQuery(ctx, s, any, ro, rd, tmax, n, prim, t, occ, counters, stream, noalloc, sbase);
+  if (noalloc) {
+    rc = PlanTraverseShape(ctx->tuning, ctx->num_cus, s.bvh_depth, s.wstack, n, kQueryBlock, cfg);
     if (rc != MUONX_OK) return rc;
     if (cfg.gcap > 0) {
       const size_t per_block = size_t(kQueryBlock) * size_t(cfg.gcap) * sizeof(uint2);
@@ -224,27 +358,17 @@ int LaunchQuery(muonx_ctx *ctx, const DevSceneView &s, bool any, bool exact, con
       cfg.spill = reinterpret_cast<uint2 *>(sbase + kStaticScratchHead);
     }
   } else {
-    rc = PlanTraverse(ctx, s, n, kQueryBlock, exact, cfg);
+    rc = PlanTraverse(ctx, s, n, kQueryBlock, cfg);
     if (rc != MUONX_OK) return rc;
     if ((rc = BeginSpill(ctx, cfg, stream)) != MUONX_OK) return rc;
   }
-#define MX_Q(A, C, E) DispatchTraverse(cfg, QueryLaunch<A, C, E>{cfg, s, ro, rd, tmax, n, prim, t, occ, counters, stream})
-#define MX_QE(A, C) DispatchExact(cfg, QueryLaunch<A, C, true>{cfg, s, ro, rd, tmax, n, prim, t, occ, counters, stream})
+#define MX_Q(A, C) DispatchTraverse(cfg, QueryLaunch<A, C>{cfg, s, ro, rd, tmax, n, prim, t, occ, counters, stream})
   const bool cnt = counters != nullptr;
   const int fetch = ctx->tuning.ray_fetch;
-  if (!exact && fetch > 0 && n <= (1u << 31)) {  // the claim counter stays below 2^32 (n + chunk x waves)
-    // per-lane ray fetch; the claim counter is ordered like the spill region
+  if (fetch > 0 && n <= (1u << 31)) {  // the claim counter stays below 2^32 (n + chunk x waves)
+    // per-lane ray fetch
     uint32_t *next;
-    if (noalloc) {
-      next = reinterpret_cast<uint32_t *>(sbase);
-      hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(1), 0, stream, next);
-    } else {
-      MX_HIP(ctx->fetch_ctr.Reserve(sizeof(uint32_t)));
-      if (!ctx->spill_done) MX_HIP(hipEventCreateWithFlags(&ctx->spill_done, hipEventDisableTiming));
-      MX_HIP(hipStreamWaitEvent(stream, ctx->spill_done, 0));
-      MX_HIP(hipMemsetAsync(ctx->fetch_ctr.ptr, 0, sizeof(uint32_t), stream));
-      next = ctx->fetch_ctr.as<uint32_t>();
-    }
+    if ((rc = ClearClaims(ctx, stream, noalloc, sbase, &next)) != MUONX_OK) return rc;
 #define MX_QD(A, C) DispatchTraverse(cfg, QueryDynLaunch<A, C>{cfg, s, ro, rd, tmax, n, prim, t, occ, counters, next, fetch, stream})
     if (any) {
       if (cnt) MX_QD(true, true);
@@ -258,20 +382,14 @@ int LaunchQuery(muonx_ctx *ctx, const DevSceneView &s, bool any, bool exact, con
     if (!noalloc) MX_HIP(hipEventRecord(ctx->spill_done, stream));
     return MUONX_OK;
   }
-  if (exact) {
-    // exact mode: full LDS stack, one node or leaf step per iteration
-    if (any) MX_QE(true, false);
-    else if (cnt) MX_QE(false, true);
-    else MX_QE(false, false);
-  } else if (any) {
-    if (cnt) MX_Q(true, true, false);
-    else MX_Q(true, false, false);
+  if (any) {
+    if (cnt) MX_Q(true, true);
+    else MX_Q(true, false);
   } else {
-    if (cnt) MX_Q(false, true, false);
-    else MX_Q(false, false, false);
+    if (cnt) MX_Q(false, true);
+    else MX_Q(false, false);
   }
 #undef MX_Q
-#undef MX_QE
   MX_HIP(hipGetLastError());
   return noalloc ? MUONX_OK : EndSpill(ctx, cfg, stream);
 }

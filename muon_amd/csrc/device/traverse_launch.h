@@ -59,51 +59,45 @@ __device__ __forceinline__ typename StackOf<KIND>::T make_stack(uint2 *lds, int 
 // deterministic modes are not performance-critical and keep the simplest
 // form). Allocates nothing.
 inline int PlanTraverseShape(const muonx_tuning &t, int num_cus, uint32_t bvh_depth, uint32_t wstack,
-                             uint64_t work_items, int block, TraverseCfg &cfg, bool want_exact = false) {
+                             uint64_t work_items, int block, TraverseCfg &cfg) {
   const int cus = num_cus > 0 ? num_cus : 256;
-  cfg.width = want_exact || t.bvh_width != 4 ? kNodesBinary : (t.node_bits == 8 ? kNodesWideQ : kNodesWide);
+  cfg.width = t.bvh_width != 4 ? kNodesBinary : (t.node_bits == 8 ? kNodesWideQ : kNodesWide);
   const int bpc = std::max(1, t.blocks_per_cu);
   cfg.grid = int(std::max<uint64_t>(1, std::min<uint64_t>(uint64_t(cus) * bpc, (work_items + block - 1) / block)));
   cfg.threads = cfg.grid * block;
-  cfg.ww = t.while_while != 0 && !want_exact;
+  cfg.ww = t.while_while != 0;
   cfg.spill = nullptr;
   cfg.gcap = 0;
   // binary: entries never exceed depth - 1; wide: the collapse's bound
   const int need = int(cfg.width != kNodesBinary ? std::max<uint32_t>(wstack, 1) : bvh_depth);
-  const bool ring = !want_exact && (t.stack_entries == 8 || t.stack_entries == 16);
+  const bool ring = t.stack_entries == 8 || t.stack_entries == 16;
   if (ring && need <= t.stack_entries) {
     cfg.kind = need <= 8 ? 8 : 16;  // a ring that never spills
     return MUONX_OK;
   }
-  if (ring || (!want_exact && need > 96)) {
+  if (ring || need > 96) {
     cfg.kind = ring ? t.stack_entries : 16;
     cfg.gcap = need - cfg.kind;
     return MUONX_OK;
   }
   if (need <= 24) cfg.kind = 24;
   else if (need <= 48) cfg.kind = 48;
-  else if (need <= 96) cfg.kind = 96;
-  else {
-    SetError("BVH depth " + std::to_string(need) + " exceeds the exact-mode traversal stack (96)");
-    return MUONX_ERR_CAPACITY;
-  }
+  else cfg.kind = 96;
   return MUONX_OK;
 }
 
 // PlanTraverseShape, then reserves the spill region in `spill`.
 inline int PlanTraverseInto(const muonx_tuning &t, int num_cus, uint32_t bvh_depth, uint32_t wstack,
-                            uint64_t work_items, int block, DevBuf &spill, TraverseCfg &cfg, bool want_exact = false) {
-  const int rc = PlanTraverseShape(t, num_cus, bvh_depth, wstack, work_items, block, cfg, want_exact);
+                            uint64_t work_items, int block, DevBuf &spill, TraverseCfg &cfg) {
+  const int rc = PlanTraverseShape(t, num_cus, bvh_depth, wstack, work_items, block, cfg);
   if (rc != MUONX_OK || cfg.gcap == 0) return rc;
   MX_HIP(spill.Reserve(size_t(cfg.threads) * cfg.gcap * sizeof(uint2)));
   cfg.spill = spill.as<uint2>();
   return MUONX_OK;
 }
 
-inline int PlanTraverse(muonx_ctx *ctx, const DevSceneView &s, uint64_t work_items, int block, bool want_exact,
-                        TraverseCfg &cfg) {
-  return PlanTraverseInto(ctx->tuning, ctx->num_cus, s.bvh_depth, s.wstack, work_items, block, ctx->spill, cfg,
-                          want_exact);
+inline int PlanTraverse(muonx_ctx *ctx, const DevSceneView &s, uint64_t work_items, int block, TraverseCfg &cfg) {
+  return PlanTraverseInto(ctx->tuning, ctx->num_cus, s.bvh_depth, s.wstack, work_items, block, ctx->spill, cfg);
 }
 
 // Kernels that use the spill region wait for its previous user when issued
@@ -137,16 +131,6 @@ inline void DispatchTraverse(const TraverseCfg &cfg, F &&f) {
   else if (cfg.width == kNodesWide) DispatchKind<kNodesWide>(cfg, f);
   else DispatchKind<kNodesBinary>(cfg, f);
 }
-// Exact mode: binary nodes, full LDS stack, if-if loop.
-template <class F>
-inline void DispatchExact(const TraverseCfg &cfg, F &&f) {
-  switch (cfg.kind) {
-    case 24: f.template run<24, false, 2>(); break;
-    case 48: f.template run<48, false, 2>(); break;
-    default: f.template run<96, false, 2>(); break;
-  }
-}
-
 }  // namespace muonx
 
 #endif

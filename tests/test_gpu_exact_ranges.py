@@ -55,3 +55,19 @@ def test_exact_mode_everywhere(ctx, oracle, kind, tiny_plane):
     assert hit.any() and np.array_equal(t.cpu().numpy()[hit].view(np.uint32), tr[hit].view(np.uint32))
     oref, _ = orc.occluded(o, d, tm)
     assert np.array_equal(occ.cpu().numpy() != 0, oref != 0)
+
+
+@pytest.mark.parametrize("n", [1, 2, 129, 4097, 131073, 500009])
+def test_exact_mode_batch_sizes(ctx, oracle, n):
+    """From two rays to a wavefront, over all first chunks filled, to chunks
+    claimed from the counter (past 393,216 rays on 256 CUs)."""
+    text = scenes.icosphere_text(64, 64, 1, 2, level=3)
+    ds = DeviceScene(ctx, HostScene.from_text(text))
+    orc = oracle.load_text(text)
+    o, d = scenes.microbench_rays(n, (-0.5, 0.1, -0.5), (0.5, 1.1, 0.5), seed=n)
+    pr, tr, _, _, _ = orc.intersect(o, d)
+    prim, t = ds.intersect_closest(torch.from_numpy(o).cuda(), torch.from_numpy(d).cuda(), exact=True)
+    torch.cuda.synchronize()
+    assert np.array_equal(prim.cpu().numpy(), pr)
+    hit = pr >= 0
+    assert np.array_equal(t.cpu().numpy()[hit].view(np.uint32), tr[hit].view(np.uint32))

@@ -207,8 +207,9 @@ void muonx_ctx_destroy(muonx_ctx *ctx);
 
 /* Launch tuning of a context (no counterpart in the reference, whose only
  * knob is --parallelism). Traversal stack: 0 = whole stack in LDS (capacity
- * from the BVH depth); 8 or 16 = LDS ring of that many entries per lane with
- * older entries spilled to a per-thread HBM region (more waves per CU).
+ * from the BVH depth); 8 or 16 = LDS ring of that many entries per lane (more
+ * waves per CU) with older entries in the lane's private memory (8, up to 72
+ * entries) or spilled to a per-thread HBM region (16, or deeper trees).
  * while_while: lanes walk internal nodes until each holds a leaf, then test
  * leaves together. blocks_per_cu: persistent grid size. path_budget_mb:
  * HBM for the path tracer's per-path state and queues. bvh_width: node

@@ -91,7 +91,7 @@ extern "C" int muonx_autotune(muonx_scene *scene, const muonx_render_params *job
       for (int stack : {8, 16, 0})
         for (int ww : {1, 0})
           for (int bpc : {8, 16, 24})
-            for (int fetch : {0, 32, 48}) {
+            for (int fetch : {0, 16, 32}) {
               if (fetch > 0 && ww == 0) continue;  // the fetch kernels always walk while-while
               if (width == 2 && bits == 8) continue;  // quantized boxes exist for 4-wide nodes
               muonx_tuning c = base;
@@ -143,7 +143,7 @@ extern "C" int muonx_autotune(muonx_scene *scene, const muonx_render_params *job
     // the engine's launch settings on the job: node precision, fetch
     // threshold, grid, capacity
     for (int bits : {32, 8})
-    for (int fetch : {0, 48})
+    for (int fetch : {0, 16})
       for (int bpc : {16, 24})
         for (int mb : {2048, 8192}) {
           muonx_tuning c = tuned;

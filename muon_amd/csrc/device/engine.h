@@ -32,6 +32,7 @@
 #include "render.h"
 #include "runtime.h"
 #include "traverse_launch.h"
+#include "wave.h"
 
 namespace muonx {
 
@@ -90,11 +91,13 @@ struct alignas(256) HotCounter64 {
 };
 constexpr int kRaySlots = 16;  // partial ray counts per counter, blocks spread over them
 
+static_assert(sizeof(HotCounter) == kClaimStride * sizeof(uint32_t), "claim counters are HotCounters");
+
 struct EngCounters {
   HotCounter qcount[2];  // path queues
   HotCounter mis_count;
   HotCounter shadow_count;
-  HotCounter claim[3];   // work claimed by the per-lane-fetch extend / shadow / mis kernels
+  HotCounter claim[3][kClaimGroups];  // work claimed by the per-lane-fetch extend / shadow / mis kernels
   uint32_t plan_n, plan_base;
   unsigned long long plan_cursor;
   unsigned long long cursor;          // next work item to generate

@@ -37,6 +37,7 @@ __device__ __forceinline__ void work_count(EngCounters *c, const TraceCounters &
 template <int KIND, bool WW, int WIDTH, bool COUNT>
 __global__ void __launch_bounds__(kEngBlock) k_eng_extend(EngArgs a, StackArgs sa, int cur) {
   __shared__ uint2 lds[StackOf<KIND>::kLds * kEngBlock];
+  uint2 old[StackOf<KIND>::kPrivate];
   const uint32_t n = a.c->qcount[cur].v;
   const float4 *q = a.q_ray[cur];
   const PathState &ps = a.st[cur];
@@ -56,7 +57,7 @@ __global__ void __launch_bounds__(kEngBlock) k_eng_extend(EngArgs a, StackArgs s
         const DevSceneView sv = a.scenes[PathSceneSlot(jw)];
         const TraceRay r = make_ray(V3{qo.x, qo.y, qo.z}, V3{qd.x, qd.y, qd.z});
         float best = __builtin_inff();
-        auto st = make_stack<KIND>(lds, kEngBlock, sa);
+        auto st = make_stack<KIND>(lds, kEngBlock, sa, old);
         hit = trace_fast<WIDTH, false, COUNT, WW>(sv, r, best, st, c);
         if (depth == 0) ++prim_rays;
         else ++sec_rays;
@@ -449,6 +450,7 @@ __global__ void __launch_bounds__(kShadeBlock) __attribute__((amdgpu_waves_per_e
 template <int KIND, bool WW, int WIDTH, bool COUNT>
 __global__ void __launch_bounds__(kEngBlock) k_eng_shadow(EngArgs a, StackArgs sa, int cur) {
   __shared__ uint2 lds[StackOf<KIND>::kLds * kEngBlock];
+  uint2 old[StackOf<KIND>::kPrivate];
   const uint32_t P = a.capacity;
   const uint32_t n = a.c->shadow_count.v;
   const PathState &ps = a.st[cur];
@@ -463,7 +465,7 @@ __global__ void __launch_bounds__(kEngBlock) k_eng_shadow(EngArgs a, StackArgs s
       const float4 so = a.shift[i], sd = a.s_dir[sl];
       const TraceRay r = make_ray(V3{so.x, so.y, so.z}, V3{sd.x, sd.y, sd.z});
       float best = sd.w;
-      auto st = make_stack<KIND>(lds, kEngBlock, sa);
+      auto st = make_stack<KIND>(lds, kEngBlock, sa, old);
       const int32_t hit = trace_fast<WIDTH, true, COUNT, WW>(sv, r, best, st, c);
       a.s_vis[sl] = hit < 0 ? 1 : 0;
       ++traced;
@@ -477,6 +479,7 @@ __global__ void __launch_bounds__(kEngBlock) k_eng_shadow(EngArgs a, StackArgs s
 template <int KIND, bool WW, int WIDTH, bool COUNT>
 __global__ void __launch_bounds__(kEngBlock) k_eng_mis(EngArgs a, StackArgs sa, int cur) {
   __shared__ uint2 lds[StackOf<KIND>::kLds * kEngBlock];
+  uint2 old[StackOf<KIND>::kPrivate];
   const uint32_t n = a.c->mis_count.v;
   const PathState &ps = a.st[cur];
   uint32_t traced = 0;
@@ -489,7 +492,7 @@ __global__ void __launch_bounds__(kEngBlock) k_eng_mis(EngArgs a, StackArgs sa, 
       const DevSceneView s = a.scenes[PathSceneSlot(ps.job[i])];
       const TraceRay r = make_ray(V3{mo.x, mo.y, mo.z}, V3{md.x, md.y, md.z});
       float best = md.w;  // the nearest emitter hit, or +inf
-      auto st = make_stack<KIND>(lds, kEngBlock, sa);
+      auto st = make_stack<KIND>(lds, kEngBlock, sa, old);
       a.m_hit[i] = trace_fast<WIDTH, false, COUNT, WW>(s, r, best, st, c);
       ++traced;
     }
@@ -505,22 +508,22 @@ __global__ void __launch_bounds__(kEngBlock) k_eng_mis(EngArgs a, StackArgs sa, 
 template <int KIND, int WIDTH, bool COUNT>
 __global__ void __launch_bounds__(kEngBlock) __attribute__((amdgpu_waves_per_eu(7, 8))) k_eng_extend_dyn(EngArgs a, StackArgs sa, int cur, int fetch_min) {
   __shared__ uint2 lds[StackOf<KIND>::kLds * kEngBlock];
+  uint2 old[StackOf<KIND>::kPrivate];
   const uint32_t n = a.c->qcount[cur].v;
   const float4 *q = a.q_ray[cur];
   const PathState &ps = a.st[cur];
-  auto st = make_stack<KIND>(lds, kEngBlock, sa);
+  auto st = make_stack<KIND>(lds, kEngBlock, sa, old);
   LaneTrace<WIDTH, false, COUNT> lt;
   DevSceneView sv;
   TraceCounters c;
-  WaveFetch<> wf(n);
+  WaveFetch wf(n);
   uint32_t i = 0, prim_rays = 0, sec_rays = 0;
-  bool have = false, drained = false;
+  bool walking = false, have = false, drained = false;
   while (true) {
-    const bool need = !have && !drained;
-    const uint64_t needm = __ballot(need);
-    if (needm && (__popcll(needm) >= fetch_min || __ballot(have) == 0)) {
-      const uint32_t k = wf.claim(needm, &a.c->claim[0].v);
-      if (need) {
+    const uint64_t needm = __builtin_amdgcn_ballot_w64(!have && !drained);
+    if (needm) {
+      const uint32_t k = wf.claim(needm, &a.c->claim[0][0].v);
+      if (!have && !drained) {
         if (k < n) {
           i = k;
           const uint32_t jw = ps.job[i], js = PathJobSlot(jw);
@@ -533,20 +536,20 @@ __global__ void __launch_bounds__(kEngBlock) __attribute__((amdgpu_waves_per_eu(
           sv = a.scenes[PathSceneSlot(jw)];
           lt.start(make_ray(V3{qo.x, qo.y, qo.z}, V3{qd.x, qd.y, qd.z}), __builtin_inff(), st);
           // Integrator::Trace returns 0 past the depth cutoff (muon/integration.cc:29-33)
-          if (depth <= a.jobs[js].cutoff && depth < kMaxBounces) {
-            have = true;
+          have = true;
+          walking = depth <= a.jobs[js].cutoff && depth < kMaxBounces;
+          if (walking) {
             if (depth == 0) ++prim_rays;
             else ++sec_rays;
-          } else {
-            a.hit_prim[i] = -1;
           }
         } else {
           drained = true;
         }
       }
     }
-    if (__ballot(have) == 0) break;
-    if (have && lt.round(sv, st, c)) {
+    if (__builtin_amdgcn_ballot_w64(have) == 0) break;
+    run_walks(sv, lt, walking, st, c, __builtin_amdgcn_ballot_w64(drained) ? 65 : fetch_min);
+    if (have && !walking) {
       a.hit_prim[i] = lt.hit;
       have = false;
     }
@@ -559,37 +562,38 @@ __global__ void __launch_bounds__(kEngBlock) __attribute__((amdgpu_waves_per_eu(
 template <int KIND, int WIDTH, bool COUNT>
 __global__ void __launch_bounds__(kEngBlock) __attribute__((amdgpu_waves_per_eu(7, 8))) k_eng_shadow_dyn(EngArgs a, StackArgs sa, int cur, int fetch_min) {
   __shared__ uint2 lds[StackOf<KIND>::kLds * kEngBlock];
+  uint2 old[StackOf<KIND>::kPrivate];
   const uint32_t P = a.capacity;
   const uint32_t n = a.c->shadow_count.v;
   const PathState &ps = a.st[cur];
-  auto st = make_stack<KIND>(lds, kEngBlock, sa);
+  auto st = make_stack<KIND>(lds, kEngBlock, sa, old);
   LaneTrace<WIDTH, true, COUNT> lt;
   DevSceneView sv;
   TraceCounters c;
-  WaveFetch<> wf(n);
+  WaveFetch wf(n);
   uint32_t sl = 0, traced = 0;
-  bool have = false, drained = false;
+  bool walking = false, have = false, drained = false;
   while (true) {
-    const bool need = !have && !drained;
-    const uint64_t needm = __ballot(need);
-    if (needm && (__popcll(needm) >= fetch_min || __ballot(have) == 0)) {
-      const uint32_t k = wf.claim(needm, &a.c->claim[1].v);
-      if (need) {
+    const uint64_t needm = __builtin_amdgcn_ballot_w64(!have && !drained);
+    if (needm) {
+      const uint32_t k = wf.claim(needm, &a.c->claim[1][0].v);
+      if (!have && !drained) {
         if (k < n) {
           sl = a.s_queue[k];
           const uint32_t i = sl % P;
           sv = a.scenes[PathSceneSlot(ps.job[i])];
           const float4 so = a.shift[i], sd = a.s_dir[sl];
           lt.start(make_ray(V3{so.x, so.y, so.z}, V3{sd.x, sd.y, sd.z}), sd.w, st);
-          have = true;
+          walking = have = true;
           ++traced;
         } else {
           drained = true;
         }
       }
     }
-    if (__ballot(have) == 0) break;
-    if (have && lt.round(sv, st, c)) {
+    if (__builtin_amdgcn_ballot_w64(have) == 0) break;
+    run_walks(sv, lt, walking, st, c, __builtin_amdgcn_ballot_w64(drained) ? 65 : fetch_min);
+    if (have && !walking) {
       a.s_vis[sl] = lt.hit < 0 ? 1 : 0;
       have = false;
     }
@@ -601,35 +605,36 @@ __global__ void __launch_bounds__(kEngBlock) __attribute__((amdgpu_waves_per_eu(
 template <int KIND, int WIDTH, bool COUNT>
 __global__ void __launch_bounds__(kEngBlock) __attribute__((amdgpu_waves_per_eu(7, 8))) k_eng_mis_dyn(EngArgs a, StackArgs sa, int cur, int fetch_min) {
   __shared__ uint2 lds[StackOf<KIND>::kLds * kEngBlock];
+  uint2 old[StackOf<KIND>::kPrivate];
   const uint32_t n = a.c->mis_count.v;
   const PathState &ps = a.st[cur];
-  auto st = make_stack<KIND>(lds, kEngBlock, sa);
+  auto st = make_stack<KIND>(lds, kEngBlock, sa, old);
   LaneTrace<WIDTH, false, COUNT> lt;
   DevSceneView sv;
   TraceCounters c;
-  WaveFetch<> wf(n);
+  WaveFetch wf(n);
   uint32_t i = 0, traced = 0;
-  bool have = false, drained = false;
+  bool walking = false, have = false, drained = false;
   while (true) {
-    const bool need = !have && !drained;
-    const uint64_t needm = __ballot(need);
-    if (needm && (__popcll(needm) >= fetch_min || __ballot(have) == 0)) {
-      const uint32_t k = wf.claim(needm, &a.c->claim[2].v);
-      if (need) {
+    const uint64_t needm = __builtin_amdgcn_ballot_w64(!have && !drained);
+    if (needm) {
+      const uint32_t k = wf.claim(needm, &a.c->claim[2][0].v);
+      if (!have && !drained) {
         if (k < n) {
           const float4 mo = a.m_ray[2 * k], md = a.m_ray[2 * k + 1];
           i = __float_as_uint(mo.w);
           sv = a.scenes[PathSceneSlot(ps.job[i])];
           lt.start(make_ray(V3{mo.x, mo.y, mo.z}, V3{md.x, md.y, md.z}), md.w, st);
-          have = true;
+          walking = have = true;
           ++traced;
         } else {
           drained = true;
         }
       }
     }
-    if (__ballot(have) == 0) break;
-    if (have && lt.round(sv, st, c)) {
+    if (__builtin_amdgcn_ballot_w64(have) == 0) break;
+    run_walks(sv, lt, walking, st, c, __builtin_amdgcn_ballot_w64(drained) ? 65 : fetch_min);
+    if (have && !walking) {
       a.m_hit[i] = lt.hit;  // retire adds the weighted emission when it is a light
       have = false;
     }
@@ -747,11 +752,11 @@ __global__ void k_eng_plan(EngArgs a, int cur) {
     for (int off = 32; off > 0; off >>= 1) v[id] += __shfl_down(v[id], off);
     if (lane == 0) c->rays[id] = tot[id] + v[id];
   }
+  if (lane < 3 * int(kClaimGroups)) c->claim[lane / kClaimGroups][lane % kClaimGroups].v = 0;
   if (lane != 0) return;
   c->qcount[cur].v = 0;
   c->mis_count.v = 0;
   c->shadow_count.v = 0;
-  c->claim[0].v = c->claim[1].v = c->claim[2].v = 0;
   const uint32_t next = c->qcount[cur ^ 1].v;
   const uint32_t nfill = FillCount(c->total_items, c->cursor, a.capacity, next);
   c->plan_n = nfill;

@@ -5,46 +5,15 @@
 #define MUONX_DEVICE_EXACT_TRACE_H_
 
 #include "trace.h"
-#include "wave.h"
 
 namespace muonx {
-
-// Stack of an exact walk: the newest kExactRing entries in LDS (lane
-// columns, conflict free), older ones in the lane's private memory. An exact
-// walk holds at most the binary tree's depth minus one entries, which
-// `private_old` (CAP - kExactRing entries) is sized for.
-constexpr int kExactRing = 8;
-template <int CAP>
-struct ExactStack {
-  static constexpr int kOld = CAP - kExactRing;
-  uint2 *base, *old;
-  int stride, sp = 0;
-  __device__ __forceinline__ ExactStack(uint2 *lds, int s, uint2 *private_old) : base(lds), old(private_old), stride(s) {}
-  __device__ __forceinline__ void reset() { sp = 0; }
-  __device__ __forceinline__ bool empty() const { return sp == 0; }
-  __device__ __forceinline__ void push(uint2 v) {
-    uint2 *slot = base + (sp & (kExactRing - 1)) * stride;
-    if (sp >= kExactRing) {
-      if (sp >= CAP) return;  // sized from the BVH depth: never taken
-      old[sp - kExactRing] = *slot;
-    }
-    *slot = v;
-    ++sp;
-  }
-  __device__ __forceinline__ uint2 pop() {
-    --sp;
-    uint2 *slot = base + (sp & (kExactRing - 1)) * stride;
-    const uint2 v = *slot;
-    if (sp >= kExactRing) *slot = old[sp - kExactRing];
-    return v;
-  }
-};
 
 // Which queries a walk answers: Intersect, HasIntersection, or either, as
 // start() is told.
 constexpr int kWalkClosest = 0, kWalkAny = 1, kWalkEither = 2;
 
-// One lane's walk. COUNT counts the reference's tests (TraceCounters).
+// One lane's walk. COUNT counts the reference's tests (TraceCounters). It
+// holds at most the binary tree's depth minus one stack entries.
 template <bool COUNT, int KIND>
 struct ExactWalk {
   TraceRay r;
@@ -179,31 +148,6 @@ struct ExactWalk {
     return pop(s, st, cnt);
   }
 };
-
-// Advances the wavefront's walks (the lanes with `walking`) until at least
-// `stop` of its lanes have none, at least one step. Lanes step through
-// internal nodes together while at least kWalkNodeLanes of them (or all
-// that walk) are at one; then those at a leaf test its primitives. Every lane
-// makes its own walk's steps in order, whatever the others do. All 64 lanes
-// call it. With 8, 16, 24 and 32 node lanes 300,007 rays on the level-6
-// icosphere take 257 / 260 / 266 / 279 us, 200,000 any-hit rays on 5000
-// spheres 129 / 124 / 127 / 127 us.
-constexpr int kWalkNodeLanes = 16;
-template <class Walk, class Stack>
-__device__ __forceinline__ void run_walks(const DevSceneView &s, Walk &w, bool &walking, Stack &st,
-                                          TraceCounters &cnt, int stop) {
-  uint64_t active = __builtin_amdgcn_ballot_w64(walking);
-  do {
-    uint64_t nodes = __builtin_amdgcn_ballot_w64(walking && !w.at_leaf());
-    while (nodes && (__popcll(nodes) >= kWalkNodeLanes || nodes == active)) {
-      if (walking && !w.at_leaf()) walking = w.node(s, st, cnt);
-      active = __builtin_amdgcn_ballot_w64(walking);
-      nodes = __builtin_amdgcn_ballot_w64(walking && !w.at_leaf());
-    }
-    if (walking && w.at_leaf()) walking = w.leaf(s, st, cnt);
-    active = __builtin_amdgcn_ballot_w64(walking);
-  } while (active && 64 - __popcll(active) < stop);
-}
 
 }  // namespace muonx
 

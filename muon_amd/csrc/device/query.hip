@@ -13,16 +13,11 @@
 namespace muonx {
 
 constexpr uint32_t kWavesPerBlock = kQueryBlock / 64;
-// chunks of at most 128 rays: 2^24 closest-hit rays over the level-7
-// icosphere trace in 3.245 ms against 3.285 ms with 256 (and 3.41 ms with
-// 512, 3.45 ms with 64); the engine's kernels keep 256, with which the
-// path-traced render of the same scene is 4 % faster than with 128
-constexpr uint32_t kQueryChunk = 128;
-
-// Blocks for n rays: no more than the wavefronts that get a first chunk.
+// Blocks for n rays: as many as hold a wavefront with a first chunk, at most
+// max_blocks.
 static uint32_t QueryGrid(uint32_t n, uint32_t max_blocks) {
-  const uint32_t chunk = ClaimChunk(n, max_blocks * kWavesPerBlock, kQueryChunk, true);
-  return std::max(1u, std::min(max_blocks, (n / chunk + kWavesPerBlock) / kWavesPerBlock));
+  const uint64_t waves = uint64_t(n) / FirstChunk(n, max_blocks * kWavesPerBlock) + 1;
+  return uint32_t(std::min<uint64_t>(max_blocks, (waves + kWavesPerBlock - 1) / kWavesPerBlock));
 }
 
 template <int KIND, bool WW, int WIDTH, bool ANY, bool COUNT>
@@ -32,13 +27,14 @@ __global__ void __launch_bounds__(kQueryBlock) k_query(DevSceneView s, StackArgs
                                                        float *__restrict__ t_out, uint8_t *__restrict__ occ_out,
                                                        unsigned long long *__restrict__ counters) {
   __shared__ uint2 lds[StackOf<KIND>::kLds * kQueryBlock];
+  uint2 old[StackOf<KIND>::kPrivate];
   TraceCounters cnt{0, 0};
   for (uint32_t i = blockIdx.x * kQueryBlock + threadIdx.x; i < n; i += gridDim.x * kQueryBlock) {
     const V3 o{ro[3 * i], ro[3 * i + 1], ro[3 * i + 2]};
     const V3 d{rd[3 * i], rd[3 * i + 1], rd[3 * i + 2]};
     float best = tmax ? tmax[i] : __builtin_inff();
     const TraceRay r = make_ray(o, d);
-    auto st = make_stack<KIND>(lds, kQueryBlock, sa);
+    auto st = make_stack<KIND>(lds, kQueryBlock, sa, old);
     const int32_t p = trace_fast<WIDTH, ANY, COUNT, WW>(s, r, best, st, cnt);
     if (ANY) {
       occ_out[i] = p >= 0 ? 1 : 0;
@@ -64,7 +60,6 @@ __global__ void __launch_bounds__(kQueryBlock) k_query(DevSceneView s, StackArgs
 // Fast mode with per-lane ray fetch: a lane whose ray is finished takes the
 // next unclaimed ray once at least `fetch_min` lanes of its wavefront are
 // idle, so long rays no longer hold idle lanes (claims: WaveFetch).
-
 template <int KIND, int WIDTH, bool ANY, bool COUNT>
 __global__ void __launch_bounds__(kQueryBlock) __attribute__((amdgpu_waves_per_eu(8, 8)))
     k_query_dyn(DevSceneView s, StackArgs sa, const float *__restrict__ ro, const float *__restrict__ rd,
@@ -72,50 +67,44 @@ __global__ void __launch_bounds__(kQueryBlock) __attribute__((amdgpu_waves_per_e
                 uint8_t *__restrict__ occ_out, unsigned long long *__restrict__ counters, uint32_t *next,
                 int fetch_min) {
   __shared__ uint2 lds[StackOf<KIND>::kLds * kQueryBlock];
+  uint2 old[StackOf<KIND>::kPrivate];
   TraceCounters cnt{0, 0};
-  auto st = make_stack<KIND>(lds, kQueryBlock, sa);
+  auto st = make_stack<KIND>(lds, kQueryBlock, sa, old);
   LaneTrace<WIDTH, ANY, COUNT> lt;
   uint32_t idx = 0;
-  WaveFetch<> wf(n, kQueryChunk);
-  bool have = false, drained = false;
+  WaveFetch wf(n, kChunk);
+  bool walking = false, have = false, drained = false;
   while (true) {
-    const bool need = !have && !drained;
-    const uint64_t needm = __ballot(need);
-    if (needm && (__popcll(needm) >= fetch_min || __ballot(have) == 0)) {
+    const uint64_t needm = __builtin_amdgcn_ballot_w64(!have && !drained);
+    if (needm) {
       const uint32_t k = wf.claim(needm, next);
-      if (need) {
+      if (!have && !drained) {
         if (k < n) {
           idx = k;
           const V3 o{ro[3 * k], ro[3 * k + 1], ro[3 * k + 2]};
           const V3 d{rd[3 * k], rd[3 * k + 1], rd[3 * k + 2]};
           lt.start(make_ray(o, d), tmax ? tmax[k] : __builtin_inff(), st);
-          have = true;
+          walking = have = true;
         } else {
           drained = true;
         }
       }
     }
-    if (__ballot(have) == 0) break;
-    if (have && lt.round(s, st, cnt)) {
+    if (__builtin_amdgcn_ballot_w64(have) == 0) break;
+    run_walks(s, lt, walking, st, cnt, __builtin_amdgcn_ballot_w64(drained) ? 65 : fetch_min);
+    if (have && !walking) {
+      have = false;
       if (ANY) {
         occ_out[idx] = lt.hit >= 0 ? 1 : 0;
       } else {
         prim_out[idx] = lt.hit >= 0 ? s.prim_id[lt.hit] : -1;
         if (t_out) t_out[idx] = lt.hit >= 0 ? lt.best : 0.0f;
       }
-      have = false;
     }
   }
   if (COUNT) {
-    unsigned long long a = cnt.nodes, b = cnt.prims;
-    for (int off = 32; off > 0; off >>= 1) {
-      a += __shfl_down(a, off);
-      b += __shfl_down(b, off);
-    }
-    if ((threadIdx.x & 63) == 0) {
-      atomicAdd(&counters[0], a);
-      atomicAdd(&counters[1], b);
-    }
+    wave_count(cnt.nodes, &counters[0]);
+    wave_count(cnt.prims, &counters[1]);
   }
 }
 
@@ -134,12 +123,12 @@ __global__ void __launch_bounds__(kQueryBlock)
                   const float *__restrict__ tmax, uint32_t n, int32_t *__restrict__ prim_out,
                   float *__restrict__ t_out, uint8_t *__restrict__ occ_out, unsigned long long *__restrict__ counters,
                   uint32_t *next) {
-  __shared__ uint2 lds[kExactRing * kQueryBlock];
-  uint2 old[ExactStack<CAP>::kOld];
-  ExactStack<CAP> st(lds + threadIdx.x, kQueryBlock, old);
+  __shared__ uint2 lds[kPrivateRing * kQueryBlock];
+  uint2 old[PrivateStack<CAP>::kOld];
+  PrivateStack<CAP> st(lds + threadIdx.x, kQueryBlock, old);
   ExactWalk<COUNT, ANY ? kWalkAny : kWalkClosest> w;
   TraceCounters cnt;
-  WaveFetch<true> wf(n, kQueryChunk);
+  WaveFetch wf(n, kChunk);
   uint32_t idx = 0;
   bool walking = false, have = false, drained = false;
   while (true) {
@@ -218,14 +207,14 @@ struct QueryLaunch {
 };
 }  // namespace
 
-// Static scratch of muonx_intersect_noalloc: the claim counter of the
-// per-lane fetch kernels (the first 256 bytes) and the traversal stacks'
+// Static scratch of muonx_intersect_noalloc: the claim counters of the
+// per-lane fetch kernels (the first kClaimBytes) and the traversal stacks'
 // spill region (the rest). Every GPU holds its own copy until the process
 // ends; its device address is looked up once per device by
 // InitStaticScratch (with the device current), never used by name on the
 // host.
 constexpr size_t kStaticScratchBytes = size_t(32) << 20;
-constexpr size_t kStaticScratchHead = 256;
+constexpr size_t kStaticScratchHead = kClaimBytes;
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 
 namespace {
@@ -239,7 +228,7 @@ void *StaticScratch(int device) {
   return g_scratch_ptr[device];
 }
 
-__global__ void k_zero_u32(uint32_t *p) { *p = 0u; }
+__global__ void k_clear_claims(uint32_t *p) { p[threadIdx.x * kClaimStride] = 0u; }
 }  // namespace
 
 int InitStaticScratch(int device) {
@@ -256,26 +245,25 @@ int InitStaticScratch(int device) {
   return MUONX_OK;
 }
 
-// The claim counter of the per-lane fetch kernels, cleared on `stream`: in
+// The claim counters of the per-lane fetch kernels, cleared on `stream`: in
 // the static scratch with `noalloc` (by a kernel rather than a memset node),
 // else in the context, ordered after its previous user like the spill region.
 static int ClearClaims(muonx_ctx *ctx, hipStream_t stream, bool noalloc, void *scratch_base, uint32_t **next) {
   if (noalloc) {
     *next = static_cast<uint32_t *>(scratch_base);
-    hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(1), 0, stream, *next);
+    hipLaunchKernelGGL(k_clear_claims, dim3(1), dim3(kClaimGroups), 0, stream, *next);
     return MUONX_OK;
   }
-  MX_HIP(ctx->fetch_ctr.Reserve(sizeof(uint32_t)));
+  MX_HIP(ctx->fetch_ctr.Reserve(kClaimBytes));
   if (!ctx->spill_done) MX_HIP(hipEventCreateWithFlags(&ctx->spill_done, hipEventDisableTiming));
   MX_HIP(hipStreamWaitEvent(stream, ctx->spill_done, 0));
-  MX_HIP(hipMemsetAsync(ctx->fetch_ctr.ptr, 0, sizeof(uint32_t), stream));
+  MX_HIP(hipMemsetAsync(ctx->fetch_ctr.ptr, 0, kClaimBytes, stream));
   *next = ctx->fetch_ctr.as<uint32_t>();
   return MUONX_OK;
 }
 
-// Exact mode: stacks in LDS and private memory, so the claim counter is the
-// only scratch, and a batch that the wavefronts' first chunks cover needs
-// none. 6, 8, 12 or 16 blocks per CU: 308 / 301 / 260 / 260 us for 300,007
+// Exact mode: stacks in LDS and private memory, so the claim counters are
+// the only scratch, and a batch without claims needs none. 6, 8, 12 or 16 blocks per CU: 308 / 301 / 260 / 260 us for 300,007
 // rays on the level-6 icosphere.
 constexpr int kExactBlocksPerCu = 12;
 constexpr uint32_t kExactPart = 1u << 30;  // rays per launch: 3 * index stays below 2^32
@@ -291,7 +279,7 @@ static int LaunchExactQuery(muonx_ctx *ctx, const DevSceneView &s, bool any, con
     const uint64_t cus = uint64_t(ctx->num_cus > 0 ? ctx->num_cus : 256);
     const uint32_t grid = QueryGrid(m, uint32_t(cus) * kExactBlocksPerCu);
     uint32_t *next = nullptr;
-    const bool claims = !CoveredByFirstChunks(m, grid * kWavesPerBlock, kQueryChunk);
+    const bool claims = NeedsClaims(m, grid * kWavesPerBlock);
     if (claims) {
       const int rc = ClearClaims(ctx, stream, noalloc, scratch_base, &next);
       if (rc != MUONX_OK) return rc;
@@ -365,10 +353,11 @@ int LaunchQuery(muonx_ctx *ctx, const DevSceneView &s, bool any, bool exact, con
 #define MX_Q(A, C) DispatchTraverse(cfg, QueryLaunch<A, C>{cfg, s, ro, rd, tmax, n, prim, t, occ, counters, stream})
   const bool cnt = counters != nullptr;
   const int fetch = ctx->tuning.ray_fetch;
-  if (fetch > 0 && n <= (1u << 31)) {  // the claim counter stays below 2^32 (n + chunk x waves)
+  if (fetch > 0 && n <= (1u << 31)) {  // claimed indices stay below 2^32
     // per-lane ray fetch
-    uint32_t *next;
-    if ((rc = ClearClaims(ctx, stream, noalloc, sbase, &next)) != MUONX_OK) return rc;
+    uint32_t *next = nullptr;
+    const bool claims = NeedsClaims(n, uint32_t(cfg.grid) * kWavesPerBlock);
+    if (claims && (rc = ClearClaims(ctx, stream, noalloc, sbase, &next)) != MUONX_OK) return rc;
 #define MX_QD(A, C) DispatchTraverse(cfg, QueryDynLaunch<A, C>{cfg, s, ro, rd, tmax, n, prim, t, occ, counters, next, fetch, stream})
     if (any) {
       if (cnt) MX_QD(true, true);
@@ -379,7 +368,7 @@ int LaunchQuery(muonx_ctx *ctx, const DevSceneView &s, bool any, bool exact, con
     }
 #undef MX_QD
     MX_HIP(hipGetLastError());
-    if (!noalloc) MX_HIP(hipEventRecord(ctx->spill_done, stream));
+    if (!noalloc && (claims || cfg.spill)) MX_HIP(hipEventRecord(ctx->spill_done, stream));
     return MUONX_OK;
   }
   if (any) {

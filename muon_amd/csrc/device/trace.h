@@ -236,23 +236,6 @@ struct LdsStack {
       ++sp;
     }
   }
-  // Pushes c, b, a (the last m of them, m <= 3) in that order: a ends on top.
-  // Three unconditional writes, c then b then a: an entry that is not pushed
-  // is written to a's slot first and overwritten by a.
-  __device__ __forceinline__ void push_last(int m, uint2 a, uint2 b, uint2 c) {
-    if (m <= 0) return;
-    if (sp + m > CAP) {
-      if (m >= 3) push(c);
-      if (m >= 2) push(b);
-      push(a);
-      return;
-    }
-    const int pa = sp + m - 1, pb = m >= 2 ? sp + m - 2 : pa, pc = m >= 3 ? sp : pa;
-    base[pc * stride] = c;
-    base[pb * stride] = b;
-    base[pa * stride] = a;
-    sp += m;
-  }
   __device__ __forceinline__ bool empty() const { return sp == 0; }
   __device__ __forceinline__ uint2 pop() {
     --sp;
@@ -262,7 +245,7 @@ struct LdsStack {
 
 // RingStack: the top S entries (S a power of two) in an LDS ring, older
 // entries spilled to a per-thread global region g[k * gstride], k <
-// gcap. Keeps LDS use small (high occupancy) while supporting deep trees.
+// gcap: any depth, at the cost of a region that the launch reserves.
 template <int S>
 struct RingStack {
   uint2 *base;
@@ -283,30 +266,46 @@ struct RingStack {
     base[slot * stride] = v;
     ++sp;
   }
-  // Pushes c, b, a (the last m of them, m <= 3) in that order: a ends on top.
-  // Without a spill (the common case) the entries go straight to their ring
-  // slots (all below S) with three unconditional writes, c then b then a: an
-  // entry that is not pushed is written to a's slot first and overwritten.
-  __device__ __forceinline__ void push_last(int m, uint2 a, uint2 b, uint2 c) {
-    if (m <= 0) return;
-    if (sp + m > S) {
-      if (m >= 3) push(c);
-      if (m >= 2) push(b);
-      push(a);
-      return;
-    }
-    const int pa = sp + m - 1, pb = m >= 2 ? sp + m - 2 : pa, pc = m >= 3 ? sp : pa;
-    base[pc * stride] = c;
-    base[pb * stride] = b;
-    base[pa * stride] = a;
-    sp += m;
-  }
   __device__ __forceinline__ bool empty() const { return sp == 0; }
   __device__ __forceinline__ uint2 pop() {
     --sp;
     const int slot = sp & (S - 1);
     const uint2 v = base[slot * stride];
     if (sp >= S) base[slot * stride] = g[(sp - S) * gstride];
+    return v;
+  }
+};
+
+// PrivateStack: the top kPrivateRing entries in an LDS ring, older ones in
+// the lane's private memory `private_old` (CAP - kPrivateRing entries, an
+// array of the kernel): as little LDS as a RingStack of 8, with no region to
+// reserve or to order between launches, and without that region's addresses
+// in registers (the closest-hit query kernel then fits eight wavefronts per
+// SIMD without register spills).
+constexpr int kPrivateRing = 8;
+template <int CAP>
+struct PrivateStack {
+  static constexpr int kOld = CAP - kPrivateRing;
+  uint2 *base, *old;
+  int stride, sp;
+  __device__ __forceinline__ PrivateStack(uint2 *b, int s, uint2 *private_old)
+      : base(b), old(private_old), stride(s), sp(0) {}
+  __device__ __forceinline__ void reset() { sp = 0; }
+  __device__ __forceinline__ void push(uint2 v) {
+    uint2 *slot = base + (sp & (kPrivateRing - 1)) * stride;
+    if (sp >= kPrivateRing) {
+      if (sp >= CAP) return;  // sized from the BVH depth: never taken
+      old[sp - kPrivateRing] = *slot;
+    }
+    *slot = v;
+    ++sp;
+  }
+  __device__ __forceinline__ bool empty() const { return sp == 0; }
+  __device__ __forceinline__ uint2 pop() {
+    --sp;
+    uint2 *slot = base + (sp & (kPrivateRing - 1)) * stride;
+    const uint2 v = *slot;
+    if (sp >= kPrivateRing) *slot = old[sp - kPrivateRing];
     return v;
   }
 };
@@ -525,7 +524,7 @@ __device__ __forceinline__ void use_now(uint4 &v) { asm volatile("" : "+v"(v.x),
 // children farthest first (so they pop nearest first). Returns false when no
 // child is hit.
 template <bool COUNT, class Stack>
-__device__ __forceinline__ bool wnode_step(const DevSceneView &s, const TraceRay &r, float best, Stack &stack,
+__device__ __forceinline__ bool wnode_step(const DevSceneView &s, const TraceRay &r, float bm, Stack &stack,
                                            uint32_t &ref, TraceCounters &cnt) {
   const float4 *np = s.wnodes + 8 * size_t(ref);
   const float4 lx = ldg(np), hx = ldg(np + 1), ly = ldg(np + 2), hy = ldg(np + 3), lz = ldg(np + 4),
@@ -535,7 +534,6 @@ __device__ __forceinline__ bool wnode_step(const DevSceneView &s, const TraceRay
   if (COUNT) cnt.nodes++;
   constexpr float kInf = __builtin_inff();
   float t0, t1, t2, t3;
-  const float bm = below(best);
   const bool h0 = box_hit(r, lx.x, hx.x, ly.x, hy.x, lz.x, hz.x, bm, t0);
   const bool h1 = box_hit(r, lx.y, hx.y, ly.y, hy.y, lz.y, hz.y, bm, t1) && n > 1;
   const bool h2 = box_hit(r, lx.z, hx.z, ly.z, hy.z, lz.z, hz.z, bm, t2) && n > 2;
@@ -565,8 +563,9 @@ __device__ __forceinline__ bool wnode_step(const DevSceneView &s, const TraceRay
   cswap(k0, r0, k2, r2);
   cswap(k1, r1, k3, r3);
   cswap(k1, r1, k2, r2);
-  stack.push_last(nhit - 1, make_uint2(r1, __float_as_uint(k1)), make_uint2(r2, __float_as_uint(k2)),
-                  make_uint2(r3, __float_as_uint(k3)));
+  if (k3 < kInf) stack.push(make_uint2(r3, __float_as_uint(k3)));
+  if (k2 < kInf) stack.push(make_uint2(r2, __float_as_uint(k2)));
+  if (k1 < kInf) stack.push(make_uint2(r1, __float_as_uint(k1)));
   ref = r0;
   return true;
 }
@@ -579,6 +578,13 @@ constexpr int kNodesWideQ = 5;   // 4-wide nodes, 8-bit quantized child boxes
 // Byte k of a packed plane word as a float (v_cvt_f32_ubyte<k>).
 __device__ __forceinline__ float plane_q(uint32_t word, int k) { return float((word >> (8 * k)) & 255u); }
 
+// The reciprocals of qnode_step's rays.
+__device__ __forceinline__ void clamp_inv(TraceRay &r) {
+  constexpr float kBig = 18446744073709551616.0f;  // 2^64
+  r.inv = V3{__builtin_amdgcn_fmed3f(r.inv.x, -kBig, kBig), __builtin_amdgcn_fmed3f(r.inv.y, -kBig, kBig),
+             __builtin_amdgcn_fmed3f(r.inv.z, -kBig, kBig)};
+}
+
 // One quantized wide-node step (as wnode_step). Per axis, the distance to
 // the plane origin + q * 2^e is folded to one fused multiply-add,
 //   t = q * A + B,  A = 2^e * inv (exact),  B = (origin - o) * inv,
@@ -588,7 +594,8 @@ __device__ __forceinline__ float plane_q(uint32_t word, int k) { return float((w
 // fma leaves |t' - t| <= ~3 eps |B| + eps |t|. The slack 2^-20 |B| per axis
 // (down on entry planes, up on exit planes) covers the first term and the
 // 2^-20 relative widening the second, so the test stays a superset of the
-// exact one. Reciprocals are clamped to +-2^64: a zero direction component
+// exact one. Reciprocals are clamped to +-2^64 (clamp_inv, when the ray
+// starts): a zero direction component
 // then gives finite plane distances whose sign says whether the origin lies
 // in the slab (an infinite one would make inf - inf and lose the axis), and
 // the per-axis slack keeps a ray that runs in an exit plane inside the box
@@ -601,7 +608,7 @@ __device__ __forceinline__ float plane_q(uint32_t word, int k) { return float((w
 // pushed child passes the pop test anyway; the hit children are moved ahead
 // of the missed ones in child order by flags alone and pushed with key 0.
 template <bool COUNT, bool ANY, class Stack>
-__device__ __forceinline__ bool qnode_step(const DevSceneView &s, const TraceRay &r, float best, Stack &stack,
+__device__ __forceinline__ bool qnode_step(const DevSceneView &s, const TraceRay &r, float bm, Stack &stack,
                                            uint32_t &ref, TraceCounters &cnt) {
   const uint4 *np = s.qnodes + 4 * size_t(ref);
   const uint4 n0 = ldg(np), n1 = ldg(np + 1), n2 = ldg(np + 2);
@@ -622,10 +629,7 @@ __device__ __forceinline__ bool qnode_step(const DevSceneView &s, const TraceRay
   const uint32_t nxw = (n1.w & mx) | (n1.x & ~mx), fxw = (n1.x & mx) | (n1.w & ~mx);
   const uint32_t nyw = (n2.x & my) | (n1.y & ~my), fyw = (n1.y & my) | (n2.x & ~my);
   const uint32_t nzw = (n2.y & mz) | (n1.z & ~mz), fzw = (n1.z & mz) | (n2.y & ~mz);
-  const float bm = below(best);
-  constexpr float kBig = 18446744073709551616.0f;  // 2^64
-  const float ix = __builtin_amdgcn_fmed3f(r.inv.x, -kBig, kBig), iy = __builtin_amdgcn_fmed3f(r.inv.y, -kBig, kBig),
-              iz = __builtin_amdgcn_fmed3f(r.inv.z, -kBig, kBig);
+  const float ix = r.inv.x, iy = r.inv.y, iz = r.inv.z;
   const float Ax = sx * ix, Ay = sy * iy, Az = sz * iz;
   const float Bx = (ox - r.o.x) * ix, By = (oy - r.o.y) * iy, Bz = (oz - r.o.z) * iz;
   const float ex = fabsf(Bx) * kSlack, ey = fabsf(By) * kSlack, ez = fabsf(Bz) * kSlack;
@@ -667,7 +671,9 @@ __device__ __forceinline__ bool qnode_step(const DevSceneView &s, const TraceRay
     cpart(h0, r0, h2, r2);
     cpart(h1, r1, h3, r3);
     cpart(h1, r1, h2, r2);
-    stack.push_last(nhit - 1, make_uint2(r1, 0u), make_uint2(r2, 0u), make_uint2(r3, 0u));
+    if (h3) stack.push(make_uint2(r3, 0u));
+    if (h2) stack.push(make_uint2(r2, 0u));
+    if (h1) stack.push(make_uint2(r1, 0u));
     ref = r0;
     return true;
   } else {
@@ -686,27 +692,30 @@ __device__ __forceinline__ bool qnode_step(const DevSceneView &s, const TraceRay
     cswap(k0, r0, k2, r2);
     cswap(k1, r1, k3, r3);
     cswap(k1, r1, k2, r2);
-    stack.push_last(nhit - 1, make_uint2(r1, __float_as_uint(k1)), make_uint2(r2, __float_as_uint(k2)),
-                    make_uint2(r3, __float_as_uint(k3)));
+    if (k3 < kInf) stack.push(make_uint2(r3, __float_as_uint(k3)));
+    if (k2 < kInf) stack.push(make_uint2(r2, __float_as_uint(k2)));
+    if (k1 < kInf) stack.push(make_uint2(r1, __float_as_uint(k1)));
     ref = r0;
     return true;
   }
 }
 
-// One internal-node step of the fast mode for node format NODES.
+// One internal-node step of the fast mode for node format NODES; `bm` is
+// below(best), and the reciprocals of a quantized format's ray are clamped.
 template <int NODES, bool COUNT, bool ANY, class Stack>
-__device__ __forceinline__ bool fast_step(const DevSceneView &s, const TraceRay &r, float best, Stack &stack,
-                                          uint32_t &ref, TraceCounters &cnt) {
-  if constexpr (NODES == kNodesWideQ) return qnode_step<COUNT, ANY>(s, r, best, stack, ref, cnt);
-  else if constexpr (NODES == kNodesWide) return wnode_step<COUNT>(s, r, best, stack, ref, cnt);
+__device__ __forceinline__ bool fast_step(const DevSceneView &s, const TraceRay &r, float best, float bm,
+                                          Stack &stack, uint32_t &ref, TraceCounters &cnt) {
+  if constexpr (NODES == kNodesWideQ) return qnode_step<COUNT, ANY>(s, r, bm, stack, ref, cnt);
+  else if constexpr (NODES == kNodesWide) return wnode_step<COUNT>(s, r, bm, stack, ref, cnt);
   else return node_step<COUNT, false>(s, r, false, best, stack, ref, cnt);
 }
 
 // Closest / any hit over the wide BVH (fast mode only: children are visited
 // nearest first, so ties may resolve differently from the reference's order).
 template <int NODES, bool ANY, bool COUNT, bool WW, class Stack>
-__device__ __forceinline__ int32_t trace_bvh4_s(const DevSceneView &s, const TraceRay &r, float &best, Stack &stack,
+__device__ __forceinline__ int32_t trace_bvh4_s(const DevSceneView &s, TraceRay r, float &best, Stack &stack,
                                                 TraceCounters &cnt) {
+  if (NODES == kNodesWideQ) clamp_inv(r);
   int32_t hit_prim = -1;
   ObjCache oc;
   oc.tid = -1;
@@ -715,7 +724,7 @@ __device__ __forceinline__ int32_t trace_bvh4_s(const DevSceneView &s, const Tra
     while (true) {
       bool alive = true;
       while (!(ref & kLeafBit)) {
-        if (!fast_step<NODES, COUNT, ANY>(s, r, best, stack, ref, cnt) && !pop_next(stack, best, ref)) {
+        if (!fast_step<NODES, COUNT, ANY>(s, r, best, below(best), stack, ref, cnt) && !pop_next(stack, best, ref)) {
           alive = false;
           break;
         }
@@ -727,7 +736,7 @@ __device__ __forceinline__ int32_t trace_bvh4_s(const DevSceneView &s, const Tra
   } else {
     while (true) {
       if (!(ref & kLeafBit)) {
-        if (fast_step<NODES, COUNT, ANY>(s, r, best, stack, ref, cnt)) continue;
+        if (fast_step<NODES, COUNT, ANY>(s, r, best, below(best), stack, ref, cnt)) continue;
       } else {
         if (leaf_step<ANY, COUNT, true>(s, r, best, ref, oc, hit_prim, cnt)) return hit_prim;
       }
@@ -745,35 +754,73 @@ __device__ __forceinline__ int32_t trace_fast(const DevSceneView &s, const Trace
   else return trace_bvh4_s<WIDTH, ANY, COUNT, WW>(s, r, best, stack, cnt);
 }
 
-// Resumable fast-mode traversal of one lane, for kernels that hand a lane a
-// new ray as soon as its current one is finished instead of waiting for the
-// slowest ray of the wavefront. round() walks internal nodes to the next leaf
-// and tests it (one while-while step); it returns true when the ray is done.
+// Resumable fast-mode walk of one lane, for kernels that hand a lane a new
+// ray as soon as its current one is finished (run_walks).
 template <int WIDTH, bool ANY, bool COUNT>
 struct LaneTrace {
   TraceRay r;
-  float best;
-  int32_t hit;
-  uint32_t ref;
+  float best, bm;  // bm = below(best)
+  int32_t hit;     // leaf-order primitive or -1
+  uint32_t ref;    // the node or leaf to visit next
   ObjCache oc;
   template <class Stack>
   __device__ __forceinline__ void start(const TraceRay &ray, float tmax, Stack &st) {
     r = ray;
+    if (WIDTH == kNodesWideQ) clamp_inv(r);
     best = tmax;
+    bm = below(tmax);
     hit = -1;
     ref = 0;
     oc.tid = -1;
     st.reset();
   }
+  __device__ __forceinline__ bool at_leaf() const { return (ref & kLeafBit) != 0u; }
+  // Visits the internal node `ref`; false when the walk is over.
   template <class Stack>
-  __device__ __forceinline__ bool round(const DevSceneView &s, Stack &st, TraceCounters &cnt) {
-    while (!(ref & kLeafBit)) {
-      if (!fast_step<WIDTH, COUNT, ANY>(s, r, best, st, ref, cnt) && !pop_next(st, best, ref)) return true;
-    }
-    if (leaf_step<ANY, COUNT, WIDTH != kNodesBinary>(s, r, best, ref, oc, hit, cnt)) return true;
-    return !pop_next(st, best, ref);
+  __device__ __forceinline__ bool node(const DevSceneView &s, Stack &st, TraceCounters &cnt) {
+    return fast_step<WIDTH, COUNT, ANY>(s, r, best, bm, st, ref, cnt) || pop_next(st, best, ref);
+  }
+  // Tests the primitives of the leaf `ref`; false when the walk is over.
+  template <class Stack>
+  __device__ __forceinline__ bool leaf(const DevSceneView &s, Stack &st, TraceCounters &cnt) {
+    if (leaf_step<ANY, COUNT, WIDTH != kNodesBinary>(s, r, best, ref, oc, hit, cnt)) return false;
+    bm = below(best);
+    return pop_next(st, best, ref);
   }
 };
+
+// Advances the wavefront's walks (the lanes with `walking`) until at least
+// `stop` of its lanes have none, at least one step. Lanes step through
+// internal nodes together while at least a kNodeShare-th of those that walk are
+// at one; then those at a leaf test its primitives. Every lane makes its own
+// walk's steps in order, whatever the others do. All 64 lanes call it.
+// Waiting instead until every lane holds a leaf
+// keeps few lanes busy (2^24 closest hits on the level-7 icosphere, one
+// counter for the claims: 159 wavefront instructions per ray at 26 % lane
+// use; with a half 110 at 40 %). A half, a third, a quarter, a sixth and a
+// 16th: 2460 / 2574 / 2724 / 2886 / 3230 us there, 400 / 397 / 407 / 429 /
+// 484 us for 3,000,017 any-hit rays on 10,000 spheres, 31.3 / 31.5 / 31.9 /
+// 32.8 / 35.2 ms for the 512x512, 64 spp render of the icosphere; two
+// thirds: 2535 us, 420 us, 32.0 ms. A fixed number of lanes (16) costs the
+// small batches, whose wavefronts hold a few rays each, 15 %. Exact walks,
+// 10^6 rays on 10,000 spheres: 324 / 348 / 367 / 400 us with a half, a third,
+// a quarter and a sixth.
+constexpr int kNodeShare = 2;
+template <class Walk, class Stack>
+__device__ __forceinline__ void run_walks(const DevSceneView &s, Walk &w, bool &walking, Stack &st,
+                                          TraceCounters &cnt, int stop) {
+  uint64_t active = __builtin_amdgcn_ballot_w64(walking);
+  do {
+    uint64_t nodes = __builtin_amdgcn_ballot_w64(walking && !w.at_leaf());
+    while (nodes && __popcll(nodes) * kNodeShare >= __popcll(active)) {
+      if (walking && !w.at_leaf()) walking = w.node(s, st, cnt);
+      active = __builtin_amdgcn_ballot_w64(walking);
+      nodes = __builtin_amdgcn_ballot_w64(walking && !w.at_leaf());
+    }
+    if (walking && w.at_leaf()) walking = w.leaf(s, st, cnt);
+    active = __builtin_amdgcn_ballot_w64(walking);
+  } while (active && 64 - __popcll(active) < stop);
+}
 
 // Fixed LDS stack at stack[k * stride], k < STACK (STACK >= BVH depth).
 template <int STACK, bool ANY, bool COUNT, bool EXACT = false>

@@ -7,11 +7,14 @@
 
 #include "runtime.h"
 #include "trace.h"
+#include "wave.h"
 
 namespace muonx {
 
-// Stack variants: kinds 24/48/96 = full LDS stack of that capacity, 8/16 =
-// LDS ring with HBM spill.
+// Stack variants: kinds 24/48/96 = full LDS stack of that capacity, 8 = LDS
+// ring of 8 with older entries in private memory (kPrivateCap in all), 16 =
+// LDS ring of 16 with HBM spill.
+constexpr int kPrivateCap = 72;
 struct TraverseCfg {
   int kind;     // 24, 48, 96, 8 or 16
   bool ww;
@@ -31,19 +34,26 @@ struct StackArgs {
 template <int KIND>
 struct StackOf;
 template <>
-struct StackOf<24> { using T = LdsStack<24>; static constexpr int kLds = 24; };
+struct StackOf<24> { using T = LdsStack<24>; static constexpr int kLds = 24, kPrivate = 1; };
 template <>
-struct StackOf<48> { using T = LdsStack<48>; static constexpr int kLds = 48; };
+struct StackOf<48> { using T = LdsStack<48>; static constexpr int kLds = 48, kPrivate = 1; };
 template <>
-struct StackOf<96> { using T = LdsStack<96>; static constexpr int kLds = 96; };
+struct StackOf<96> { using T = LdsStack<96>; static constexpr int kLds = 96, kPrivate = 1; };
 template <>
-struct StackOf<8> { using T = RingStack<8>; static constexpr int kLds = 8; };
+struct StackOf<8> {
+  using T = PrivateStack<kPrivateCap>;
+  static constexpr int kLds = kPrivateRing, kPrivate = T::kOld;
+};
 template <>
-struct StackOf<16> { using T = RingStack<16>; static constexpr int kLds = 16; };
+struct StackOf<16> { using T = RingStack<16>; static constexpr int kLds = 16, kPrivate = 1; };
 
+// `old`: a kernel's private array of StackOf<KIND>::kPrivate entries.
 template <int KIND>
-__device__ __forceinline__ typename StackOf<KIND>::T make_stack(uint2 *lds, int block, const StackArgs &sa) {
-  if constexpr (KIND == 8 || KIND == 16) {
+__device__ __forceinline__ typename StackOf<KIND>::T make_stack(uint2 *lds, int block, const StackArgs &sa,
+                                                                uint2 *old) {
+  if constexpr (KIND == 8) {
+    return typename StackOf<KIND>::T(lds + threadIdx.x, block, old);
+  } else if constexpr (KIND == 16) {
     const int gtid = int(blockIdx.x) * block + int(threadIdx.x);
     const int nthreads = int(gridDim.x) * block;
     return typename StackOf<KIND>::T(lds + threadIdx.x, block, sa.spill + gtid, nthreads, sa.gcap);
@@ -63,7 +73,11 @@ inline int PlanTraverseShape(const muonx_tuning &t, int num_cus, uint32_t bvh_de
   const int cus = num_cus > 0 ? num_cus : 256;
   cfg.width = t.bvh_width != 4 ? kNodesBinary : (t.node_bits == 8 ? kNodesWideQ : kNodesWide);
   const int bpc = std::max(1, t.blocks_per_cu);
-  cfg.grid = int(std::max<uint64_t>(1, std::min<uint64_t>(uint64_t(cus) * bpc, (work_items + block - 1) / block)));
+  // enough wavefronts for each to hold a first chunk of the work (wave.h)
+  const uint32_t most = uint32_t(cus * bpc), wpb = uint32_t(block / 64);
+  const uint64_t waves =
+      work_items / FirstChunk(uint32_t(std::min<uint64_t>(work_items, UINT32_MAX)), most * wpb) + 1;
+  cfg.grid = int(std::max<uint64_t>(1, std::min<uint64_t>(most, (waves + wpb - 1) / wpb)));
   cfg.threads = cfg.grid * block;
   cfg.ww = t.while_while != 0;
   cfg.spill = nullptr;
@@ -71,13 +85,13 @@ inline int PlanTraverseShape(const muonx_tuning &t, int num_cus, uint32_t bvh_de
   // binary: entries never exceed depth - 1; wide: the collapse's bound
   const int need = int(cfg.width != kNodesBinary ? std::max<uint32_t>(wstack, 1) : bvh_depth);
   const bool ring = t.stack_entries == 8 || t.stack_entries == 16;
-  if (ring && need <= t.stack_entries) {
-    cfg.kind = need <= 8 ? 8 : 16;  // a ring that never spills
+  if (ring && need <= (t.stack_entries == 8 ? kPrivateCap : 8)) {
+    cfg.kind = 8;
     return MUONX_OK;
   }
   if (ring || need > 96) {
-    cfg.kind = ring ? t.stack_entries : 16;
-    cfg.gcap = need - cfg.kind;
+    cfg.kind = 16;
+    cfg.gcap = std::max(0, need - 16);
     return MUONX_OK;
   }
   if (need <= 24) cfg.kind = 24;

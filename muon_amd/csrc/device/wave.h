@@ -7,6 +7,8 @@
 
 #include <cstdint>
 
+#include "claim_plan.h"
+
 namespace muonx {
 
 // Appends the lanes with `want` to a queue: returns each such lane's index
@@ -95,70 +97,36 @@ __device__ __forceinline__ void wave_count(uint32_t n, unsigned long long *ctr) 
 }
 
 // Work claiming for kernels that give each lane a new item as soon as its
-// current one is finished. Items are handed out in chunks of `chunk`
-// consecutive indices (64..max_chunk, about four chunks per wavefront of the
-// grid; larger chunks leave more work in a few wavefronts' last chunks,
-// smaller ones put more atomics on the one counter): wavefront w's first chunk
-// is [w * chunk, (w + 1) * chunk) with no
-// atomic, later chunks come from a global counter (one atomic per chunk,
-// offset past the first chunks of all wavefronts). A wavefront whose first
-// chunk lies past the item count exits without touching the counter, so a
-// launch over few or no items costs no contended atomics. cbase / cend /
-// chunk are the same in every lane.
-//
-// SPREAD: few items are spread over two wavefronts per SIMD before a
-// wavefront gets all of its lanes an item (a wavefront takes as long as the
-// longest of its lanes at every step, and idle SIMDs cost nothing), and a
-// launch whose first chunks cover every item (CoveredByFirstChunks) never
-// touches the counter. 10,000 exact closest hits on the level-5 icosphere
-// take 95 us against 128 us with 64 rays to each wavefront, 1000 on the
-// Cornell box 18 against 34 us; at least 2, 4, 8 or 16 rays each: 95 / 94 /
-// 102 / 113 and 18 / 21 / 27 / 34 us; 1024, 2048, 4096 or 6144 wavefronts:
-// within 1 % but for 200,000 any-hit rays, which 6144 make 16 % slower.
-constexpr uint32_t kSpreadWaves = 2048, kSpreadMin = 2;
-constexpr uint32_t ClaimChunk(uint32_t items, uint32_t waves, uint32_t max_chunk, bool spread) {
-  const uint32_t c = (items / (4u * waves)) & ~63u;
-  if (c >= 64u || !spread) return c < 64u ? 64u : (c < max_chunk ? c : max_chunk);
-  const uint32_t each = items / (waves < kSpreadWaves ? waves : kSpreadWaves) + 1u;
-  return each >= 64u ? 64u : (each < kSpreadMin ? kSpreadMin : each);
-}
-constexpr bool CoveredByFirstChunks(uint32_t items, uint32_t waves, uint32_t max_chunk) {
-  return items <= uint64_t(waves) * ClaimChunk(items, waves, max_chunk, true);
-}
-
-template <bool SPREAD = false>
+// current one is finished: the wavefront's ClaimPlan (claim_plan.h), the same
+// in every lane.
 struct WaveFetch {
-  static constexpr uint32_t kMaxChunk = 256;
-  static constexpr uint32_t kNone = 0x80000000u;  // past every item (at most 2^31 of them)
-  uint32_t chunk, first, cbase, cend;
-  __device__ __forceinline__ explicit WaveFetch(uint32_t items, uint32_t max_chunk = kMaxChunk) {
-    const uint32_t wpb = (blockDim.x + 63u) >> 6;
-    const uint32_t waves = gridDim.x * wpb;
-    chunk = ClaimChunk(items, waves, max_chunk, SPREAD);
-    first = waves * chunk;
-    if (SPREAD && items <= first) first = kNone;
-    cbase = (blockIdx.x * wpb + (threadIdx.x >> 6)) * chunk;
-    cend = cbase + chunk;
-  }
+  ClaimPlan p;
+  __device__ __forceinline__ explicit WaveFetch(uint32_t items, uint32_t max_chunk = 256)
+      : p(items, gridDim.x, gridDim.x * (blockDim.x >> 6),
+          uint32_t(__builtin_amdgcn_readfirstlane(int(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)))),
+          blockIdx.x, max_chunk) {}
   // Called by every lane of the wavefront with the ballot of `need`; returns
   // the index claimed for this lane (meaningful where `need` is set; an
   // index >= the item count means none is left).
-  __device__ __forceinline__ uint32_t claim(uint64_t needm, uint32_t *counter) {
+  __device__ __forceinline__ uint32_t claim(uint64_t needm, uint32_t *counters) {
     const uint32_t lane = __lane_id();
     const uint32_t cnt = uint32_t(__popcll(needm));
     const uint32_t rank = uint32_t(__popcll(needm & ((1ull << lane) - 1ull)));
-    const uint32_t rem = cend - cbase;
+    const uint32_t rem = p.cend - p.cbase;
     uint32_t k;
     if (rem >= cnt) {
-      k = cbase + rank;
-      cbase += cnt;
+      k = p.cbase + rank;
+      p.cbase += cnt;
     } else {
-      uint32_t nb = 0;
-      if (lane == 0) nb = SPREAD && first == kNone ? kNone : first + atomicAdd(counter, chunk);
-      nb = uint32_t(__shfl(int(nb), 0));
-      k = rank < rem ? cbase + rank : nb + (rank - rem);
-      cbase = nb + (cnt - rem);
-      cend = nb + chunk;
+      uint32_t v = 0;
+      if (p.counted()) {
+        if (lane == 0) v = atomicAdd(counters + p.group * kClaimStride, 1u);
+        v = uint32_t(__builtin_amdgcn_readfirstlane(int(v)));
+      }
+      const uint32_t nb = p.next(v);
+      k = rank < rem ? p.cbase + rank : nb + (rank - rem);
+      p.cbase = nb + (cnt - rem);
+      p.cend = nb + p.chunk;
     }
     return k;
   }

@@ -45,6 +45,15 @@ constexpr uint32_t FirstChunk(uint32_t items, uint32_t waves) {
   return each >= kChunk ? kChunk : (each < kSpreadMin ? kSpreadMin : each);
 }
 
+// Blocks of `wpb` wavefronts for a grid of at most `max_blocks`: as many as hold
+// a wavefront with a first chunk.
+constexpr uint32_t ClaimBlocks(uint64_t items, uint32_t max_blocks, uint32_t wpb) {
+  const uint64_t waves =
+      items / FirstChunk(items < 0xffffffffull ? uint32_t(items) : 0xffffffffu, max_blocks * wpb) + 1;
+  const uint64_t blocks = (waves + wpb - 1) / wpb;
+  return blocks < max_blocks ? uint32_t(blocks) : max_blocks;
+}
+
 // One wavefront's share: the chunk in hand and where the next one comes from.
 // Item counts up to 2^31, at most 2^20 wavefronts.
 struct ClaimPlan {

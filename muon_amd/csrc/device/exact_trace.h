@@ -22,6 +22,7 @@ struct ExactWalk {
   uint32_t ref;  // the node or leaf to visit next
   ObjCache oc;
   bool plain, any_hit;
+  uint32_t missed;  // counting any-hit walks: missed far children not popped yet
 
   __device__ __forceinline__ bool any() const { return KIND == kWalkEither ? any_hit : KIND == kWalkAny; }
   __device__ __forceinline__ bool at_leaf() const { return (ref & kLeafBit) != 0u; }
@@ -38,6 +39,7 @@ struct ExactWalk {
     ref = 0;
     oc.tid = -1;
     any_hit = any_query;
+    missed = 0;
     plain = plain_ray(s, ray);
     st.reset();
     if (!counts(s)) return true;
@@ -64,16 +66,19 @@ struct ExactWalk {
   }
 
   // The next stack entry whose box starts before `best`; false when there is
-  // none. Counting, every popped far child is the reference's bounds test at
-  // its pop.
+  // none. Counting, a popped far child is the reference's bounds test at its
+  // pop.
   template <class Stack>
   __device__ __forceinline__ bool pop(const DevSceneView &s, Stack &st, TraceCounters &cnt) {
     const bool count = counts(s);
     while (!st.empty()) {
       const uint2 e = st.pop();
       if (count) cnt.btests++;
-      if (__uint_as_float(e.y) < best) {
+      // (an any-hit walk's `best` stays its tmax, which the box passed when
+      // it was pushed)
+      if (any() || __uint_as_float(e.y) < best) {
         if (count) cnt.bhits++;
+        if (any()) missed = e.y;
         ref = e.x;
         return true;
       }
@@ -104,15 +109,18 @@ struct ExactWalk {
     if (count) {
       // The reference (muon/acceleration.cc:137,197) always pushes the far
       // child and tests its box only when it pops it, which an any-hit query
-      // that stops at its first hit (:182-183) never does. So with the near
-      // box hit the far child is pushed too, with an infinite key when its
-      // box was missed here, and its test is counted at its pop; with the
-      // near box missed the far one is popped at once.
-      cnt.btests += hn ? 1u : 2u;
+      // that stops at its first hit (:182-183) may never do. A far child
+      // whose box is missed would be popped for that test alone, so it is
+      // counted here and not pushed; an any-hit walk takes back the tests of
+      // those it did not come to (`missed`, as it was when the entry it works
+      // on was pushed, plus those met since). With the near box missed the
+      // far one is popped at once.
+      cnt.btests += hn && hf ? 1u : 2u;
       cnt.bhits += uint32_t(hn || hf);
+      missed += uint32_t(hn && !hf);
     }
     if (hn) {
-      if (count || hf) st.push(make_uint2(far_ref, hf ? __float_as_uint(lof) : 0x7f800000u));
+      if (hf) st.push(make_uint2(far_ref, any() ? missed : __float_as_uint(lof)));
       ref = near_ref;
       return true;
     }
@@ -141,7 +149,10 @@ struct ExactWalk {
       if (closer) {
         best = dist;
         hit = int32_t(i);
-        if (any()) return false;
+        if (any()) {
+          if (count) cnt.btests -= missed;
+          return false;
+        }
       }
       if (flags & 1u) break;
     }

@@ -13,13 +13,6 @@
 namespace muonx {
 
 constexpr uint32_t kWavesPerBlock = kQueryBlock / 64;
-// Blocks for n rays: as many as hold a wavefront with a first chunk, at most
-// max_blocks.
-static uint32_t QueryGrid(uint32_t n, uint32_t max_blocks) {
-  const uint64_t waves = uint64_t(n) / FirstChunk(n, max_blocks * kWavesPerBlock) + 1;
-  return uint32_t(std::min<uint64_t>(max_blocks, (waves + kWavesPerBlock - 1) / kWavesPerBlock));
-}
-
 template <int KIND, bool WW, int WIDTH, bool ANY, bool COUNT>
 __global__ void __launch_bounds__(kQueryBlock) k_query(DevSceneView s, StackArgs sa, const float *__restrict__ ro,
                                                        const float *__restrict__ rd, const float *__restrict__ tmax,
@@ -277,7 +270,7 @@ static int LaunchExactQuery(muonx_ctx *ctx, const DevSceneView &s, bool any, con
   for (uint32_t at = 0; at < n; at += std::min(n - at, kExactPart)) {
     const uint32_t m = std::min(n - at, kExactPart);
     const uint64_t cus = uint64_t(ctx->num_cus > 0 ? ctx->num_cus : 256);
-    const uint32_t grid = QueryGrid(m, uint32_t(cus) * kExactBlocksPerCu);
+    const uint32_t grid = ClaimBlocks(m, uint32_t(cus) * kExactBlocksPerCu, kWavesPerBlock);
     uint32_t *next = nullptr;
     const bool claims = NeedsClaims(m, grid * kWavesPerBlock);
     if (claims) {

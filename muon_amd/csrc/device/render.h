@@ -4,6 +4,7 @@
 #define MUONX_DEVICE_RENDER_H_
 
 #include "../common/vecmath.h"
+#include "claim_plan.h"
 #include "rng.h"
 #include "runtime.h"
 
@@ -20,6 +21,19 @@ constexpr int kCtrObjectHits = 4;
 constexpr int kCtrBoundsTests = 5;
 constexpr int kCtrBoundsHits = 6;
 constexpr int kNumCounters = 8;
+// Device counters of one muonx_render: the claim counters of the image kernels
+// (claim_plan.h), then the trace counters.
+struct RenderCounters {
+  unsigned long long *trace;
+  uint32_t *claims;
+};
+// Wavefronts add their counts to one of kCounterSlots copies of the trace
+// counters, which the host sums: a wavefront has up to seven counts to add and
+// atomics on one line take 11.3 ns each (on one copy they were 270 us of a
+// 640x480 normals image's 520 us).
+constexpr uint32_t kCounterSlots = 64, kCounterSlotStride = 32;  // 256 bytes apart
+constexpr size_t kTraceCounterBytes = size_t(kCounterSlots) * kCounterSlotStride * sizeof(unsigned long long);
+constexpr size_t kRenderCounterBytes = kClaimBytes + kTraceCounterBytes;
 
 struct CamParams {
   V3 eye, u, v, w;
@@ -63,7 +77,8 @@ class Scheduler;
 // Per-context device workspace: grown on demand, reused across renders.
 struct RenderWorkspace {
   DevBuf counters;
-  DevBuf film;  // staging film of muonx_render_host
+  DevBuf film;     // staging film of muonx_render_host
+  DevBuf samples;  // a launch's samples of the deterministic integrators
   // path-tracer engine of muonx_render / muonx_render_batch
   Scheduler *sched = nullptr;
   muonx_tuning sched_tuning{};

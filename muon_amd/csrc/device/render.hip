@@ -1,12 +1,14 @@
 // muonx_render: camera ray generation + integrators on the GPU.
-// Deterministic integrators (normals / albedo / depth, muon/integration.cc:47-76)
-// run as one fused kernel with the exact traversal mode (the reference's
-// node visits, so ties and edge hits resolve as in muon); the path tracer runs as a wavefront pipeline
+// Deterministic integrators (normals / albedo / depth, muon/integration.cc:47-76;
+// raytracer / analyticdirect) run as one fused kernel with the exact traversal
+// mode (the reference's node visits, so ties and edge hits resolve as in muon); the path tracer runs as a wavefront pipeline
 // (pathtracer.hip).
+#include <algorithm>
 #include <chrono>
-
 #include <climits>
+#include <vector>
 
+#include "exact_trace.h"
 #include "hitrec.h"
 #include "render.h"
 #include "wave.h"
@@ -41,34 +43,126 @@ CamParams MakeCam(const muonx_render_params &p) {
   return c;
 }
 
-template <int STACK>
-__global__ void __launch_bounds__(kSimpleBlock) k_simple(DevSceneView s, CamParams cam, int integrator, int spp,
-                                                         int depth0_ok, uint32_t seed, float *__restrict__ accum,
-                                                         unsigned long long *__restrict__ ctr) {
-  __shared__ uint2 stack[STACK * kSimpleBlock];
-  const uint32_t pixel = blockIdx.x * kSimpleBlock + threadIdx.x;
-  const uint32_t npix = uint32_t(cam.width) * uint32_t(cam.height);
-  uint32_t traced = 0;
+// Image kernels: every lane takes one sample of a pixel, follows it to its end
+// and takes the next. Samples are handed out in tiles of 8x8 pixels, a
+// wavefront's rays being neighbours in both directions; the walks are
+// run_walks'. A pixel's samples are added in their order, so the film has the
+// reference's bits: with several at once they go to a buffer first
+// (k_sum_samples).
+struct ImageItems {
+  uint32_t width, height, across;
+  int first, count;  // the samples of this launch
+  uint64_t tile0;    // tile of item 0
+  float *buffer;     // count > 1: sample colours, [sample][pixel]
+};
+struct ImageItem {
+  uint32_t px, py, pixel;
+  int sample;
+};
+// Item k: tile k / (64 count), sample, pixel of the tile; false for a pixel
+// outside the image (ragged last tiles).
+__device__ __forceinline__ bool image_item(const ImageItems &it, uint32_t k, ImageItem &i) {
+  const uint32_t wave = k >> 6;
+  const uint64_t tile = it.tile0 + wave / uint32_t(it.count);
+  i.sample = it.first + int(wave % uint32_t(it.count));
+  i.px = uint32_t(tile % it.across) * 8u + (k & 7u);
+  i.py = uint32_t(tile / it.across) * 8u + ((k >> 3) & 7u);
+  i.pixel = i.py * it.width + i.px;
+  return i.px < it.width && i.py < it.height;
+}
+__device__ __forceinline__ void sample_ray(const CamParams &cam, const ImageItem &i, uint32_t seed, V3 &o, V3 &d) {
+  float x, y;
+  sample_position(int(i.px), int(i.py), i.sample, path_key(seed, 0, i.pixel, uint32_t(i.sample)), x, y);
+  cast_ray(cam, x, y, o, d);
+}
+// The sample's colour, to the buffer or added to the pixel.
+__device__ __forceinline__ void write_sample(const ImageItems &it, const ImageItem &i, V3 c, float *accum) {
+  if (it.count > 1) {
+    float *out = it.buffer + 3 * (size_t(i.sample - it.first) * it.width * it.height + i.pixel);
+    out[0] = c.x;
+    out[1] = c.y;
+    out[2] = c.z;
+  } else {
+    float *out = accum + 3 * size_t(i.pixel);
+    const V3 acc = i.sample ? V3{out[0], out[1], out[2]} : V3{0.0f, 0.0f, 0.0f};
+    out[0] = acc.x + c.x;
+    out[1] = acc.y + c.y;
+    out[2] = acc.z + c.z;
+  }
+}
+// Adds the buffered samples to the film in their order.
+__global__ void k_sum_samples(const float *__restrict__ buffer, int first, int count, uint64_t n,
+                              float *__restrict__ accum) {
+  for (uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += uint64_t(gridDim.x) * blockDim.x) {
+    float acc = first ? accum[i] : 0.0f;
+    for (int k = 0; k < count; ++k) acc = acc + buffer[uint64_t(k) * n + i];
+    accum[i] = acc;
+  }
+}
+
+// Where this wavefront's counts go.
+__device__ __forceinline__ uint32_t CounterSlot() {
+  return (blockIdx.x * (kSimpleBlock / 64) + (threadIdx.x >> 6)) % kCounterSlots * kCounterSlotStride;
+}
+// Idle lanes, beyond those that no sample is left for, at which a wavefront
+// stops to give them samples. A tile's rays that start together walk in step:
+// at 16, 32 and 64 idle lanes a 1024x1024 depth image of the level-7 icosphere
+// takes 672 / 681 / 610 us (12 blocks per CU). Whitted paths differ in length:
+// 2202 / 2205 / 3067 us for 500 spheres at 641x479, 4 samples.
+constexpr int kSimpleRefill = 64, kWhittedRefill = 16;
+
+// Normals, albedo, depth. Bound by the latency of the few wavefronts along
+// silhouettes (lanes 57 % used, 1.1 wavefronts per SIMD on average). Against one
+// thread per pixel in rows of 64, a node or a leaf step per iteration, the
+// whole stack in LDS and one set of counters: 640x480 normals of the level-6
+// icosphere 523 -> 393 us, a 100x100 Cornell box 62 -> 60, 512x512 with four
+// samples of 10,000 spheres 1100 -> 441.
+template <int CAP>
+__global__ void __launch_bounds__(kSimpleBlock) __attribute__((amdgpu_waves_per_eu(4, 8)))
+    k_simple(DevSceneView s, CamParams cam, int integrator, int depth0_ok, uint32_t seed, ImageItems it, uint32_t items,
+             float *__restrict__ accum, unsigned long long *__restrict__ ctr, uint32_t *next) {
+  __shared__ uint2 lds[kPrivateRing * kSimpleBlock];
+  uint2 old[PrivateStack<CAP>::kOld];
+  PrivateStack<CAP> st(lds + threadIdx.x, kSimpleBlock, old);
+  ExactWalk<true, kWalkClosest> w;
   TraceCounters cnt;
-  if (pixel < npix) {
-    const int px = int(pixel % uint32_t(cam.width)), py = int(pixel / uint32_t(cam.width));
-    V3 acc{0.0f, 0.0f, 0.0f};
-    for (int sidx = 0; sidx < spp && depth0_ok; ++sidx) {
-      float x, y;
-      sample_position(px, py, sidx, path_key(seed, 0, pixel, uint32_t(sidx)), x, y);
-      V3 o, d;
-      cast_ray(cam, x, y, o, d);
-      const TraceRay r = make_ray(o, d);
-      float best = __builtin_inff();
-      ++traced;
-      const int32_t p = trace_bvh<STACK, false, true, true>(s, r, best, stack + threadIdx.x, kSimpleBlock, cnt);
+  WaveFetch wf(items, kChunk);
+  uint32_t traced = 0;
+  ImageItem i;
+  bool walking = false, have = false, drained = false;
+  while (true) {
+    const uint64_t needm = __builtin_amdgcn_ballot_w64(!have && !drained);
+    if (needm) {
+      const uint32_t k = wf.claim(needm, next);
+      if (!have && !drained) {
+        if (k >= items) {
+          drained = true;
+        } else if (image_item(it, k, i)) {
+          have = true;
+          w.hit = -1;
+          if (depth0_ok) {
+            V3 o, d;
+            sample_ray(cam, i, seed, o, d);
+            ++traced;
+            walking = w.start(s, make_ray(o, d), __builtin_inff(), false, st, cnt);
+          }
+        }
+      }
+    }
+    const uint64_t drainedm = __builtin_amdgcn_ballot_w64(drained);
+    if (__builtin_amdgcn_ballot_w64(have) == 0) {
+      if (~drainedm == 0) break;
+      continue;
+    }
+    run_walks(s, w, walking, st, cnt, __popcll(drainedm) + kSimpleRefill);
+    if (have && !walking) {
       V3 c{0.0f, 0.0f, 0.0f};
-      if (p >= 0) {
+      if (w.hit >= 0) {
         if (integrator == MUONX_INTEGRATOR_ALBEDO) {
-          const float *m = s.materials + size_t(s.prim_mat[p]) * kMatStride;
+          const float *m = s.materials + size_t(s.prim_mat[w.hit]) * kMatStride;
           c = V3{m[3], m[4], m[5]} + V3{m[6], m[7], m[8]};
         } else {
-          const HitRecord h = hit_record(s, uint32_t(p), o, d);
+          const HitRecord h = hit_record(s, uint32_t(w.hit), w.r.o, w.r.d);
           if (integrator == MUONX_INTEGRATOR_NORMALS) {
             c = h.normal * 0.5f + 0.5f;
           } else {
@@ -77,12 +171,11 @@ __global__ void __launch_bounds__(kSimpleBlock) k_simple(DevSceneView s, CamPara
           }
         }
       }
-      acc = acc + c;
+      write_sample(it, i, c, accum);
+      have = false;
     }
-    accum[3 * size_t(pixel)] = acc.x;
-    accum[3 * size_t(pixel) + 1] = acc.y;
-    accum[3 * size_t(pixel) + 2] = acc.z;
   }
+  ctr += CounterSlot();
   wave_count(traced, &ctr[kCtrPrimary]);
   wave_count(cnt.prims, &ctr[kCtrObjectTests]);
   wave_count(cnt.ohits, &ctr[kCtrObjectHits]);
@@ -118,106 +211,154 @@ __device__ __forceinline__ void shading_info(const float *L, V3 p, V3 &color, V3
   }
 }
 
-template <int STACK>
-__global__ void __launch_bounds__(kSimpleBlock) k_whitted(DevSceneView s, CamParams cam, int integrator, int spp,
-                                                          int cutoff, uint32_t seed, float *__restrict__ accum,
-                                                          unsigned long long *__restrict__ rays) {
-  __shared__ uint2 stack[STACK * kSimpleBlock];
-  const uint32_t pixel = blockIdx.x * kSimpleBlock + threadIdx.x;
-  const uint32_t npix = uint32_t(cam.width) * uint32_t(cam.height);
-  uint32_t n_primary = 0, n_secondary = 0, n_shadow = 0;
+// A lane goes through its sample's bounces and each bounce's shadow rays as a
+// sequence of walks, whichever kind the other lanes are at, so a short path
+// waits for no longer one. Bound by instruction issue at 25 % lane use. 500
+// shiny spheres under two lights, 641x479, 4 samples, depth 5: 4.08 -> 2.20 ms
+// against nested loops in one thread per pixel.
+template <int CAP>
+__global__ void __launch_bounds__(kSimpleBlock) __attribute__((amdgpu_waves_per_eu(4, 8)))
+    k_whitted(DevSceneView s, CamParams cam, int integrator, int cutoff, uint32_t seed, ImageItems it, uint32_t items,
+              float *__restrict__ accum, unsigned long long *__restrict__ rays, uint32_t *next) {
+  __shared__ uint2 lds[kPrivateRing * kSimpleBlock];
+  uint2 old[PrivateStack<CAP>::kOld];
+  PrivateStack<CAP> st(lds + threadIdx.x, kSimpleBlock, old);
+  ExactWalk<true, kWalkEither> w;
   TraceCounters cnt;
-  if (pixel < npix) {
-    const int px = int(pixel % uint32_t(cam.width)), py = int(pixel / uint32_t(cam.width));
-    V3 acc{0.0f, 0.0f, 0.0f};
-    V3 local[kWhittedMaxBounces], ks[kWhittedMaxBounces];
-    for (int sidx = 0; sidx < spp; ++sidx) {
-      float x, y;
-      sample_position(px, py, sidx, path_key(seed, 0, pixel, uint32_t(sidx)), x, y);
-      V3 o, d;
-      cast_ray(cam, x, y, o, d);
-      int nb = 0;       // bounces with a hit
-      bool more = true;
-      for (int depth = 0; more && depth < kWhittedMaxBounces; ++depth) {
-        more = false;
-        // Integrator::Trace returns 0 past the cutoff (muon/integration.cc:29-33)
-        if (cutoff != INT_MAX && depth > cutoff) break;
-        if (depth == 0) ++n_primary;
-        else ++n_secondary;
-        const TraceRay r = make_ray(o, d);
-        float best = __builtin_inff();
-        const int32_t p = trace_bvh<STACK, false, true, true>(s, r, best, stack + threadIdx.x, kSimpleBlock, cnt);
-        if (p < 0) break;
-        const HitRecord h = hit_record(s, uint32_t(p), o, d);
-        const float *m = s.materials + size_t(s.prim_mat[p]) * kMatStride;
-        const V3 amb{m[0], m[1], m[2]}, kd{m[3], m[4], m[5]}, spec{m[6], m[7], m[8]}, em{m[9], m[10], m[11]};
-        const V3 shift = h.pos + kEps * h.normal;
-        V3 color;
-        if (integrator == MUONX_INTEGRATOR_RAYTRACER) {
-          color = amb + em;
-          for (uint32_t l = 0; l < s.num_lights; ++l) {
-            V3 lc, ldir;
-            float ldist;
-            shading_info(s.lights + size_t(l) * kLightStride, h.pos, lc, ldir, ldist);
-            ++n_shadow;
-            const TraceRay sr = make_ray(shift, ldir);
-            float sbest = ldist;
-            const int32_t occ = trace_bvh<STACK, true, true, true>(s, sr, sbest, stack + threadIdx.x, kSimpleBlock,
-                                                                   cnt);
-            if (occ >= 0) continue;
-            const V3 diffuse = kd * gmax(dot(h.normal, ldir), 0.0f);
-            const V3 half = normalize(ldir - d);
-            const V3 sp = spec * powf(gmax(dot(h.normal, half), 0.0f), m[12]);
-            color = color + lc * (diffuse + sp);
+  WaveFetch wf(items, kChunk);
+  uint32_t n_primary = 0, n_secondary = 0, n_shadow = 0;
+  ImageItem i;
+  int nb = 0;  // bounces with a hit (the depth of the next)
+  uint32_t light = 0;
+  int32_t prim = 0;
+  V3 d, color;
+  V3 pos, normal;  // the bounce's hit
+  V3 local[kWhittedMaxBounces], ks[kWhittedMaxBounces];
+  bool walking = false, have = false, drained = false, shadow = false;
+  while (true) {
+    const uint64_t needm = __builtin_amdgcn_ballot_w64(!have && !drained);
+    if (needm) {
+      const uint32_t k = wf.claim(needm, next);
+      if (!have && !drained) {
+        if (k >= items) {
+          drained = true;
+        } else if (image_item(it, k, i)) {
+          have = true;
+          nb = 0;
+          shadow = false;
+          w.hit = -1;
+          if (cutoff >= 0) {  // Integrator::Trace returns 0 past the cutoff (muon/integration.cc:29-33)
+            V3 o;
+            sample_ray(cam, i, seed, o, d);
+            ++n_primary;
+            walking = w.start(s, make_ray(o, d), __builtin_inff(), false, st, cnt);
           }
+        }
+      }
+    }
+    const uint64_t drainedm = __builtin_amdgcn_ballot_w64(drained);
+    if (__builtin_amdgcn_ballot_w64(have) == 0) {
+      if (~drainedm == 0) break;
+      continue;
+    }
+    run_walks(s, w, walking, st, cnt, __popcll(drainedm) + kWhittedRefill);
+    if (have && !walking) {
+      bool path_done = false;
+      const float *m = s.materials;
+      if (!shadow) {
+        if (w.hit < 0) {
+          path_done = true;
+        } else {
+          prim = w.hit;
+          const HitRecord h = hit_record(s, uint32_t(prim), w.r.o, d);
+          pos = h.pos;
+          normal = h.normal;
+          m += size_t(s.prim_mat[prim]) * kMatStride;
+          const V3 amb{m[0], m[1], m[2]}, kd{m[3], m[4], m[5]}, em{m[9], m[10], m[11]};
+          if (integrator == MUONX_INTEGRATOR_RAYTRACER) {
+            color = amb + em;
+            light = 0;
+            shadow = true;
+          } else {
+            color = em;
+            for (uint32_t l = 0; l < s.num_lights; ++l) {
+              const float *L = s.lights + size_t(l) * kLightStride;
+              if (int(L[0]) != MUONX_LIGHT_QUAD) continue;
+              const V3 c0{L[4], L[5], L[6]}, e0{L[7], L[8], L[9]}, e1{L[10], L[11], L[12]};
+              const V3 verts[4] = {c0, c0 + e0, (c0 + e0) + e1, c0 + e1};
+              const V3 brdf = kd * kOneOverPi;
+              const V3 radiance{L[1], L[2], L[3]};
+              V3 irr{0.0f, 0.0f, 0.0f};
+              for (int v = 0; v < 4; ++v) {
+                const int ni = (v + 1) % 4;
+                const V3 ui = normalize(verts[v] - pos);
+                const V3 un = normalize(verts[ni] - pos);
+                const float theta = acosf(dot(ui, un));
+                const V3 gamma = normalize(cross(ui, un));
+                irr = irr + theta * gamma;
+              }
+              irr = irr * 0.5f;
+              color = color + (brdf * radiance) * dot(irr, normal);
+            }
+            local[nb] = color;
+            ks[nb] = V3{0.0f, 0.0f, 0.0f};
+            ++nb;
+            path_done = true;
+          }
+        }
+      } else {
+        m += size_t(s.prim_mat[prim]) * kMatStride;
+        if (w.hit < 0) {  // light `light` is visible
+          const V3 kd{m[3], m[4], m[5]}, spec{m[6], m[7], m[8]};
+          V3 lc, ldir;
+          float ldist;
+          shading_info(s.lights + size_t(light) * kLightStride, pos, lc, ldir, ldist);
+          const V3 diffuse = kd * gmax(dot(normal, ldir), 0.0f);
+          const V3 half = normalize(ldir - d);
+          const V3 sp = spec * powf(gmax(dot(normal, half), 0.0f), m[12]);
+          color = color + lc * (diffuse + sp);
+        }
+        ++light;
+      }
+      if (shadow) {
+        const V3 shift = pos + kEps * normal;
+        if (light < s.num_lights) {
+          V3 lc, ldir;
+          float ldist;
+          shading_info(s.lights + size_t(light) * kLightStride, pos, lc, ldir, ldist);
+          ++n_shadow;
+          walking = w.start(s, make_ray(shift, ldir), ldist, true, st, cnt);
+        } else {
+          // the bounce is lit: reflect or end
+          const V3 spec{m[6], m[7], m[8]};
           local[nb] = color;
           ks[nb] = spec;
           ++nb;
-          if (spec.x > 0.0f || spec.y > 0.0f || spec.z > 0.0f) {
-            o = shift;
-            d = reflect(d, h.normal);
-            more = true;
+          shadow = false;
+          if ((spec.x > 0.0f || spec.y > 0.0f || spec.z > 0.0f) && nb < kWhittedMaxBounces && nb <= cutoff) {
+            d = reflect(d, normal);
+            ++n_secondary;
+            walking = w.start(s, make_ray(shift, d), __builtin_inff(), false, st, cnt);
+          } else {
+            path_done = true;
           }
-        } else {
-          color = em;
-          for (uint32_t l = 0; l < s.num_lights; ++l) {
-            const float *L = s.lights + size_t(l) * kLightStride;
-            if (int(L[0]) != MUONX_LIGHT_QUAD) continue;
-            const V3 c0{L[4], L[5], L[6]}, e0{L[7], L[8], L[9]}, e1{L[10], L[11], L[12]};
-            const V3 verts[4] = {c0, c0 + e0, (c0 + e0) + e1, c0 + e1};
-            const V3 brdf = kd * kOneOverPi;
-            const V3 radiance{L[1], L[2], L[3]};
-            V3 irr{0.0f, 0.0f, 0.0f};
-            for (int i = 0; i < 4; ++i) {
-              const int ni = (i + 1) % 4;
-              const V3 ui = normalize(verts[i] - h.pos);
-              const V3 un = normalize(verts[ni] - h.pos);
-              const float theta = acosf(dot(ui, un));
-              const V3 gamma = normalize(cross(ui, un));
-              irr = irr + theta * gamma;
-            }
-            irr = irr * 0.5f;
-            color = color + (brdf * radiance) * dot(irr, h.normal);
-          }
-          local[nb] = color;
-          ks[nb] = V3{0.0f, 0.0f, 0.0f};
-          ++nb;
         }
       }
-      V3 c{0.0f, 0.0f, 0.0f};
-      if (nb > 0) {
-        // color_d = local_d + ks_d * color_{d+1}, innermost first; a bounce
-        // whose reflected ray found nothing adds ks * 0
-        c = local[nb - 1];
-        if (ks[nb - 1].x > 0.0f || ks[nb - 1].y > 0.0f || ks[nb - 1].z > 0.0f) c = c + ks[nb - 1] * V3{0.0f, 0.0f, 0.0f};
-        for (int b = nb - 2; b >= 0; --b) c = local[b] + ks[b] * c;
+      if (path_done) {
+        V3 c{0.0f, 0.0f, 0.0f};
+        if (nb > 0) {
+          // color_d = local_d + ks_d * color_{d+1}, innermost first; a bounce
+          // whose reflected ray found nothing adds ks * 0
+          c = local[nb - 1];
+          if (ks[nb - 1].x > 0.0f || ks[nb - 1].y > 0.0f || ks[nb - 1].z > 0.0f) c = c + ks[nb - 1] * V3{0.0f, 0.0f, 0.0f};
+          for (int b = nb - 2; b >= 0; --b) c = local[b] + ks[b] * c;
+        }
+        write_sample(it, i, c, accum);
+        have = false;
       }
-      acc = acc + c;
     }
-    accum[3 * size_t(pixel)] = acc.x;
-    accum[3 * size_t(pixel) + 1] = acc.y;
-    accum[3 * size_t(pixel) + 2] = acc.z;
   }
+  rays += CounterSlot();
   wave_count(n_primary, &rays[kCtrPrimary]);
   wave_count(n_secondary, &rays[kCtrSecondary]);
   wave_count(n_shadow, &rays[kCtrShadow]);
@@ -227,50 +368,69 @@ __global__ void __launch_bounds__(kSimpleBlock) k_whitted(DevSceneView s, CamPar
   wave_count(cnt.bhits, &rays[kCtrBoundsHits]);
 }
 
-int RenderWhitted(muonx_scene *scene, const muonx_render_params &p, float *accum, unsigned long long *rays,
-                  hipStream_t stream) {
+// Blocks per CU of the image kernels. More than their registers let a CU hold
+// start late with a chunk of their own, which costs k_whitted (8, 10, 12: 2.20 /
+// 2.87 / 2.67 ms above) and helps k_simple's short wavefronts even out (8, 10,
+// 12: 668 / 725 / 615 us for the depth image).
+constexpr uint32_t kSimpleBlocksPerCu = 12, kWhittedBlocksPerCu = 8;
+// The most memory for a launch's samples.
+constexpr uint64_t kSampleBytes = uint64_t(64) << 20;
+
+// Runs one of the deterministic integrators; `counters` holds the trace
+// counters and the (cleared) claim counters.
+int RenderDeterministic(muonx_scene *scene, const muonx_render_params &p, float *accum, const RenderCounters &counters,
+                        DevBuf &samples, hipStream_t stream) {
   const DevSceneView &s = scene->view;
-  const CamParams cam = MakeCam(p);
-  const int cutoff =
-      p.max_depth == -1 ? INT_MAX : (p.nee != MUONX_NEE_OFF ? p.max_depth - 1 : p.max_depth);
-  const uint32_t npix = uint32_t(p.width) * uint32_t(p.height);
-  const dim3 grid((npix + kSimpleBlock - 1) / kSimpleBlock);
-#define MX_W(S)                                                                                                     \
-  hipLaunchKernelGGL(k_whitted<S>, grid, dim3(kSimpleBlock), 0, stream, s, cam, p.integrator, p.spp, cutoff, p.seed, \
-                     accum, rays)
-  if (s.bvh_depth <= 24) MX_W(24);
-  else if (s.bvh_depth <= 48) MX_W(48);
-  else if (s.bvh_depth <= 96) MX_W(96);
-  else {
+  if (s.bvh_depth > 96) {
     SetError("BVH too deep for the traversal stack");
     return MUONX_ERR_CAPACITY;
   }
-#undef MX_W
-  MX_HIP(hipGetLastError());
-  return MUONX_OK;
-}
-
-int RenderSimple(muonx_scene *scene, const muonx_render_params &p, float *accum, unsigned long long *rays,
-                 hipStream_t stream) {
-  const DevSceneView &s = scene->view;
   const CamParams cam = MakeCam(p);
-  // muon/integration.cc:29-33 applied at depth 0
-  const int cutoff = p.nee != MUONX_NEE_OFF ? p.max_depth - 1 : p.max_depth;
-  const int depth0_ok = (p.max_depth == -1 || 0 <= cutoff) ? 1 : 0;
-  const uint32_t npix = uint32_t(p.width) * uint32_t(p.height);
-  const dim3 grid((npix + kSimpleBlock - 1) / kSimpleBlock);
-  if (s.bvh_depth <= 24) {
-    hipLaunchKernelGGL(k_simple<24>, grid, dim3(kSimpleBlock), 0, stream, s, cam, p.integrator, p.spp, depth0_ok,
-                       p.seed, accum, rays);
-  } else if (s.bvh_depth <= 48) {
-    hipLaunchKernelGGL(k_simple<48>, grid, dim3(kSimpleBlock), 0, stream, s, cam, p.integrator, p.spp, depth0_ok,
-                       p.seed, accum, rays);
-  } else if (s.bvh_depth <= 96) {
-    hipLaunchKernelGGL(k_simple<96>, grid, dim3(kSimpleBlock), 0, stream, s, cam, p.integrator, p.spp, depth0_ok,
-                       p.seed, accum, rays);
-  } else {
-    SetError("BVH too deep for the traversal stack");
-    return MUONX_ERR_CAPACITY;
+  const uint64_t tiles = ((uint64_t(p.width) + 7) / 8) * ((uint64_t(p.height) + 7) / 8);
+  const uint32_t cus = uint32_t(scene->ctx->num_cus > 0 ? scene->ctx->num_cus : 256);
+  // samples per launch: their buffer stays within kSampleBytes
+  const uint64_t film = uint64_t(p.width) * uint64_t(p.height) * 3 * sizeof(float);
+  const int batch = int(std::max<uint64_t>(1, std::min<uint64_t>(uint64_t(p.spp), kSampleBytes / film)));
+  if (batch > 1) MX_HIP(samples.Reserve(film * uint64_t(batch)));
+  ImageItems it{uint32_t(p.width), uint32_t(p.height), (uint32_t(p.width) + 7u) >> 3, 0, 0, 0, samples.as<float>()};
+  unsigned long long *ctr = counters.trace;
+  uint32_t *next = counters.claims;
+  // muon/integration.cc:29-33
+  const int cutoff = p.max_depth == -1 ? INT_MAX : (p.nee != MUONX_NEE_OFF ? p.max_depth - 1 : p.max_depth);
+  const bool whitted = p.integrator == MUONX_INTEGRATOR_RAYTRACER || p.integrator == MUONX_INTEGRATOR_ANALYTICDIRECT;
+  bool cleared = true;  // the claim counters
+  for (it.first = 0; it.first < p.spp; it.first += it.count) {
+    it.count = std::min(batch, p.spp - it.first);
+    const uint64_t part = std::max<uint64_t>(1, (1u << 24) / uint64_t(it.count));  // tiles per launch: below 2^31 items
+    for (it.tile0 = 0; it.tile0 < tiles; it.tile0 += part) {
+      const uint32_t items = uint32_t(std::min(tiles - it.tile0, part)) * uint32_t(it.count) * 64u;
+      const uint32_t blocks = ClaimBlocks(items, cus * (whitted ? kWhittedBlocksPerCu : kSimpleBlocksPerCu), kSimpleBlock / 64);
+      if (NeedsClaims(items, blocks * (kSimpleBlock / 64))) {
+        if (!cleared) MX_HIP(hipMemsetAsync(next, 0, kClaimBytes, stream));
+        cleared = false;
+      }
+      const dim3 grid(blocks), block(kSimpleBlock);
+#define MX_IMAGE(CAP)                                                                                                \
+  if (whitted)                                                                                                       \
+    hipLaunchKernelGGL(k_whitted<CAP>, grid, block, 0, stream, s, cam, p.integrator, cutoff, p.seed, it, items, accum, \
+                       ctr, next);                                                                                   \
+  else                                                                                                               \
+    hipLaunchKernelGGL(k_simple<CAP>, grid, block, 0, stream, s, cam, p.integrator, cutoff >= 0 ? 1 : 0, p.seed, it,  \
+                       items, accum, ctr, next)
+      if (s.bvh_depth <= 24) {
+        MX_IMAGE(24);
+      } else if (s.bvh_depth <= 48) {
+        MX_IMAGE(48);
+      } else {
+        MX_IMAGE(96);
+      }
+#undef MX_IMAGE
+    }
+    if (it.count > 1) {
+      const uint64_t n = film / sizeof(float);
+      hipLaunchKernelGGL(k_sum_samples, dim3(uint32_t(std::min<uint64_t>(4096, (n + 255) / 256))), dim3(256), 0, stream,
+                         it.buffer, it.first, it.count, n, accum);
+    }
   }
   MX_HIP(hipGetLastError());
   return MUONX_OK;
@@ -305,25 +465,24 @@ extern "C" int muonx_render(muonx_scene *scene, const muonx_render_params *param
   MX_HIP(hipSetDevice(ctx->device));
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   RenderWorkspace *ws = GetWorkspace(ctx);
-  MX_HIP(ws->counters.Reserve(sizeof(unsigned long long) * kNumCounters));
-  MX_HIP(hipMemsetAsync(ws->counters.ptr, 0, sizeof(unsigned long long) * kNumCounters, stream));
+  MX_HIP(ws->counters.Reserve(kRenderCounterBytes));
+  MX_HIP(hipMemsetAsync(ws->counters.ptr, 0, kRenderCounterBytes, stream));
   hipEvent_t e0, e1;
   MX_HIP(hipEventCreate(&e0));
   MX_HIP(hipEventCreate(&e1));
   MX_HIP(hipEventRecord(e0, stream));
   int rc;
-  unsigned long long *ctr = ws->counters.as<unsigned long long>();
+  const RenderCounters ctr{ws->counters.as<unsigned long long>() + kClaimBytes / sizeof(unsigned long long),
+                           ws->counters.as<uint32_t>()};
   bool host_rays = false;
   unsigned long long rays[kEngineCounters] = {};
   switch (p.integrator) {
     case MUONX_INTEGRATOR_NORMALS:
     case MUONX_INTEGRATOR_ALBEDO:
     case MUONX_INTEGRATOR_DEPTH:
-      rc = RenderSimple(scene, p, accum, ctr, stream);
-      break;
     case MUONX_INTEGRATOR_RAYTRACER:
     case MUONX_INTEGRATOR_ANALYTICDIRECT:
-      rc = RenderWhitted(scene, p, accum, ctr, stream);
+      rc = RenderDeterministic(scene, p, accum, ctr, ws->samples, stream);
       break;
     case MUONX_INTEGRATOR_PATHTRACER:
       rc = RenderPathTracer(scene, p, accum, stream, rays);
@@ -340,8 +499,14 @@ extern "C" int muonx_render(muonx_scene *scene, const muonx_render_params *param
   }
   MX_HIP(hipEventRecord(e1, stream));
   if (stats) {
-    unsigned long long h[kNumCounters];
-    MX_HIP(hipMemcpyAsync(h, ws->counters.ptr, sizeof(h), hipMemcpyDeviceToHost, stream));
+    unsigned long long h[kNumCounters] = {};
+    if (!host_rays) {
+      std::vector<unsigned long long> slots(kTraceCounterBytes / sizeof(unsigned long long));
+      MX_HIP(hipMemcpyAsync(slots.data(), ctr.trace, kTraceCounterBytes, hipMemcpyDeviceToHost, stream));
+      MX_HIP(hipStreamSynchronize(stream));
+      for (uint32_t k = 0; k < kCounterSlots; ++k)
+        for (int c = 0; c < kNumCounters; ++c) h[c] += slots[size_t(k) * kCounterSlotStride + size_t(c)];
+    }
     MX_HIP(hipStreamSynchronize(stream));
     float ms = 0.0f;
     MX_HIP(hipEventElapsedTime(&ms, e0, e1));

@@ -310,35 +310,21 @@ struct PrivateStack {
   }
 };
 
-// Traverses the BVH. ANY: stop at the first primitive with 0 < dist < tmax
-// (HasIntersection); otherwise closest hit (Intersect). EXACT selects the
-// reference's division slab test (identical node visits, used by the
-// deterministic integrators and the exact query mode); the default is the
-// conservative reciprocal test. WW ("while-while"): each lane walks internal
-// nodes until it holds a leaf, then the wavefront tests leaves together,
-// instead of interleaving node and leaf steps lane by lane. Returns the
-// leaf-order primitive index or -1; `best` holds the distance on return.
-// One internal-node step: tests both child boxes, pushes the far child when
-// both are hit, and moves `ref` to the next node; returns false when the
-// stack is exhausted.
-template <bool COUNT, bool EXACT, class Stack>
-__device__ __forceinline__ bool node_step(const DevSceneView &s, const TraceRay &r, bool plain, float best,
-                                          Stack &stack, uint32_t &ref, TraceCounters &cnt) {
+// One internal-node step of the binary tree in the fast mode: tests both child
+// boxes, pushes the far child when both are hit, and moves `ref` to the next
+// node; returns false when no child is hit.
+template <bool COUNT, class Stack>
+__device__ __forceinline__ bool node_step(const DevSceneView &s, const TraceRay &r, float best, Stack &stack,
+                                          uint32_t &ref, TraceCounters &cnt) {
   const float4 *np = s.nodes + 4 * size_t(ref);
   const float4 n0 = ldg(np), n1 = ldg(np + 1), n2 = ldg(np + 2);
   const int4 n3 = ldg(reinterpret_cast<const int4 *>(np + 3));
   if (COUNT) cnt.nodes++;
   float lo0, lo1;
-  bool h0, h1;
-  if (EXACT) {
-    h0 = box_hit_exact(r, plain, n0.x, n0.y, n0.z, n0.w, n2.x, n2.y, best, lo0);
-    h1 = box_hit_exact(r, plain, n1.x, n1.y, n1.z, n1.w, n2.z, n2.w, best, lo1);
-  } else {
-    const float bm = below(best);
-    h0 = box_hit(r, n0.x, n0.y, n0.z, n0.w, n2.x, n2.y, bm, lo0);
-    h1 = box_hit(r, n1.x, n1.y, n1.z, n1.w, n2.z, n2.w, bm, lo1);
-  }
-  if (COUNT && !EXACT) {  // the fast mode's own work: both child boxes tested
+  const float bm = below(best);
+  const bool h0 = box_hit(r, n0.x, n0.y, n0.z, n0.w, n2.x, n2.y, bm, lo0);
+  const bool h1 = box_hit(r, n1.x, n1.y, n1.z, n1.w, n2.z, n2.w, bm, lo1);
+  if (COUNT) {  // the fast mode's own work: both child boxes tested
     cnt.btests += 2;
     cnt.bhits += uint32_t(h0) + uint32_t(h1);
   }
@@ -349,27 +335,6 @@ __device__ __forceinline__ bool node_step(const DevSceneView &s, const TraceRay 
   const bool hn = swap ? h1 : h0;
   const bool hf = swap ? h0 : h1;
   const float lof = swap ? lo0 : lo1;
-  if (COUNT && EXACT) {
-    // The reference (muon/acceleration.cc:137,197) always pushes the far
-    // child and tests its box only when it pops it, which an any-hit query
-    // that stops at its first hit (:182-183) never does. So with the near box hit the
-    // far child is pushed too, with an infinite key when its box was missed
-    // here, and its test is counted at its pop (pop_next_counted).
-    if (hn) {
-      cnt.btests++;
-      cnt.bhits++;
-      stack.push(make_uint2(far_ref, hf ? __float_as_uint(lof) : 0x7f800000u));
-      ref = near_ref;
-      return true;
-    }
-    cnt.btests += 2;  // the near box, then the far one popped at once
-    if (hf) {
-      cnt.bhits++;
-      ref = far_ref;
-      return true;
-    }
-    return false;
-  }
   if (hn) {
     if (hf) stack.push(make_uint2(far_ref, __float_as_uint(lof)));
     ref = near_ref;
@@ -388,23 +353,6 @@ __device__ __forceinline__ bool pop_next(Stack &stack, float best, uint32_t &ref
   while (!stack.empty()) {
     const uint2 e = stack.pop();
     if (__uint_as_float(e.y) < best) {
-      ref = e.x;
-      return true;
-    }
-  }
-  return false;
-}
-
-// pop_next for the counted exact traversal: every popped far child is the
-// reference's bounds test at its pop, a hit when its box still starts
-// before `best`.
-template <class Stack>
-__device__ __forceinline__ bool pop_next_counted(Stack &stack, float best, uint32_t &ref, TraceCounters &cnt) {
-  while (!stack.empty()) {
-    const uint2 e = stack.pop();
-    cnt.btests++;
-    if (__uint_as_float(e.y) < best) {
-      cnt.bhits++;
       ref = e.x;
       return true;
     }
@@ -439,77 +387,6 @@ __device__ __forceinline__ bool leaf_step(const DevSceneView &s, const TraceRay 
     if (left ? --left == 0u : (flags & 1u) != 0u) return false;
     ++i;
   }
-}
-
-// Traverses the BVH. ANY: stop at the first primitive with 0 < dist < tmax
-// (HasIntersection); otherwise closest hit (Intersect). EXACT selects the
-// reference's division slab test (identical node visits, used by the
-// deterministic integrators and the exact query mode); the default is the
-// conservative reciprocal test. WW ("while-while"): every lane walks
-// internal nodes until it holds a leaf, then the wavefront tests leaves
-// together; otherwise each iteration does one node or one leaf step per lane.
-// Returns the leaf-order primitive index or -1; `best` holds the distance.
-template <bool ANY, bool COUNT, bool EXACT, bool WW, class Stack>
-__device__ __forceinline__ int32_t trace_bvh_s(const DevSceneView &s, const TraceRay &r, float &best, Stack &stack,
-                                               TraceCounters &cnt) {
-  int32_t hit_prim = -1;
-  ObjCache oc;
-  oc.tid = -1;
-  const bool plain = EXACT && plain_ray(s, r);
-  uint32_t ref = 0;  // root: internal node 0
-  constexpr bool kRefStats = COUNT && EXACT;
-  if (kRefStats && s.linear) {
-    // Linear::Intersect tests every primitive and counts object tests and
-    // hits only; Linear::HasIntersection counts nothing
-    // (muon/acceleration.cc:14-45). The one leaf is node 0's first child.
-    if constexpr (ANY) {
-      TraceCounters none;
-      return trace_bvh_s<ANY, false, EXACT, WW>(s, r, best, stack, none);
-    }
-    ref = __float_as_uint(ldg(s.nodes + 3).x);
-  } else if (kRefStats) {
-    // The reference tests the root's box first (muon/acceleration.cc:92-99);
-    // here it is the union of node 0's child boxes. A ray that misses it
-    // misses every box below, so stopping changes no result. A root that is
-    // a leaf sits in node 0's first child (the second is a sentinel).
-    const float4 *np = s.nodes;
-    const float4 n0 = ldg(np), n1 = ldg(np + 1), n2 = ldg(np + 2);
-    float lo;
-    cnt.btests++;
-    if (!box_hit_exact(r, plain, fminf(n0.x, n1.x), fmaxf(n0.y, n1.y), fminf(n0.z, n1.z), fmaxf(n0.w, n1.w),
-                       fminf(n2.x, n2.z), fmaxf(n2.y, n2.w), best, lo))
-      return -1;
-    cnt.bhits++;
-    if (s.root_leaf) ref = __float_as_uint(np[3].x);
-  }
-  auto pop = [&](uint32_t &rf) {
-    if constexpr (kRefStats) return pop_next_counted(stack, best, rf, cnt);
-    else return pop_next(stack, best, rf);
-  };
-  if (WW) {
-    while (true) {
-      bool alive = true;
-      while (!(ref & kLeafBit)) {
-        if (!node_step<COUNT, EXACT>(s, r, plain, best, stack, ref, cnt) && !pop(ref)) {
-          alive = false;
-          break;
-        }
-      }
-      if (!alive) break;
-      if (leaf_step<ANY, COUNT>(s, r, best, ref, oc, hit_prim, cnt)) return hit_prim;
-      if (!pop(ref)) break;
-    }
-  } else {
-    while (true) {
-      if (!(ref & kLeafBit)) {
-        if (node_step<COUNT, EXACT>(s, r, plain, best, stack, ref, cnt)) continue;
-      } else {
-        if (leaf_step<ANY, COUNT>(s, r, best, ref, oc, hit_prim, cnt)) return hit_prim;
-      }
-      if (!pop(ref)) break;
-    }
-  }
-  return hit_prim;
 }
 
 // Makes a loaded value count as used at this point. A node's child
@@ -707,19 +584,26 @@ __device__ __forceinline__ bool fast_step(const DevSceneView &s, const TraceRay 
                                           Stack &stack, uint32_t &ref, TraceCounters &cnt) {
   if constexpr (NODES == kNodesWideQ) return qnode_step<COUNT, ANY>(s, r, bm, stack, ref, cnt);
   else if constexpr (NODES == kNodesWide) return wnode_step<COUNT>(s, r, bm, stack, ref, cnt);
-  else return node_step<COUNT, false>(s, r, false, best, stack, ref, cnt);
+  else return node_step<COUNT>(s, r, best, stack, ref, cnt);
 }
 
-// Closest / any hit over the wide BVH (fast mode only: children are visited
-// nearest first, so ties may resolve differently from the reference's order).
+// Closest / any hit over the nodes of a format (kNodes*; the wide ones visit
+// children nearest first, so ties may resolve differently from the
+// reference's order). ANY: stop at the first primitive with 0 < dist < tmax
+// (HasIntersection); otherwise closest hit (Intersect). WW ("while-while"):
+// every lane walks internal nodes until it holds a leaf, then the wavefront
+// tests leaves together; otherwise each iteration does one node or one leaf
+// step per lane. Returns the leaf-order primitive index or -1; `best` holds
+// the distance.
 template <int NODES, bool ANY, bool COUNT, bool WW, class Stack>
-__device__ __forceinline__ int32_t trace_bvh4_s(const DevSceneView &s, TraceRay r, float &best, Stack &stack,
-                                                TraceCounters &cnt) {
+__device__ __forceinline__ int32_t trace_fast(const DevSceneView &s, TraceRay r, float &best, Stack &stack,
+                                              TraceCounters &cnt) {
+  constexpr bool kWide = NODES != kNodesBinary;
   if (NODES == kNodesWideQ) clamp_inv(r);
   int32_t hit_prim = -1;
   ObjCache oc;
   oc.tid = -1;
-  uint32_t ref = 0;  // root: wide node 0
+  uint32_t ref = 0;  // root
   if (WW) {
     while (true) {
       bool alive = true;
@@ -730,7 +614,7 @@ __device__ __forceinline__ int32_t trace_bvh4_s(const DevSceneView &s, TraceRay 
         }
       }
       if (!alive) break;
-      if (leaf_step<ANY, COUNT, true>(s, r, best, ref, oc, hit_prim, cnt)) return hit_prim;
+      if (leaf_step<ANY, COUNT, kWide>(s, r, best, ref, oc, hit_prim, cnt)) return hit_prim;
       if (!pop_next(stack, best, ref)) break;
     }
   } else {
@@ -738,20 +622,12 @@ __device__ __forceinline__ int32_t trace_bvh4_s(const DevSceneView &s, TraceRay 
       if (!(ref & kLeafBit)) {
         if (fast_step<NODES, COUNT, ANY>(s, r, best, below(best), stack, ref, cnt)) continue;
       } else {
-        if (leaf_step<ANY, COUNT, true>(s, r, best, ref, oc, hit_prim, cnt)) return hit_prim;
+        if (leaf_step<ANY, COUNT, kWide>(s, r, best, ref, oc, hit_prim, cnt)) return hit_prim;
       }
       if (!pop_next(stack, best, ref)) break;
     }
   }
   return hit_prim;
-}
-
-// Dispatch on the node format (kNodes*).
-template <int WIDTH, bool ANY, bool COUNT, bool WW, class Stack>
-__device__ __forceinline__ int32_t trace_fast(const DevSceneView &s, const TraceRay &r, float &best, Stack &stack,
-                                              TraceCounters &cnt) {
-  if constexpr (WIDTH == kNodesBinary) return trace_bvh_s<ANY, COUNT, false, WW>(s, r, best, stack, cnt);
-  else return trace_bvh4_s<WIDTH, ANY, COUNT, WW>(s, r, best, stack, cnt);
 }
 
 // Resumable fast-mode walk of one lane, for kernels that hand a lane a new
@@ -820,14 +696,6 @@ __device__ __forceinline__ void run_walks(const DevSceneView &s, Walk &w, bool &
     if (walking && w.at_leaf()) walking = w.leaf(s, st, cnt);
     active = __builtin_amdgcn_ballot_w64(walking);
   } while (active && 64 - __popcll(active) < stop);
-}
-
-// Fixed LDS stack at stack[k * stride], k < STACK (STACK >= BVH depth).
-template <int STACK, bool ANY, bool COUNT, bool EXACT = false>
-__device__ __forceinline__ int32_t trace_bvh(const DevSceneView &s, const TraceRay &r, float &best, uint2 *stack,
-                                             int stride, TraceCounters &cnt) {
-  LdsStack<STACK> st(stack, stride);
-  return trace_bvh_s<ANY, COUNT, EXACT, false>(s, r, best, st, cnt);
 }
 
 }  // namespace muonx

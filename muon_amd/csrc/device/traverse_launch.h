@@ -73,11 +73,7 @@ inline int PlanTraverseShape(const muonx_tuning &t, int num_cus, uint32_t bvh_de
   const int cus = num_cus > 0 ? num_cus : 256;
   cfg.width = t.bvh_width != 4 ? kNodesBinary : (t.node_bits == 8 ? kNodesWideQ : kNodesWide);
   const int bpc = std::max(1, t.blocks_per_cu);
-  // enough wavefronts for each to hold a first chunk of the work (wave.h)
-  const uint32_t most = uint32_t(cus * bpc), wpb = uint32_t(block / 64);
-  const uint64_t waves =
-      work_items / FirstChunk(uint32_t(std::min<uint64_t>(work_items, UINT32_MAX)), most * wpb) + 1;
-  cfg.grid = int(std::max<uint64_t>(1, std::min<uint64_t>(most, (waves + wpb - 1) / wpb)));
+  cfg.grid = int(ClaimBlocks(work_items, uint32_t(cus * bpc), uint32_t(block / 64)));
   cfg.threads = cfg.grid * block;
   cfg.ww = t.while_while != 0;
   cfg.spill = nullptr;

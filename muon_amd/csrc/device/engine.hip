@@ -649,7 +649,7 @@ constexpr uint32_t kDoneTable = 64;  // per-block done-count entries (a power of
 // Adds each shaded path's NEE and MIS terms in a fixed order. A continuing
 // path's radiance moves to its place in the next queue; a finished path adds
 // it to the job's film and counts towards the job's done counter.
-__global__ void __launch_bounds__(kEngBlock) k_eng_retire(EngArgs a, int cur) {
+__global__ void __launch_bounds__(kRetireBlock) k_eng_retire(EngArgs a, int cur) {
   const uint32_t n = a.c->qcount[cur].v;
   const PathState &ps = a.st[cur];
   const PathState &pn = a.st[cur ^ 1];
@@ -661,7 +661,7 @@ __global__ void __launch_bounds__(kEngBlock) k_eng_retire(EngArgs a, int cur) {
     tcnt[k] = 0;
   }
   __syncthreads();
-  for (uint32_t base = blockIdx.x * kEngBlock; base < n; base += gridDim.x * kEngBlock) {
+  for (uint32_t base = blockIdx.x * kRetireBlock; base < n; base += gridDim.x * kRetireBlock) {
     const uint32_t i = base + threadIdx.x;
     bool fin = false;
     uint32_t js = 0xffffffffu;
@@ -935,7 +935,8 @@ struct IterLaunch {
       hipLaunchKernelGGL((k_eng_shadow<KIND, WW, WIDTH, COUNT>), grid, block, 0, st, a, sa, cur);
       hipLaunchKernelGGL((k_eng_mis<KIND, WW, WIDTH, COUNT>), grid, block, 0, st, a, sa, cur);
     }
-    hipLaunchKernelGGL(k_eng_retire, grid, block, 0, st, a, cur);
+    hipLaunchKernelGGL(k_eng_retire, dim3(std::max(1, cfg.grid * kEngBlock / kRetireBlock)), dim3(kRetireBlock), 0, st,
+                       a, cur);
     hipLaunchKernelGGL(k_eng_plan, dim3(1), dim3(64), 0, st, a, cur);
     hipLaunchKernelGGL(k_eng_fill, grid, block, 0, st, a, cur);
   }

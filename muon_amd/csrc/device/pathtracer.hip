@@ -98,7 +98,7 @@ int RunInline(Scheduler *s, const muonx_job *jobs, uint32_t n, muonx_job_result 
   std::vector<SchedJob> finished;
   finished.reserve(n);
   while (!s->Idle())
-    if ((rc = s->Step(&finished)) != MUONX_OK) return rc;
+    if ((rc = s->Step(&finished, true)) != MUONX_OK) return rc;
   if (results)
     for (const SchedJob &j : finished) results[j.ticket] = j.result;
   if (rays) std::memcpy(rays, s->rays(), kRayCounters * sizeof(unsigned long long));

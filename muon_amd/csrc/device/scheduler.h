@@ -90,7 +90,12 @@ class Scheduler {
   // in arrival order. A running job passed over kSlicePassLimit times by
   // newer work goes first (PickSlice), so no stream of new or smaller
   // requests starves it. Images do not depend on the slicing.
-  int Step(std::vector<SchedJob> *finished);
+  //
+  // `closed`: the caller submits nothing before the submitted jobs are done.
+  // A poll that starts with every one of their samples in the path queue and
+  // with bounded paths then launches the iterations that those paths need, no
+  // more, and waits for them (LastIteration).
+  int Step(std::vector<SchedJob> *finished, bool closed = false);
   bool Idle() const { return pending_.empty() && jobs_.empty(); }
   size_t pending() const { return pending_.size(); }
   size_t in_flight() const { return jobs_.size(); }
@@ -106,6 +111,7 @@ class Scheduler {
   int AdmitWork();
   int AdmitSlice(SchedJob &j);
   int Harvest(int b);
+  uint64_t LastIteration() const;
   int FinishResolves(std::vector<SchedJob> *finished, bool wait_all);
   void AdvanceWindow();
 

@@ -24,12 +24,12 @@
 //
 // Quantized wide BVH: the same nodes in 64 B = 4 x uint4, child planes as
 // 8-bit offsets from a per-node origin in steps of a per-axis power of two:
-//   q0 = (origin.xyz, biased exponents x | y << 8 | z << 16 | count << 24)
+//   q0 = (origin.xyz, step x)
 //   q1 = (min.x[4], min.y[4], min.z[4], max.x[4]) one byte per child
-//   q2 = (max.y[4], max.z[4], 0, 0)
+//   q2 = (max.y[4], max.z[4], step y, step z)
 //   q3 = child refs[4]
-// A decoded plane is origin + q * 2^e; every decoded box contains the float
-// box.
+// A decoded plane is origin + q * step; every decoded box contains the float
+// box, and an empty slot's box is inverted.
 //
 // Primitives (leaf order), 48 B = 3 x float4:
 //   tri:    (v0.xyz, tid)  (v1.xyz, 0)  (v2.xyz, 0)     object space

@@ -326,7 +326,7 @@ extern "C" int muonx_scene_create(muonx_ctx *ctx, const muonx_scene_desc *din, m
   int rc = MUONX_OK;
   // empty slots point at the sentinel primitive np (a one-primitive leaf in
   // either leaf encoding: count field 0, and the sentinel carries the end flag)
-  const std::vector<U4> qnodes = QuantizeWide(wnodes, kLeafBit | np);
+  const std::vector<U4> qnodes = DeviceSteps(QuantizeWide(wnodes, kLeafBit | np));
   std::vector<uint32_t> lprims;
   for (uint32_t k = 0; k < np; ++k)
     if (plight[k] >= 0) lprims.push_back(k);

@@ -299,6 +299,18 @@ inline std::vector<U4> QuantizeWide(const std::vector<F4> &w, uint32_t empty_ref
   return out;
 }
 
+// The quantized nodes as the device reads them: the steps 2^e as floats in
+// n0.w, n2.z and n2.w (the traversal shifts no exponents out), without the
+// count (an empty slot's box is inverted).
+inline std::vector<U4> DeviceSteps(std::vector<U4> q) {
+  for (size_t i = 0; i < q.size(); i += 4) {
+    const uint32_t e = q[i].w;
+    q[i].w = (e & 255u) << 23;
+    q[i + 2].z = ((e >> 8) & 255u) << 23;
+    q[i + 2].w = ((e >> 16) & 255u) << 23;
+  }
+  return q;
+}
 
 }  // namespace muonx
 

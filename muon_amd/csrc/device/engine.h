@@ -4,14 +4,14 @@
 //
 // Each iteration advances every queued path by one bounce:
 //   extend   closest hit of the queue's rays
-//   shade    emission and NEE shadow rays; then the MIS BRDF ray and the
+//   shade    emission, NEE shadow rays, the MIS BRDF ray and the
 //            continuation: a continuing path is appended to the next queue
 //            together with its state
 //   shadow   any hit of the compacted shadow rays
-//   mis      closest hit of the MIS rays
-//   retire   adds the NEE terms and, for MIS rays that hit a light, the
-//            weighted emission; continuing paths carry their radiance
-//            into the next queue, finished ones add it to their job's film
+//   mis      closest hit of the MIS rays; a light hit's weighted emission
+//   retire   adds the NEE and MIS terms; continuing paths carry their
+//            radiance into the next queue, finished ones add it to their
+//            job's film
 //   plan     decides how many new samples fit behind the continuing paths
 //   fill     appends camera samples of admitted jobs, in work order
 // so new jobs join between any two bounces (continuous batching). Path state
@@ -39,6 +39,7 @@ namespace muonx {
 constexpr int kEngBlock = 128;
 constexpr int kShadeBlock = 512;  // shade kernels: one queue-append atomic per block and append
 constexpr int kShadeWaves = kShadeBlock / 64;
+static_assert(BlockAppend3::kWaves == kShadeWaves, "one partial count per wavefront");
 // Retire kernel: a block adds its finished paths to their job's counter once,
 // and atomics on one address take 11.3 ns each, so with one job 4096 blocks of
 // 128 threads spent 46 us there (256x256 Cornell box, 16 spp: 37 us per
@@ -115,13 +116,21 @@ struct EngCounters {
   HotCounter64 ray_slots[kRayCounters][kRaySlots];
 };
 
-// Per-path state, struct of arrays over queue positions.
+// Per-path state, struct of arrays over queue positions. The depth and a
+// second copy of the job word travel in the ray's w components (q_ray), the
+// only state that extend reads.
 struct PathState {
-  uint32_t *job, *pixel, *ctr;
-  int32_t *depth;
-  float *rad, *thr;       // 3 per path
-  uint32_t *key_a, *key_b;  // the sample's random-stream key (path_key), set at fill
+  uint32_t *job;  // job word (slots of the job and its scene)
+  uint4 *meta;    // job word, draws so far, the sample's random-stream key (path_key)
+  float *thr;     // throughput, 3 per path
+  float4 *rad;    // radiance, pixel; moved by retire, not by shade
 };
+
+// nidx: the path's position in the next queue, or kPathEnds, and which of
+// the iteration's terms retire has to look for. Positions fit the 30 bits:
+// 2^30 paths would take 300 GB.
+constexpr uint32_t kPathNextMask = 0x3fffffffu, kPathEnds = kPathNextMask;
+constexpr uint32_t kPathHasMis = 0x40000000u, kPathHasShadow = 0x80000000u;
 
 struct EngArgs {
   const DevSceneView *scenes;
@@ -132,14 +141,14 @@ struct EngArgs {
   int kmax;
   EngCounters *c;
   PathState st[2];    // state of queue 0 / 1
-  float4 *q_ray[2];   // 2 per path: (o.xyz, 0), (d.xyz, 0)
+  float4 *q_ray[2];   // 2 per path: (o.xyz, job word), (d.xyz, depth)
   int32_t *hit_prim;  // closest hit of path i of the current queue
-  uint32_t *nidx;     // its position in the next queue, or ~0 when it ends
-  float4 *m_ray;      // MIS rays: (o.xyz, path index), (d.xyz, 0)
-  float *m_fac;       // MIS weight times the BRDF-sampled throughput
-  int32_t *m_hit;     // closest hit of the MIS ray, -1 for none
-  float4 *shift;      // origin of path i's shadow and MIS rays (xyz), material id (w)
-  float4 *hnorm;      // shading normal at path i's hit
+  uint32_t *nidx;     // its position in the next queue and flags (kPathNextMask)
+  // MIS rays: (o.xyz, path index), (d.xyz, tmax), (MIS weight times the
+  // BRDF-sampled throughput, job word)
+  float4 *m_ray;
+  float4 *m_add;      // path i's MIS term (xyz), when it has a MIS ray
+  float4 *shift;      // origin of path i's shadow rays (xyz), job word (w)
   // shadow rays, index k * capacity + i, and the queue of those to trace
   float4 *s_dir;      // (direction, tmax)
   float *s_contrib;

@@ -40,15 +40,14 @@ __global__ void __launch_bounds__(kEngBlock) k_eng_extend(EngArgs a, StackArgs s
   uint2 old[StackOf<KIND>::kPrivate];
   const uint32_t n = a.c->qcount[cur].v;
   const float4 *q = a.q_ray[cur];
-  const PathState &ps = a.st[cur];
   uint32_t prim_rays = 0, sec_rays = 0;
   TraceCounters c;
   for (uint32_t base = blockIdx.x * kEngBlock; base < n; base += gridDim.x * kEngBlock) {
     const uint32_t i = base + threadIdx.x;
     if (i < n) {
       const float4 qo = q[2 * i], qd = q[2 * i + 1];
-      const uint32_t jw = ps.job[i], js = PathJobSlot(jw);
-      const int depth = ps.depth[i];
+      const uint32_t jw = __float_as_uint(qo.w), js = PathJobSlot(jw);
+      const int depth = __float_as_int(qd.w);
       int32_t hit = -1;
       // Integrator::Trace returns 0 past the depth cutoff (muon/integration.cc:29-33)
       if (depth <= a.jobs[js].cutoff && depth < kMaxBounces) {
@@ -83,159 +82,63 @@ struct PathAhead {
   }
   __device__ __forceinline__ void next(const PathState &ps, const int32_t *hit_prim, uint32_t i, uint32_t n) {
     if (i < n) {
-      jw = ps.job[i];
+      jw = ps.meta[i].x;
       prim = hit_prim[i];
     }
   }
 };
 
-// PathTracer::Shade (muon/integration.cc:205-271) in two kernels, split where
-// the random draws of the light samples end, so each holds fewer registers:
-//   shade_light  hit record, emission, NEE shadow rays (ShadeDirectNEE)
-//   shade_bsdf   MIS BRDF ray (ShadeDirectImportanceSampling) and the
-//                continuation with Russian roulette (ShadeIndirect)
-__global__ void __launch_bounds__(kShadeBlock) __attribute__((amdgpu_waves_per_eu(4, 8)))
-    k_eng_shade_light(EngArgs a, int cur) {
-  __shared__ uint32_t wsum[kShadeWaves + 1];
-  const uint32_t n = a.c->qcount[cur].v;
-  const float4 *q = a.q_ray[cur];
-  const PathState &ps = a.st[cur];
-  const size_t P = a.capacity;
-  const uint32_t stride = gridDim.x * kShadeBlock;
-  PathAhead ahead(ps, a.hit_prim, blockIdx.x * kShadeBlock + threadIdx.x, n);
-  for (uint32_t base = blockIdx.x * kShadeBlock; base < n; base += stride) {
-    const uint32_t i = base + threadIdx.x;
-    const uint32_t jw = ahead.jw;
-    const int32_t prim = ahead.prim;
-    ahead.next(ps, a.hit_prim, i + stride, n);
-    uint32_t nshadow = 0;
-    uint64_t vmask = 0;  // valid shadow rays k < 64
-    int K = 0;
-    if (i < n) {
-      const JobDev job = a.jobs[PathJobSlot(jw)];
-      const int depth = ps.depth[i];
-      K = job.K;
-      for (int k = 0; k < K; ++k) {
-        a.s_vis[k * P + i] = 0;
-        a.s_valid[k * P + i] = 0;
-      }
-      a.m_hit[i] = -1;
-      if (prim >= 0) {
-        const DevSceneView s = a.scenes[PathSceneSlot(jw)];
-        const float4 qo = q[2 * i], qd = q[2 * i + 1];
-        const V3 ro{qo.x, qo.y, qo.z}, rd{qd.x, qd.y, qd.z};
-        const HitRecord h = hit_record(s, uint32_t(prim), ro, rd);
-        const int32_t mi = ldg(s.prim_mat + prim);
-        const V3 shift = h.pos + kEps * h.normal;
-        // the hit for shade_bsdf: shadow/MIS origin + material, normal
-        a.shift[i] = make_float4(shift.x, shift.y, shift.z, __int_as_float(mi));
-        a.hnorm[i] = make_float4(h.normal.x, h.normal.y, h.normal.z, 0.0f);
-        if (depth >= job.min_depth) {
-          const Mat m = load_mat(s.materials + size_t(mi) * kMatStride);
-          const V3 T{ps.thr[3 * i], ps.thr[3 * i + 1], ps.thr[3 * i + 2]};
-          V3 rad{ps.rad[3 * i], ps.rad[3 * i + 1], ps.rad[3 * i + 2]};
-          // emission (muon/integration.cc:257-264)
-          if (!((job.nee != MUONX_NEE_OFF && depth > 0) || dot(h.normal, -rd) < 0.0f)) rad = rad + T * m.emission;
-          ps.rad[3 * i] = rad.x;
-          ps.rad[3 * i + 1] = rad.y;
-          ps.rad[3 * i + 2] = rad.z;
-          if (job.nee != MUONX_NEE_OFF) {
-            // ShadeDirectNEE (muon/integration.cc:340-466): one shadow ray per light sample
-            const PathKey key{ps.key_a[i], ps.key_b[i]};
-            uint32_t ctr = ps.ctr[i];
-            const bool mis = job.nee == MUONX_NEE_MIS;
-            int k = 0;
-            for (uint32_t l = 0; l < s.num_lights; ++l) {
-              const float *L = s.lights + size_t(l) * kLightStride;
-              const int kind = int(ldg(L));
-              if (kind != MUONX_LIGHT_QUAD) {
-                V3 ldir, col{ldg(L + 1), ldg(L + 2), ldg(L + 3)};
-                float ldist;
-                if (kind == MUONX_LIGHT_POINT) {
-                  const V3 to_light = V3{ldg(L + 4), ldg(L + 5), ldg(L + 6)} - h.pos;
-                  ldir = est_normalize(to_light);
-                  ldist = est_length(to_light);
-                  const float att = ldg(L + 7) + ldg(L + 8) * ldist + ldg(L + 9) * ldist * ldist;
-                  col = est_div(col, att);
-                } else {
-                  ldir = V3{ldg(L + 4), ldg(L + 5), ldg(L + 6)};
-                  ldist = __builtin_inff();
-                }
-                V3 irr = col;
-                if (ldist < __builtin_inff()) irr = est_div(irr, ldist * ldist);
-                const float cosi = gmax(dot(h.normal, ldir), 0.0f);
-                const V3 contrib = T * (irr * cosi * brdf_eval(m, ldir, rd, h.normal));
-                const size_t sl = k * P + i;
-                a.s_contrib[3 * sl] = contrib.x;
-                a.s_contrib[3 * sl + 1] = contrib.y;
-                a.s_contrib[3 * sl + 2] = contrib.z;
-                a.s_dir[sl] = make_float4(ldir.x, ldir.y, ldir.z, ldist);
-                // a zero contribution cannot change the image: its ray is skipped
-                const uint8_t valid = (contrib.x != 0.0f || contrib.y != 0.0f || contrib.z != 0.0f) ? 1 : 0;
-                a.s_valid[sl] = valid;
-                nshadow += valid;
-                if (valid && k < 64) vmask |= 1ull << k;
-                ++k;
-                continue;
-              }
-              const QuadLight ql = load_quad(L);
-              const V3 rn = est_normalize(cross(ql.e0, ql.e1));
-              const float scale = est_div(ql.area, float(job.light_samples));
-              const float cell = est_rcp(float(job.strata));
-              for (int si = 0; si < job.strata; ++si) {
-                for (int sj = 0; sj < job.strata; ++sj) {
-                  for (int sk = 0; sk < job.per_section; ++sk) {
-                    const float u = rng_uniform(key, ctr);
-                    const float v = rng_uniform(key, ctr);
-                    V3 lp = (ql.corner + ((float(si) + u) * cell) * ql.e0) + ((float(sj) + v) * cell) * ql.e1;
-                    lp = lp - kEps * rn;
-                    const V3 to_light = lp - shift;
-                    const V3 ldir = est_normalize(to_light);
-                    const float ldist = est_length(to_light);
-                    const float cosi = gmax(dot(h.normal, ldir), 0.0f);
-                    const float cosl = gmax(dot(rn, ldir), 0.0f);
-                    const float g = est_div(cosi * cosl, ldist * ldist);
-                    V3 c = g * brdf_eval(m, ldir, rd, h.normal);
-                    if (mis) {
-                      const float lpdf = nee_pdf(s, shift, ldir);
-                      const float bpdf = is_pdf(job.is_mode, m, ldir, rd, h.normal);
-                      c = c * power_heuristic(lpdf, bpdf);
-                    }
-                    const V3 contrib = T * (ql.color * (c * scale));
-                    const size_t sl = k * P + i;
-                    a.s_contrib[3 * sl] = contrib.x;
-                    a.s_contrib[3 * sl + 1] = contrib.y;
-                    a.s_contrib[3 * sl + 2] = contrib.z;
-                    a.s_dir[sl] = make_float4(ldir.x, ldir.y, ldir.z, ldist);
-                    const uint8_t valid = (contrib.x != 0.0f || contrib.y != 0.0f || contrib.z != 0.0f) ? 1 : 0;
-                    a.s_valid[sl] = valid;
-                    nshadow += valid;
-                    if (valid && k < 64) vmask |= 1ull << k;
-                    ++k;
-                  }
-                }
-              }
-            }
-            ps.ctr[i] = ctr;
-          }
-        }
-      }
-    }
-    // the shadow rays to trace, compacted (zero contributions are skipped)
-    uint32_t si = block_append_n<kShadeWaves>(nshadow, &a.c->shadow_count.v, wsum);
-    for (uint64_t m = vmask; m; m &= m - 1)
-      a.s_queue[si++] = ShadowSlot(uint32_t(__ffsll((unsigned long long)m) - 1), a.capacity, i);
-    for (int k = 64; nshadow && k < K; ++k) {
-      const uint32_t sl = ShadowSlot(uint32_t(k), a.capacity, i);
-      if (a.s_valid[sl]) a.s_queue[si++] = sl;
-    }
-  }
-}
+// Makes the compiler take `v` as a new value: what is computed from it inside
+// a loop stays there instead of being held in registers around the loop.
+__device__ __forceinline__ void fresh(V3 &v) { asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z)); }
 
+// A vertex's shadow rays as its light samples make them: contributions and
+// directions go to memory as they come (a zero contribution cannot change the
+// image: its ray is skipped and nothing of it is stored), the mask of the
+// rays to trace stays in registers.
+struct ShadowRays {
+  uint32_t n = 0;
+  uint64_t mask = 0;  // rays to trace, k < 64
+  int k = 0;
+  __device__ __forceinline__ void add(const EngArgs &a, size_t i, V3 contrib, V3 dir, float dist) {
+    const bool valid = contrib.x != 0.0f || contrib.y != 0.0f || contrib.z != 0.0f;
+    const size_t sl = k * size_t(a.capacity) + i;
+    if (valid) {
+      a.s_contrib[3 * sl] = contrib.x;
+      a.s_contrib[3 * sl + 1] = contrib.y;
+      a.s_contrib[3 * sl + 2] = contrib.z;
+      a.s_dir[sl] = make_float4(dir.x, dir.y, dir.z, dist);
+      ++n;
+      if (k < 64) mask |= 1ull << k;
+    }
+    if (k >= 64) a.s_valid[sl] = valid;
+    ++k;
+  }
+};
+
+// PathTracer::Shade (muon/integration.cc:205-271): hit record and emission;
+// with NEE the shadow rays of the light samples (ShadeDirectNEE) and the MIS
+// BRDF ray (ShadeDirectImportanceSampling); then the continuation with
+// Russian roulette (ShadeIndirect). NEE = false is for an iteration in which
+// no admitted job has NEE on: the same arithmetic and random draws for such a
+// path (no light samples, no MIS sample), so a path's result does not depend
+// on which of the two ran.
+// Bound by memory and by the chain of fetches each path starts with. Split at
+// the light samples, as two kernels, the hit record went through memory and
+// the state was read twice: 1225 us per iteration of the level-7 icosphere
+// (512x512, 64 spp, NEE) against 893 for one kernel that leaves a path's
+// radiance to retire and stores nothing for a path without shadow or MIS
+// rays; without NEE 374 -> 309 us (sphere field, 1024x1024, 32 spp). The one
+// kernel holds 128 VGPRs, four waves per SIMD, without spills because each
+// light kind shares one BRDF evaluation, both BRDF samples share one loop,
+// the scene view is read where it is used, and `fresh` keeps what a BRDF
+// needs per vertex from being computed ahead of the light loop (all of that
+// apart: 192 B of spills and the Cornell box 1499 instead of 1256 us).
+template <bool NEE>
 __global__ void __launch_bounds__(kShadeBlock) __attribute__((amdgpu_waves_per_eu(4, 8)))
-    k_eng_shade_bsdf(EngArgs a, int cur) {
-  __shared__ uint32_t wsum[kShadeWaves + 1];
-  uint32_t culled_n = 0;
+    k_eng_shade(EngArgs a, int cur) {
+  __shared__ uint32_t sums[2][BlockAppend3::kWords];
+  uint32_t culled_n = 0, pass = 0;
   const uint32_t n = a.c->qcount[cur].v;
   const float4 *q = a.q_ray[cur];
   float4 *qn = a.q_ray[cur ^ 1];
@@ -243,75 +146,132 @@ __global__ void __launch_bounds__(kShadeBlock) __attribute__((amdgpu_waves_per_e
   const PathState &pn = a.st[cur ^ 1];
   const uint32_t stride = gridDim.x * kShadeBlock;
   PathAhead ahead(ps, a.hit_prim, blockIdx.x * kShadeBlock + threadIdx.x, n);
-  for (uint32_t base = blockIdx.x * kShadeBlock; base < n; base += stride) {
+  for (uint32_t base = blockIdx.x * kShadeBlock; base < n; base += stride, pass ^= 1) {
     const uint32_t i = base + threadIdx.x;
     const uint32_t jw = ahead.jw;
     const int32_t prim = ahead.prim;
     ahead.next(ps, a.hit_prim, i + stride, n);
-    bool cont = false, want_mis = false, culled = false;
-    uint32_t js = 0, pixel = 0, ctr = 0;
+    bool cont = false, want_mis = false;
+    ShadowRays sh;
+    uint32_t ctr = 0;
     PathKey key{0u, 0u};
-    int depth = 0;
+    int depth = 0, K = 0;
     float mis_tmax = __builtin_inff();
-    V3 shift{0, 0, 0}, next_dir{0, 0, 0}, mis_dir{0, 0, 0}, T{0, 0, 0};
+    V3 shift{0, 0, 0}, next_dir{0, 0, 0}, mis_dir{0, 0, 0}, mis_fac{0, 0, 0}, T{0, 0, 0};
     if (i < n && prim >= 0) {
-      js = jw;  // the job word: a continuing path carries it on
-      const JobDev job = a.jobs[PathJobSlot(js)];
-      const DevSceneView s = a.scenes[PathSceneSlot(js)];
-      depth = ps.depth[i];
-      const float4 sh = a.shift[i], hn = a.hnorm[i];
-      shift = V3{sh.x, sh.y, sh.z};
-      const V3 normal{hn.x, hn.y, hn.z};
-      const Mat m = load_mat(s.materials + size_t(__float_as_int(sh.w)) * kMatStride);
-      const float4 qd = q[2 * i + 1];
-      const V3 rd{qd.x, qd.y, qd.z};
-      pixel = ps.pixel[i];
-      key = PathKey{ps.key_a[i], ps.key_b[i]};
-      ctr = ps.ctr[i];
+      const JobDev &job = a.jobs[PathJobSlot(jw)];
+      const DevSceneView &s = a.scenes[PathSceneSlot(jw)];
+      const float4 qo = q[2 * i], qd = q[2 * i + 1];
+      depth = __float_as_int(qd.w);
+      const V3 ro{qo.x, qo.y, qo.z};
+      V3 rd{qd.x, qd.y, qd.z};
+      HitRecord h = hit_record(s, uint32_t(prim), ro, rd);
+      const float *mat = s.materials + size_t(ldg(s.prim_mat + prim)) * kMatStride;
+      shift = h.pos + kEps * h.normal;
+      const uint4 meta = ps.meta[i];
+      ctr = meta.y;
+      key = PathKey{meta.z, meta.w};
       T = V3{ps.thr[3 * i], ps.thr[3 * i + 1], ps.thr[3 * i + 2]};
-      if (depth >= job.min_depth && job.nee == MUONX_NEE_MIS) {
-        // ShadeDirectImportanceSampling (muon/integration.cc:468-501)
-        V3 dir, nT;
-        float bpdf;
-        if (sample_reflection(job.is_mode, m, rd, normal, T, key, ctr, dir, bpdf, nT)) {
-          const float lpdf = nee_pdf(s, shift, dir);
-          const V3 f = nT * power_heuristic(bpdf, lpdf);
-          a.m_fac[3 * i] = f.x;
-          a.m_fac[3 * i + 1] = f.y;
-          a.m_fac[3 * i + 2] = f.z;
-          want_mis = true;
-          mis_dir = dir;
-          if (s.cull_mis) {
-            // The term is nonzero only when the ray's closest hit is an
-            // emitting primitive. Test the few emitters with the traversal's
-            // own primitive test: a ray that hits none is settled here (no
-            // light hit, m_hit stays -1); otherwise the traversal only needs
-            // to look up to the nearest emitter hit.
-            const TraceRay mr = make_ray(shift, dir);
-            ObjCache oc;
-            oc.tid = -1;
-            float dmin = __builtin_inff(), blo;
-            const float *lb = s.light_box;
-            if (box_hit(mr, lb[0], lb[3], lb[1], lb[4], lb[2], lb[5], __builtin_inff(), blo)) {
-              for (uint32_t k = 0; k < s.num_light_prims; ++k) {
-                float dist;
-                uint32_t flags;
-                if (prim_hit(s, ldg(s.light_prims + k), mr, oc, dist, flags) && dist > 0.0f && dist < dmin) dmin = dist;
+      const int nee = NEE ? job.nee : int(MUONX_NEE_OFF);
+      const bool direct = depth >= job.min_depth;
+      if (direct && !((nee != MUONX_NEE_OFF && depth > 0) || dot(h.normal, -rd) < 0.0f)) {
+        // emission (muon/integration.cc:257-264); a zero term leaves the
+        // radiance, which is never -0, as it is
+        const V3 e = T * V3{ldg(mat + 9), ldg(mat + 10), ldg(mat + 11)};
+        if (e.x != 0.0f || e.y != 0.0f || e.z != 0.0f) {
+          float4 r = ps.rad[i];
+          r.x = r.x + e.x;
+          r.y = r.y + e.y;
+          r.z = r.z + e.z;
+          ps.rad[i] = r;
+        }
+      }
+      Mat m = load_mat(mat);
+      if (NEE && direct && nee != MUONX_NEE_OFF) {
+        // ShadeDirectNEE (muon/integration.cc:340-466): one shadow ray per light sample
+        const bool mis = nee == MUONX_NEE_MIS;
+        K = job.K;
+        for (uint32_t l = 0; l < s.num_lights; ++l) {
+          const float *L = s.lights + size_t(l) * kLightStride;
+          const int kind = int(ldg(L));
+          const bool quad = kind == MUONX_LIGHT_QUAD;
+          const int strata = quad ? job.strata : 1, per_section = quad ? job.per_section : 1;
+          for (int si = 0; si < strata; ++si) {
+            for (int sj = 0; sj < strata; ++sj) {
+              for (int sk = 0; sk < per_section; ++sk) {
+                fresh(h.normal);
+                fresh(rd);
+                fresh(m.diffuse);
+                fresh(m.specular);
+                V3 ldir, w{ldg(L + 1), ldg(L + 2), ldg(L + 3)};  // the light's color
+                float ldist, g = 0.0f;
+                if (quad) {
+                  const QuadLight ql = load_quad(L);
+                  const V3 rn = est_normalize(cross(ql.e0, ql.e1));
+                  const float cell = est_rcp(float(job.strata));
+                  const float u = rng_uniform(key, ctr);
+                  const float v = rng_uniform(key, ctr);
+                  V3 lp = (ql.corner + ((float(si) + u) * cell) * ql.e0) + ((float(sj) + v) * cell) * ql.e1;
+                  lp = lp - kEps * rn;
+                  const V3 to_light = lp - shift;
+                  ldir = est_normalize(to_light);
+                  ldist = est_length(to_light);
+                  const float cosi = gmax(dot(h.normal, ldir), 0.0f);
+                  const float cosl = gmax(dot(rn, ldir), 0.0f);
+                  g = est_div(cosi * cosl, ldist * ldist);
+                } else {
+                  if (kind == MUONX_LIGHT_POINT) {
+                    const V3 to_light = V3{ldg(L + 4), ldg(L + 5), ldg(L + 6)} - h.pos;
+                    ldir = est_normalize(to_light);
+                    ldist = est_length(to_light);
+                    const float att = ldg(L + 7) + ldg(L + 8) * ldist + ldg(L + 9) * ldist * ldist;
+                    w = est_div(w, att);
+                  } else {
+                    ldir = V3{ldg(L + 4), ldg(L + 5), ldg(L + 6)};
+                    ldist = __builtin_inff();
+                  }
+                  if (ldist < __builtin_inff()) w = est_div(w, ldist * ldist);
+                  w = w * gmax(dot(h.normal, ldir), 0.0f);
+                }
+                const V3 f = brdf_eval(m, ldir, rd, h.normal);
+                if (quad) {
+                  V3 c = g * f;
+                  if (mis) {
+                    const float lpdf = nee_pdf(s, shift, ldir);
+                    const float bpdf = is_pdf(job.is_mode, m, ldir, rd, h.normal);
+                    c = c * power_heuristic(lpdf, bpdf);
+                  }
+                  w = w * (c * est_div(ldg(L + 15), float(job.light_samples)));  // area / samples
+                } else {
+                  w = w * f;
+                }
+                sh.add(a, i, T * w, ldir, ldist);
               }
-            }
-            if (dmin == __builtin_inff()) {
-              want_mis = false;
-              culled = true;
-            } else {
-              mis_tmax = dmin * kWidenHi;
             }
           }
         }
+        if (sh.n) {
+          a.shift[i] = make_float4(shift.x, shift.y, shift.z, __uint_as_float(jw));
+          for (int k = 0; k < K; ++k) {  // retire reads all K flags; the traced rays' are set by the shadow kernel
+            const size_t sl = k * size_t(a.capacity) + i;
+            if (!(k < 64 ? (sh.mask >> k) & 1ull : uint64_t(a.s_valid[sl]))) a.s_vis[sl] = 0;
+          }
+        }
       }
-      // ShadeIndirect (muon/integration.cc:294-328)
-      V3 dir, nT;
-      float pdf;
-      if (sample_reflection(job.is_mode, m, rd, normal, T, key, ctr, dir, pdf, nT)) {
+      // One loop over the MIS BRDF ray (ShadeDirectImportanceSampling,
+      // muon/integration.cc:468-501) and the continuation (ShadeIndirect,
+      // muon/integration.cc:294-328): both sample the BRDF.
+#pragma unroll 1
+      for (int r = NEE && direct && nee == MUONX_NEE_MIS ? 0 : 1; r < 2; ++r) {
+        V3 dir, nT;
+        float pdf;
+        if (!sample_reflection(job.is_mode, m, rd, h.normal, T, key, ctr, dir, pdf, nT)) continue;
+        if (NEE && r == 0) {
+          mis_fac = nT * power_heuristic(pdf, nee_pdf(s, shift, dir));
+          mis_dir = dir;
+          want_mis = true;
+          continue;
+        }
         bool alive = true;
         if (job.rr) {
           const float qc = gmin(gmax(gmax(nT.x, nT.y), nT.z), 1.0f);
@@ -325,124 +285,74 @@ __global__ void __launch_bounds__(kShadeBlock) __attribute__((amdgpu_waves_per_e
           T = nT;
         }
       }
-    }
-    // a continuing path moves to the next queue with its state; its radiance
-    // follows in retire, after the NEE / MIS terms are added
-    const uint32_t ni = block_append<kShadeWaves>(cont, &a.c->qcount[cur ^ 1].v, wsum);
-    if (i < n) a.nidx[i] = cont ? ni : 0xffffffffu;
-    if (cont) {
-      qn[2 * ni] = make_float4(shift.x, shift.y, shift.z, 0.0f);
-      qn[2 * ni + 1] = make_float4(next_dir.x, next_dir.y, next_dir.z, 0.0f);
-      pn.job[ni] = js;
-      pn.pixel[ni] = pixel;
-      pn.ctr[ni] = ctr;
-      pn.key_a[ni] = key.a;
-      pn.key_b[ni] = key.b;
-      pn.depth[ni] = depth + 1;
-      pn.thr[3 * ni] = T.x;
-      pn.thr[3 * ni + 1] = T.y;
-      pn.thr[3 * ni + 2] = T.z;
-    }
-    const uint32_t mi = block_append<kShadeWaves>(want_mis, &a.c->mis_count.v, wsum);
-    if (want_mis) {
-      a.m_ray[2 * mi] = make_float4(shift.x, shift.y, shift.z, __uint_as_float(i));
-      a.m_ray[2 * mi + 1] = make_float4(mis_dir.x, mis_dir.y, mis_dir.z, mis_tmax);
-    }
-    culled_n += culled ? 1u : 0u;
-  }
-  // settled MIS rays count as traced secondary rays (the reference traces them)
-  ray_count(a.c, 1, culled_n);
-  ray_count(a.c, 3, culled_n);
-}
-
-// PathTracer::Shade without next-event estimation (muon/integration.cc:205-271
-// with NEE off: emission, then ShadeIndirect with Russian roulette) in one
-// kernel, used for an iteration in which no admitted job has NEE on. The
-// split kernels above do the same arithmetic and draw the same random numbers
-// for such a path (shade_light draws none without NEE, shade_bsdf skips its
-// MIS sample), so a path's result does not depend on which pair ran; this
-// one skips the hit-record hand-off through memory and the shadow and MIS
-// traversals, which would have no rays.
-__global__ void __launch_bounds__(kShadeBlock) __attribute__((amdgpu_waves_per_eu(4, 8)))
-    k_eng_shade_plain(EngArgs a, int cur) {
-  __shared__ uint32_t wsum[kShadeWaves + 1];
-  const uint32_t n = a.c->qcount[cur].v;
-  const float4 *q = a.q_ray[cur];
-  float4 *qn = a.q_ray[cur ^ 1];
-  const PathState &ps = a.st[cur];
-  const PathState &pn = a.st[cur ^ 1];
-  const uint32_t stride = gridDim.x * kShadeBlock;
-  PathAhead ahead(ps, a.hit_prim, blockIdx.x * kShadeBlock + threadIdx.x, n);
-  for (uint32_t base = blockIdx.x * kShadeBlock; base < n; base += stride) {
-    const uint32_t i = base + threadIdx.x;
-    const uint32_t jw = ahead.jw;
-    const int32_t prim = ahead.prim;
-    ahead.next(ps, a.hit_prim, i + stride, n);
-    bool cont = false;
-    uint32_t js = 0, pixel = 0, ctr = 0;
-    PathKey key{0u, 0u};
-    int depth = 0;
-    V3 shift{0, 0, 0}, next_dir{0, 0, 0}, T{0, 0, 0};
-    if (i < n) {
-      a.m_hit[i] = -1;  // retire: no MIS term
-      if (prim >= 0) {
-        js = jw;  // the job word: a continuing path carries it on
-        const JobDev job = a.jobs[PathJobSlot(js)];
-        const DevSceneView s = a.scenes[PathSceneSlot(js)];
-        depth = ps.depth[i];
-        const float4 qo = q[2 * i], qd = q[2 * i + 1];
-        const V3 ro{qo.x, qo.y, qo.z}, rd{qd.x, qd.y, qd.z};
-        const HitRecord h = hit_record(s, uint32_t(prim), ro, rd);
-        const int32_t mi = ldg(s.prim_mat + prim);
-        shift = h.pos + kEps * h.normal;
-        const Mat m = load_mat(s.materials + size_t(mi) * kMatStride);
-        T = V3{ps.thr[3 * i], ps.thr[3 * i + 1], ps.thr[3 * i + 2]};
-        if (depth >= job.min_depth && !(dot(h.normal, -rd) < 0.0f)) {
-          // emission (muon/integration.cc:257-264)
-          const V3 rad = V3{ps.rad[3 * i], ps.rad[3 * i + 1], ps.rad[3 * i + 2]} + T * m.emission;
-          ps.rad[3 * i] = rad.x;
-          ps.rad[3 * i + 1] = rad.y;
-          ps.rad[3 * i + 2] = rad.z;
+      if (NEE && want_mis && s.cull_mis) {
+        // The MIS term is nonzero only when the ray's closest hit is an
+        // emitting primitive. Test the few emitters with the traversal's
+        // own primitive test: a ray that hits none is settled here (no
+        // light hit); otherwise the traversal only needs to look up to
+        // the nearest emitter hit.
+        const TraceRay mr = make_ray(shift, mis_dir);
+        ObjCache oc;
+        oc.tid = -1;
+        float dmin = __builtin_inff(), blo;
+        const float *lb = s.light_box;
+        if (box_hit(mr, lb[0], lb[3], lb[1], lb[4], lb[2], lb[5], __builtin_inff(), blo)) {
+          for (uint32_t k = 0; k < s.num_light_prims; ++k) {
+            float dist;
+            uint32_t flags;
+            if (prim_hit(s, ldg(s.light_prims + k), mr, oc, dist, flags) && dist > 0.0f && dist < dmin) dmin = dist;
+          }
         }
-        pixel = ps.pixel[i];
-        key = PathKey{ps.key_a[i], ps.key_b[i]};
-        ctr = ps.ctr[i];
-        // ShadeIndirect (muon/integration.cc:294-328)
-        V3 dir, nT;
-        float pdf;
-        if (sample_reflection(job.is_mode, m, rd, h.normal, T, key, ctr, dir, pdf, nT)) {
-          bool alive = true;
-          if (job.rr) {
-            const float qc = gmin(gmax(gmax(nT.x, nT.y), nT.z), 1.0f);
-            if (qc < rng_uniform(key, ctr)) alive = false;
-            else nT = est_div(nT, qc);
-          }
-          // Trace() returns 0 past the depth cutoff (muon/integration.cc:29-33)
-          if (alive && depth + 1 <= job.cutoff && depth + 1 < kMaxBounces) {
-            cont = true;
-            next_dir = dir;
-            T = nT;
-          }
+        if (dmin == __builtin_inff()) {
+          want_mis = false;
+          ++culled_n;
+        } else {
+          mis_tmax = dmin * kWidenHi;
         }
       }
     }
     // a continuing path moves to the next queue with its state; its radiance
-    // follows in retire
-    const uint32_t ni = block_append<kShadeWaves>(cont, &a.c->qcount[cur ^ 1].v, wsum);
-    if (i < n) a.nidx[i] = cont ? ni : 0xffffffffu;
+    // and pixel follow in retire, after the NEE / MIS terms are added
+    uint32_t ni, mi = 0, si = 0;
+    if (NEE) {
+      const BlockAppend3 ap(cont, want_mis, sh.n, &a.c->qcount[cur ^ 1].v, &a.c->mis_count.v, &a.c->shadow_count.v,
+                            sums[pass]);
+      ni = ap.a;
+      mi = ap.b;
+      si = ap.c;
+    } else {
+      ni = block_append<kShadeWaves>(cont, &a.c->qcount[cur ^ 1].v, sums[0]);
+    }
+    if (i < n)
+      a.nidx[i] = (cont ? ni : kPathEnds) | (want_mis ? kPathHasMis : 0u) | (sh.n ? kPathHasShadow : 0u);
     if (cont) {
-      qn[2 * ni] = make_float4(shift.x, shift.y, shift.z, 0.0f);
-      qn[2 * ni + 1] = make_float4(next_dir.x, next_dir.y, next_dir.z, 0.0f);
-      pn.job[ni] = js;
-      pn.pixel[ni] = pixel;
-      pn.ctr[ni] = ctr;
-      pn.key_a[ni] = key.a;
-      pn.key_b[ni] = key.b;
-      pn.depth[ni] = depth + 1;
+      qn[2 * ni] = make_float4(shift.x, shift.y, shift.z, __uint_as_float(jw));
+      qn[2 * ni + 1] = make_float4(next_dir.x, next_dir.y, next_dir.z, __int_as_float(depth + 1));
+      pn.job[ni] = jw;
+      pn.meta[ni] = make_uint4(jw, ctr, key.a, key.b);
       pn.thr[3 * ni] = T.x;
       pn.thr[3 * ni + 1] = T.y;
       pn.thr[3 * ni + 2] = T.z;
     }
+    if (NEE) {
+      if (want_mis) {
+        a.m_ray[3 * mi] = make_float4(shift.x, shift.y, shift.z, __uint_as_float(i));
+        a.m_ray[3 * mi + 1] = make_float4(mis_dir.x, mis_dir.y, mis_dir.z, mis_tmax);
+        a.m_ray[3 * mi + 2] = make_float4(mis_fac.x, mis_fac.y, mis_fac.z, __uint_as_float(jw));
+      }
+      // the shadow rays to trace, compacted
+      for (uint64_t m = sh.mask; m; m &= m - 1)
+        a.s_queue[si++] = ShadowSlot(uint32_t(__ffsll((unsigned long long)m) - 1), a.capacity, i);
+      for (int k = 64; sh.n && k < K; ++k) {
+        const uint32_t sl = ShadowSlot(uint32_t(k), a.capacity, i);
+        if (a.s_valid[sl]) a.s_queue[si++] = sl;
+      }
+    }
+  }
+  // settled MIS rays count as traced secondary rays (the reference traces them)
+  if (NEE) {
+    ray_count(a.c, 1, culled_n);
+    ray_count(a.c, 3, culled_n);
   }
 }
 
@@ -453,7 +363,6 @@ __global__ void __launch_bounds__(kEngBlock) k_eng_shadow(EngArgs a, StackArgs s
   uint2 old[StackOf<KIND>::kPrivate];
   const uint32_t P = a.capacity;
   const uint32_t n = a.c->shadow_count.v;
-  const PathState &ps = a.st[cur];
   uint32_t traced = 0;
   TraceCounters c;
   for (uint32_t base = blockIdx.x * kEngBlock; base < n; base += gridDim.x * kEngBlock) {
@@ -461,8 +370,8 @@ __global__ void __launch_bounds__(kEngBlock) k_eng_shadow(EngArgs a, StackArgs s
     if (j < n) {
       const uint32_t sl = a.s_queue[j];
       const uint32_t i = sl % P;
-      const DevSceneView sv = a.scenes[PathSceneSlot(ps.job[i])];
       const float4 so = a.shift[i], sd = a.s_dir[sl];
+      const DevSceneView sv = a.scenes[PathSceneSlot(__float_as_uint(so.w))];
       const TraceRay r = make_ray(V3{so.x, so.y, so.z}, V3{sd.x, sd.y, sd.z});
       float best = sd.w;
       auto st = make_stack<KIND>(lds, kEngBlock, sa, old);
@@ -476,24 +385,37 @@ __global__ void __launch_bounds__(kEngBlock) k_eng_shadow(EngArgs a, StackArgs s
 }
 
 // ---------------------------------------------------------------- MIS extend
+// The term of MIS ray j for retire: a light hit adds next_T * color * w
+// (muon/integration.cc:490-499), zero otherwise.
+__device__ __forceinline__ void mis_add(const EngArgs &a, const DevSceneView &s, uint32_t j, int32_t hit) {
+  float4 r = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  if (hit >= 0) {
+    const int32_t light = ldg(s.prim_light + hit);
+    if (light >= 0) {
+      const float *L = s.lights + size_t(light) * kLightStride;
+      const float4 f = a.m_ray[3 * j + 2];
+      r = make_float4(f.x * ldg(L + 1), f.y * ldg(L + 2), f.z * ldg(L + 3), 0.0f);
+    }
+  }
+  a.m_add[__float_as_uint(a.m_ray[3 * j].w)] = r;
+}
+
 template <int KIND, bool WW, int WIDTH, bool COUNT>
 __global__ void __launch_bounds__(kEngBlock) k_eng_mis(EngArgs a, StackArgs sa, int cur) {
   __shared__ uint2 lds[StackOf<KIND>::kLds * kEngBlock];
   uint2 old[StackOf<KIND>::kPrivate];
   const uint32_t n = a.c->mis_count.v;
-  const PathState &ps = a.st[cur];
   uint32_t traced = 0;
   TraceCounters c;
   for (uint32_t base = blockIdx.x * kEngBlock; base < n; base += gridDim.x * kEngBlock) {
     const uint32_t j = base + threadIdx.x;
     if (j < n) {
-      const float4 mo = a.m_ray[2 * j], md = a.m_ray[2 * j + 1];
-      const uint32_t i = __float_as_uint(mo.w);
-      const DevSceneView s = a.scenes[PathSceneSlot(ps.job[i])];
+      const float4 mo = a.m_ray[3 * j], md = a.m_ray[3 * j + 1];
+      const DevSceneView s = a.scenes[PathSceneSlot(__float_as_uint(a.m_ray[3 * j + 2].w))];
       const TraceRay r = make_ray(V3{mo.x, mo.y, mo.z}, V3{md.x, md.y, md.z});
       float best = md.w;  // the nearest emitter hit, or +inf
       auto st = make_stack<KIND>(lds, kEngBlock, sa, old);
-      a.m_hit[i] = trace_fast<WIDTH, false, COUNT, WW>(s, r, best, st, c);
+      mis_add(a, s, j, trace_fast<WIDTH, false, COUNT, WW>(s, r, best, st, c));
       ++traced;
     }
   }
@@ -511,7 +433,6 @@ __global__ void __launch_bounds__(kEngBlock) __attribute__((amdgpu_waves_per_eu(
   uint2 old[StackOf<KIND>::kPrivate];
   const uint32_t n = a.c->qcount[cur].v;
   const float4 *q = a.q_ray[cur];
-  const PathState &ps = a.st[cur];
   auto st = make_stack<KIND>(lds, kEngBlock, sa, old);
   LaneTrace<WIDTH, false, COUNT> lt;
   DevSceneView sv;
@@ -526,13 +447,12 @@ __global__ void __launch_bounds__(kEngBlock) __attribute__((amdgpu_waves_per_eu(
       if (!have && !drained) {
         if (k < n) {
           i = k;
-          const uint32_t jw = ps.job[i], js = PathJobSlot(jw);
-          const int depth = ps.depth[i];
-          // the ray and scene view are fetched with the job's cutoff, not
-          // after it: every queued path has both, and starting the lane's
-          // walk only sets registers, so it happens whether or not the
-          // cutoff lets the ray be traced
+          // the scene view is fetched with the job's cutoff, not after it, and
+          // starting the lane's walk only sets registers, so both happen
+          // whether or not the cutoff lets the ray be traced
           const float4 qo = q[2 * i], qd = q[2 * i + 1];
+          const uint32_t jw = __float_as_uint(qo.w), js = PathJobSlot(jw);
+          const int depth = __float_as_int(qd.w);
           sv = a.scenes[PathSceneSlot(jw)];
           lt.start(make_ray(V3{qo.x, qo.y, qo.z}, V3{qd.x, qd.y, qd.z}), __builtin_inff(), st);
           // Integrator::Trace returns 0 past the depth cutoff (muon/integration.cc:29-33)
@@ -565,7 +485,6 @@ __global__ void __launch_bounds__(kEngBlock) __attribute__((amdgpu_waves_per_eu(
   uint2 old[StackOf<KIND>::kPrivate];
   const uint32_t P = a.capacity;
   const uint32_t n = a.c->shadow_count.v;
-  const PathState &ps = a.st[cur];
   auto st = make_stack<KIND>(lds, kEngBlock, sa, old);
   LaneTrace<WIDTH, true, COUNT> lt;
   DevSceneView sv;
@@ -581,8 +500,8 @@ __global__ void __launch_bounds__(kEngBlock) __attribute__((amdgpu_waves_per_eu(
         if (k < n) {
           sl = a.s_queue[k];
           const uint32_t i = sl % P;
-          sv = a.scenes[PathSceneSlot(ps.job[i])];
           const float4 so = a.shift[i], sd = a.s_dir[sl];
+          sv = a.scenes[PathSceneSlot(__float_as_uint(so.w))];
           lt.start(make_ray(V3{so.x, so.y, so.z}, V3{sd.x, sd.y, sd.z}), sd.w, st);
           walking = have = true;
           ++traced;
@@ -607,13 +526,12 @@ __global__ void __launch_bounds__(kEngBlock) __attribute__((amdgpu_waves_per_eu(
   __shared__ uint2 lds[StackOf<KIND>::kLds * kEngBlock];
   uint2 old[StackOf<KIND>::kPrivate];
   const uint32_t n = a.c->mis_count.v;
-  const PathState &ps = a.st[cur];
   auto st = make_stack<KIND>(lds, kEngBlock, sa, old);
   LaneTrace<WIDTH, false, COUNT> lt;
   DevSceneView sv;
   TraceCounters c;
   WaveFetch wf(n);
-  uint32_t i = 0, traced = 0;
+  uint32_t j = 0, traced = 0;
   bool walking = false, have = false, drained = false;
   while (true) {
     const uint64_t needm = __builtin_amdgcn_ballot_w64(!have && !drained);
@@ -621,9 +539,9 @@ __global__ void __launch_bounds__(kEngBlock) __attribute__((amdgpu_waves_per_eu(
       const uint32_t k = wf.claim(needm, &a.c->claim[2][0].v);
       if (!have && !drained) {
         if (k < n) {
-          const float4 mo = a.m_ray[2 * k], md = a.m_ray[2 * k + 1];
-          i = __float_as_uint(mo.w);
-          sv = a.scenes[PathSceneSlot(ps.job[i])];
+          const float4 mo = a.m_ray[3 * k], md = a.m_ray[3 * k + 1];
+          j = k;
+          sv = a.scenes[PathSceneSlot(__float_as_uint(a.m_ray[3 * k + 2].w))];
           lt.start(make_ray(V3{mo.x, mo.y, mo.z}, V3{md.x, md.y, md.z}), md.w, st);
           walking = have = true;
           ++traced;
@@ -635,7 +553,7 @@ __global__ void __launch_bounds__(kEngBlock) __attribute__((amdgpu_waves_per_eu(
     if (__builtin_amdgcn_ballot_w64(have) == 0) break;
     run_walks(sv, lt, walking, st, c, __builtin_amdgcn_ballot_w64(drained) ? 65 : fetch_min);
     if (have && !walking) {
-      a.m_hit[i] = lt.hit;  // retire adds the weighted emission when it is a light
+      mis_add(a, sv, j, lt.hit);
       have = false;
     }
   }
@@ -647,8 +565,10 @@ __global__ void __launch_bounds__(kEngBlock) __attribute__((amdgpu_waves_per_eu(
 constexpr uint32_t kDoneTable = 64;  // per-block done-count entries (a power of two)
 
 // Adds each shaded path's NEE and MIS terms in a fixed order. A continuing
-// path's radiance moves to its place in the next queue; a finished path adds
-// it to the job's film and counts towards the job's done counter.
+// path's radiance and pixel move to its place in the next queue; a finished
+// path adds its radiance to the job's film and counts towards the job's done
+// counter. A path without shadow or MIS rays (its nidx says so) reads only
+// its radiance: 36 B for a continuing one.
 __global__ void __launch_bounds__(kRetireBlock) k_eng_retire(EngArgs a, int cur) {
   const uint32_t n = a.c->qcount[cur].v;
   const PathState &ps = a.st[cur];
@@ -666,43 +586,35 @@ __global__ void __launch_bounds__(kRetireBlock) k_eng_retire(EngArgs a, int cur)
     bool fin = false;
     uint32_t js = 0xffffffffu;
     if (i < n) {
-      const uint32_t jw = ps.job[i];
-      js = PathJobSlot(jw);
-      V3 rad{ps.rad[3 * i], ps.rad[3 * i + 1], ps.rad[3 * i + 2]};
-      if (a.hit_prim[i] >= 0) {
-        const int K = a.jobs[js].K;
+      const uint32_t nw = a.nidx[i], ni = nw & kPathNextMask;
+      float4 rp = ps.rad[i];
+      fin = ni == kPathEnds;
+      if (fin || (nw & kPathHasShadow)) js = PathJobSlot(ps.job[i]);
+      if (nw & (kPathHasShadow | kPathHasMis)) {
         V3 direct{0.0f, 0.0f, 0.0f};
-        for (int k = 0; k < K; ++k) {
-          const size_t sl = k * P + i;
-          if (a.s_vis[sl]) direct = direct + V3{a.s_contrib[3 * sl], a.s_contrib[3 * sl + 1], a.s_contrib[3 * sl + 2]};
-        }
-        // the MIS BRDF ray: a light hit adds next_T * color * w
-        // (muon/integration.cc:490-499), zero otherwise
-        V3 madd{0.0f, 0.0f, 0.0f};
-        const int32_t mh = a.m_hit[i];
-        if (mh >= 0) {
-          const DevSceneView &s = a.scenes[PathSceneSlot(jw)];
-          const int32_t light = ldg(s.prim_light + mh);
-          if (light >= 0) {
-            const float *L = s.lights + size_t(light) * kLightStride;
-            madd = V3{a.m_fac[3 * i] * ldg(L + 1), a.m_fac[3 * i + 1] * ldg(L + 2), a.m_fac[3 * i + 2] * ldg(L + 3)};
+        if (nw & kPathHasShadow) {
+          const int K = a.jobs[js].K;
+          for (int k = 0; k < K; ++k) {
+            const size_t sl = k * P + i;
+            if (a.s_vis[sl]) direct = direct + V3{a.s_contrib[3 * sl], a.s_contrib[3 * sl + 1], a.s_contrib[3 * sl + 2]};
           }
         }
-        direct = direct + madd;
-        rad = rad + direct;
+        if (nw & kPathHasMis) {
+          const float4 madd = a.m_add[i];
+          direct = direct + V3{madd.x, madd.y, madd.z};
+        }
+        rp.x = rp.x + direct.x;
+        rp.y = rp.y + direct.y;
+        rp.z = rp.z + direct.z;
       }
-      const uint32_t ni = a.nidx[i];
-      if (ni != 0xffffffffu) {
-        pn.rad[3 * ni] = rad.x;
-        pn.rad[3 * ni + 1] = rad.y;
-        pn.rad[3 * ni + 2] = rad.z;
+      if (!fin) {
+        pn.rad[ni] = rp;
       } else {
-        unsigned long long *px = a.jobs[js].film + 3 * size_t(ps.pixel[i]);
-        const unsigned long long fx = to_fixed(rad.x), fy = to_fixed(rad.y), fz = to_fixed(rad.z);
+        unsigned long long *px = a.jobs[js].film + 3 * size_t(__float_as_uint(rp.w));
+        const unsigned long long fx = to_fixed(rp.x), fy = to_fixed(rp.y), fz = to_fixed(rp.z);
         if (fx) atomic_add_global(px, fx);
         if (fy) atomic_add_global(px + 1, fy);
         if (fz) atomic_add_global(px + 2, fz);
-        fin = true;
       }
     }
     // done counters: per block, counts gather in a small LDS table keyed by
@@ -788,20 +700,15 @@ __global__ void __launch_bounds__(kEngBlock) k_eng_fill(EngArgs a, int cur) {
     V3 o, d;
     cast_ray(job.cam, x, y, o, d);
     const uint32_t ni = qbase + j;
-    pn.key_a[ni] = key.a;
-    pn.key_b[ni] = key.b;
-    pn.job[ni] = PackPathJob(js, job.scene);
-    pn.pixel[ni] = pixel;
-    pn.ctr[ni] = 0;
-    pn.depth[ni] = 0;
+    const uint32_t jw = PackPathJob(js, job.scene);
+    pn.job[ni] = jw;
+    pn.meta[ni] = make_uint4(jw, 0u, key.a, key.b);
     pn.thr[3 * ni] = 1.0f;
     pn.thr[3 * ni + 1] = 1.0f;
     pn.thr[3 * ni + 2] = 1.0f;
-    pn.rad[3 * ni] = 0.0f;
-    pn.rad[3 * ni + 1] = 0.0f;
-    pn.rad[3 * ni + 2] = 0.0f;
-    qn[2 * ni] = make_float4(o.x, o.y, o.z, 0.0f);
-    qn[2 * ni + 1] = make_float4(d.x, d.y, d.z, 0.0f);
+    pn.rad[ni] = make_float4(0.0f, 0.0f, 0.0f, __uint_as_float(pixel));
+    qn[2 * ni] = make_float4(o.x, o.y, o.z, __uint_as_float(jw));
+    qn[2 * ni + 1] = make_float4(d.x, d.y, d.z, __int_as_float(0));  // depth 0
   }
 }
 
@@ -868,23 +775,17 @@ size_t CarvePaths(uintptr_t base, size_t P, EngArgs &a) {
   Carver c(base, kPathArrays, kNumPathArrays, P);
   for (auto &st : a.st) {
     c(st.job);
-    c(st.pixel);
-    c(st.ctr);
-    c(st.depth);
-    c(st.rad);
+    c(st.meta);
     c(st.thr);
-    c(st.key_a);
-    c(st.key_b);
+    c(st.rad);
   }
   c(a.q_ray[0]);
   c(a.q_ray[1]);
   c(a.m_ray);
   c(a.hit_prim);
   c(a.nidx);
-  c(a.m_fac);
-  c(a.m_hit);
+  c(a.m_add);
   c(a.shift);
-  c(a.hnorm);
   return c.bytes();
 }
 
@@ -921,17 +822,15 @@ struct IterLaunch {
         hipLaunchKernelGGL((k_eng_extend_dyn<KIND, WIDTH, COUNT>), grid, block, 0, st, a, sa, cur, fetch);
       else
         hipLaunchKernelGGL((k_eng_extend<KIND, WW, WIDTH, COUNT>), grid, block, 0, st, a, sa, cur);
-      hipLaunchKernelGGL(k_eng_shade_plain, sgrid, sblock, 0, st, a, cur);
+      hipLaunchKernelGGL(k_eng_shade<false>, sgrid, sblock, 0, st, a, cur);
     } else if (fetch > 0) {
       hipLaunchKernelGGL((k_eng_extend_dyn<KIND, WIDTH, COUNT>), grid, block, 0, st, a, sa, cur, fetch);
-      hipLaunchKernelGGL(k_eng_shade_light, sgrid, sblock, 0, st, a, cur);
-      hipLaunchKernelGGL(k_eng_shade_bsdf, sgrid, sblock, 0, st, a, cur);
+      hipLaunchKernelGGL(k_eng_shade<true>, sgrid, sblock, 0, st, a, cur);
       hipLaunchKernelGGL((k_eng_shadow_dyn<KIND, WIDTH, COUNT>), grid, block, 0, st, a, sa, cur, fetch);
       hipLaunchKernelGGL((k_eng_mis_dyn<KIND, WIDTH, COUNT>), grid, block, 0, st, a, sa, cur, fetch);
     } else {
       hipLaunchKernelGGL((k_eng_extend<KIND, WW, WIDTH, COUNT>), grid, block, 0, st, a, sa, cur);
-      hipLaunchKernelGGL(k_eng_shade_light, sgrid, sblock, 0, st, a, cur);
-      hipLaunchKernelGGL(k_eng_shade_bsdf, sgrid, sblock, 0, st, a, cur);
+      hipLaunchKernelGGL(k_eng_shade<true>, sgrid, sblock, 0, st, a, cur);
       hipLaunchKernelGGL((k_eng_shadow<KIND, WW, WIDTH, COUNT>), grid, block, 0, st, a, sa, cur);
       hipLaunchKernelGGL((k_eng_mis<KIND, WW, WIDTH, COUNT>), grid, block, 0, st, a, sa, cur);
     }

@@ -72,17 +72,17 @@ constexpr size_t CarveSize(size_t count, size_t elem_bytes) {
   return (count * elem_bytes + kCarveAlign - 1) & ~(kCarveAlign - 1);
 }
 
-// Path buffer: two path states (job, pixel, RNG counter, depth, radiance x3,
-// throughput x3, the two words of the sample's random-stream key), the two
-// ray queues and the MIS rays (two float4 per path each), the hit primitive,
-// the next-queue index, the MIS factor x3, the MIS hit, the shadow / MIS
-// origin and the hit normal (one float4 each).
+// Path buffer: two path states (job word; job word, RNG counter and the two
+// words of the sample's random-stream key; throughput x3; radiance x3 and
+// pixel), the two ray queues (two float4 per path, with the job word and the
+// depth) and the MIS rays (three float4), the hit primitive, the next-queue
+// index, the MIS term and the shadow origin (one float4 each).
 constexpr ArraySpec kPathArrays[] = {
-    {4, 1}, {4, 1}, {4, 1}, {4, 1}, {4, 3}, {4, 3}, {4, 1}, {4, 1},  // state 0
-    {4, 1}, {4, 1}, {4, 1}, {4, 1}, {4, 3}, {4, 3}, {4, 1}, {4, 1},  // state 1
-    {16, 2}, {16, 2}, {16, 2},                                // ray queues 0, 1; MIS rays
-    {4, 1}, {4, 1}, {4, 3}, {4, 1},                           // hit prim, next index, MIS factor, MIS hit
-    {16, 1}, {16, 1}};                                        // shadow origin + material, hit normal
+    {4, 1}, {16, 1}, {4, 3}, {16, 1},  // state 0
+    {4, 1}, {16, 1}, {4, 3}, {16, 1},  // state 1
+    {16, 2}, {16, 2}, {16, 3},         // ray queues 0, 1; MIS rays
+    {4, 1}, {4, 1},                    // hit prim, next index
+    {16, 1}, {16, 1}};                 // MIS term, shadow origin + job word
 constexpr int kNumPathArrays = int(sizeof(kPathArrays) / sizeof(kPathArrays[0]));
 // Shadow buffer, per shadow ray: direction + tmax (float4), contribution
 // x3, visible and valid flags, the trace-queue entry.

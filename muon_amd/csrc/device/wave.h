@@ -90,6 +90,51 @@ __device__ __forceinline__ uint32_t block_append(bool want, uint32_t *counter, u
   return base + uint32_t(__popcll(m & ((1ull << lane) - 1ull)));
 }
 
+// Three appends of a block at once, one entry per lane for `want_a` and
+// `want_b` and `cnt` for the third queue: three threads take the block's
+// places together, so a block waits for one round of atomics instead of
+// three. `sh` is used by this call only: callers in a loop alternate between
+// two, so that the next call does not overwrite what a slower wavefront
+// still reads (the call after it comes behind that wavefront's next barrier).
+struct BlockAppend3 {
+  static constexpr int kWaves = 8, kWords = 3 * (kWaves + 1);
+  uint32_t a, b, c;
+  __device__ __forceinline__ BlockAppend3(bool want_a, bool want_b, uint32_t cnt, uint32_t *ca, uint32_t *cb,
+                                          uint32_t *cc, uint32_t *sh) {
+    const int lane = int(__lane_id());
+    const int w = int(threadIdx.x) >> 6;
+    const uint64_t ma = __ballot(want_a), mb = __ballot(want_b), below = (1ull << lane) - 1ull;
+    uint32_t incl = cnt;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const uint32_t v = uint32_t(__shfl_up(int(incl), off));
+      if (lane >= off) incl += v;
+    }
+    if (lane == 63) {
+      sh[w] = uint32_t(__popcll(ma));
+      sh[kWaves + w] = uint32_t(__popcll(mb));
+      sh[2 * kWaves + w] = incl;
+    }
+    __syncthreads();
+    if (threadIdx.x < 3) {
+      uint32_t tot = 0;
+#pragma unroll
+      for (int k = 0; k < kWaves; ++k) tot += sh[threadIdx.x * kWaves + k];
+      uint32_t *ctr = threadIdx.x == 0 ? ca : threadIdx.x == 1 ? cb : cc;
+      sh[3 * kWaves + threadIdx.x] = tot ? atomicAdd(ctr, tot) : 0u;
+    }
+    __syncthreads();
+    a = sh[3 * kWaves] + uint32_t(__popcll(ma & below));
+    b = sh[3 * kWaves + 1] + uint32_t(__popcll(mb & below));
+    c = sh[3 * kWaves + 2] + incl - cnt;
+    for (int k = 0; k < w; ++k) {
+      a += sh[k];
+      b += sh[kWaves + k];
+      c += sh[2 * kWaves + k];
+    }
+  }
+};
+
 __device__ __forceinline__ void wave_count(uint32_t n, unsigned long long *ctr) {
   unsigned long long a = n;
   for (int off = 32; off > 0; off >>= 1) a += __shfl_down(a, off);

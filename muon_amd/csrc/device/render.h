@@ -22,7 +22,8 @@ constexpr int kCtrBoundsTests = 5;
 constexpr int kCtrBoundsHits = 6;
 constexpr int kNumCounters = 8;
 // Device counters of one muonx_render: the claim counters of the image kernels
-// (claim_plan.h), then the trace counters.
+// (claim_plan.h; none under capture), then the trace counters. Captured renders
+// have trace counters of their own, which nobody reads.
 struct RenderCounters {
   unsigned long long *trace;
   uint32_t *claims;

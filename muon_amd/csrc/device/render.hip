@@ -126,7 +126,7 @@ __global__ void __launch_bounds__(kSimpleBlock) __attribute__((amdgpu_waves_per_
   PrivateStack<CAP> st(lds + threadIdx.x, kSimpleBlock, old);
   ExactWalk<true, kWalkClosest> w;
   TraceCounters cnt;
-  WaveFetch wf(items, kChunk);
+  WaveFetch wf(items, kChunk, next != nullptr);
   uint32_t traced = 0;
   ImageItem i;
   bool walking = false, have = false, drained = false;
@@ -225,7 +225,7 @@ __global__ void __launch_bounds__(kSimpleBlock) __attribute__((amdgpu_waves_per_
   PrivateStack<CAP> st(lds + threadIdx.x, kSimpleBlock, old);
   ExactWalk<true, kWalkEither> w;
   TraceCounters cnt;
-  WaveFetch wf(items, kChunk);
+  WaveFetch wf(items, kChunk, next != nullptr);
   uint32_t n_primary = 0, n_secondary = 0, n_shadow = 0;
   ImageItem i;
   int nb = 0;  // bounces with a hit (the depth of the next)
@@ -377,7 +377,8 @@ constexpr uint32_t kSimpleBlocksPerCu = 12, kWhittedBlocksPerCu = 8;
 constexpr uint64_t kSampleBytes = uint64_t(64) << 20;
 
 // Runs one of the deterministic integrators; `counters` holds the trace
-// counters and the (cleared) claim counters.
+// counters and the (cleared) claim counters. Without claim counters the launches
+// use no other buffer of the context either: one sample each, added directly.
 int RenderDeterministic(muonx_scene *scene, const muonx_render_params &p, float *accum, const RenderCounters &counters,
                         DevBuf &samples, hipStream_t stream) {
   const DevSceneView &s = scene->view;
@@ -390,7 +391,8 @@ int RenderDeterministic(muonx_scene *scene, const muonx_render_params &p, float 
   const uint32_t cus = uint32_t(scene->ctx->num_cus > 0 ? scene->ctx->num_cus : 256);
   // samples per launch: their buffer stays within kSampleBytes
   const uint64_t film = uint64_t(p.width) * uint64_t(p.height) * 3 * sizeof(float);
-  const int batch = int(std::max<uint64_t>(1, std::min<uint64_t>(uint64_t(p.spp), kSampleBytes / film)));
+  const int batch =
+      counters.claims ? int(std::max<uint64_t>(1, std::min<uint64_t>(uint64_t(p.spp), kSampleBytes / film))) : 1;
   if (batch > 1) MX_HIP(samples.Reserve(film * uint64_t(batch)));
   ImageItems it{uint32_t(p.width), uint32_t(p.height), (uint32_t(p.width) + 7u) >> 3, 0, 0, 0, samples.as<float>()};
   unsigned long long *ctr = counters.trace;
@@ -405,7 +407,7 @@ int RenderDeterministic(muonx_scene *scene, const muonx_render_params &p, float 
     for (it.tile0 = 0; it.tile0 < tiles; it.tile0 += part) {
       const uint32_t items = uint32_t(std::min(tiles - it.tile0, part)) * uint32_t(it.count) * 64u;
       const uint32_t blocks = ClaimBlocks(items, cus * (whitted ? kWhittedBlocksPerCu : kSimpleBlocksPerCu), kSimpleBlock / 64);
-      if (NeedsClaims(items, blocks * (kSimpleBlock / 64))) {
+      if (next && NeedsClaims(items, blocks * (kSimpleBlock / 64))) {
         if (!cleared) MX_HIP(hipMemsetAsync(next, 0, kClaimBytes, stream));
         cleared = false;
       }
@@ -464,16 +466,19 @@ extern "C" int muonx_render(muonx_scene *scene, const muonx_render_params *param
   std::lock_guard<std::mutex> lock(ctx->mu);
   MX_HIP(hipSetDevice(ctx->device));
   hipStream_t stream = static_cast<hipStream_t>(stream_);
+  bool capturing = false;
+  int rc = IsCapturing(stream, &capturing);
+  if (rc != MUONX_OK) return rc;
   RenderWorkspace *ws = GetWorkspace(ctx);
-  MX_HIP(ws->counters.Reserve(kRenderCounterBytes));
-  MX_HIP(hipMemsetAsync(ws->counters.ptr, 0, kRenderCounterBytes, stream));
+  MX_HIP(ws->counters.Reserve(kRenderCounterBytes + kTraceCounterBytes));
+  if (!capturing) MX_HIP(hipMemsetAsync(ws->counters.ptr, 0, kRenderCounterBytes, stream));
   hipEvent_t e0, e1;
   MX_HIP(hipEventCreate(&e0));
   MX_HIP(hipEventCreate(&e1));
   MX_HIP(hipEventRecord(e0, stream));
-  int rc;
-  const RenderCounters ctr{ws->counters.as<unsigned long long>() + kClaimBytes / sizeof(unsigned long long),
-                           ws->counters.as<uint32_t>()};
+  const size_t trace_at = capturing ? kRenderCounterBytes : kClaimBytes;
+  const RenderCounters ctr{ws->counters.as<unsigned long long>() + trace_at / sizeof(unsigned long long),
+                           capturing ? nullptr : ws->counters.as<uint32_t>()};
   bool host_rays = false;
   unsigned long long rays[kEngineCounters] = {};
   switch (p.integrator) {

@@ -56,6 +56,16 @@ struct DevBuf {
   }
 };
 
+// Whether work issued to `stream` goes into a graph (the null stream's cannot).
+// A graph is replayed at any time and on any stream: its kernels use no buffer
+// that the context shares between calls or may move.
+inline int IsCapturing(hipStream_t stream, bool *yes) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (stream) MX_HIP(hipStreamIsCapturing(stream, &st));
+  *yes = st != hipStreamCaptureStatusNone;
+  return MUONX_OK;
+}
+
 struct RenderWorkspace;
 
 // Scenes get ids that are never reused, so caches keyed by id cannot mistake

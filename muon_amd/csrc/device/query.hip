@@ -65,7 +65,7 @@ __global__ void __launch_bounds__(kQueryBlock) __attribute__((amdgpu_waves_per_e
   auto st = make_stack<KIND>(lds, kQueryBlock, sa, old);
   LaneTrace<WIDTH, ANY, COUNT> lt;
   uint32_t idx = 0;
-  WaveFetch wf(n, kChunk);
+  WaveFetch wf(n, kChunk, next != nullptr);
   bool walking = false, have = false, drained = false;
   while (true) {
     const uint64_t needm = __builtin_amdgcn_ballot_w64(!have && !drained);
@@ -121,7 +121,7 @@ __global__ void __launch_bounds__(kQueryBlock)
   PrivateStack<CAP> st(lds + threadIdx.x, kQueryBlock, old);
   ExactWalk<COUNT, ANY ? kWalkAny : kWalkClosest> w;
   TraceCounters cnt;
-  WaveFetch wf(n, kChunk);
+  WaveFetch wf(n, kChunk, next != nullptr);
   uint32_t idx = 0;
   bool walking = false, have = false, drained = false;
   while (true) {
@@ -241,7 +241,16 @@ int InitStaticScratch(int device) {
 // The claim counters of the per-lane fetch kernels, cleared on `stream`: in
 // the static scratch with `noalloc` (by a kernel rather than a memset node),
 // else in the context, ordered after its previous user like the spill region.
+// None under capture: on replays after the first the recorded memset has left
+// the counters as they were, and no replay waits for the context's other calls.
 static int ClearClaims(muonx_ctx *ctx, hipStream_t stream, bool noalloc, void *scratch_base, uint32_t **next) {
+  bool capturing = false;
+  if (!noalloc) {
+    const int rc = IsCapturing(stream, &capturing);
+    if (rc != MUONX_OK) return rc;
+  }
+  *next = nullptr;
+  if (capturing) return MUONX_OK;
   if (noalloc) {
     *next = static_cast<uint32_t *>(scratch_base);
     hipLaunchKernelGGL(k_clear_claims, dim3(1), dim3(kClaimGroups), 0, stream, *next);
@@ -273,8 +282,7 @@ static int LaunchExactQuery(muonx_ctx *ctx, const DevSceneView &s, bool any, con
     const uint64_t cus = uint64_t(ctx->num_cus > 0 ? ctx->num_cus : 256);
     const uint32_t grid = ClaimBlocks(m, uint32_t(cus) * kExactBlocksPerCu, kWavesPerBlock);
     uint32_t *next = nullptr;
-    const bool claims = NeedsClaims(m, grid * kWavesPerBlock);
-    if (claims) {
+    if (NeedsClaims(m, grid * kWavesPerBlock)) {
       const int rc = ClearClaims(ctx, stream, noalloc, scratch_base, &next);
       if (rc != MUONX_OK) return rc;
     }
@@ -299,7 +307,7 @@ static int LaunchExactQuery(muonx_ctx *ctx, const DevSceneView &s, bool any, con
 #undef MX_QXC
 #undef MX_QX
     MX_HIP(hipGetLastError());
-    if (claims && !noalloc) MX_HIP(hipEventRecord(ctx->spill_done, stream));
+    if (next && !noalloc) MX_HIP(hipEventRecord(ctx->spill_done, stream));
   }
   return MUONX_OK;
 }
@@ -350,8 +358,9 @@ int LaunchQuery(muonx_ctx *ctx, const DevSceneView &s, bool any, bool exact, con
   if (fetch > 0 && n <= (1u << 31)) {  // claimed indices stay below 2^32
     // per-lane ray fetch
     uint32_t *next = nullptr;
-    const bool claims = NeedsClaims(n, uint32_t(cfg.grid) * kWavesPerBlock);
-    if (claims && (rc = ClearClaims(ctx, stream, noalloc, sbase, &next)) != MUONX_OK) return rc;
+    if (NeedsClaims(n, uint32_t(cfg.grid) * kWavesPerBlock) &&
+        (rc = ClearClaims(ctx, stream, noalloc, sbase, &next)) != MUONX_OK)
+      return rc;
 #define MX_QD(A, C) DispatchTraverse(cfg, QueryDynLaunch<A, C>{cfg, s, ro, rd, tmax, n, prim, t, occ, counters, next, fetch, stream})
     if (any) {
       if (cnt) MX_QD(true, true);
@@ -362,7 +371,7 @@ int LaunchQuery(muonx_ctx *ctx, const DevSceneView &s, bool any, bool exact, con
     }
 #undef MX_QD
     MX_HIP(hipGetLastError());
-    if (!noalloc && (claims || cfg.spill)) MX_HIP(hipEventRecord(ctx->spill_done, stream));
+    if (!noalloc && (next || cfg.spill)) MX_HIP(hipEventRecord(ctx->spill_done, stream));
     return MUONX_OK;
   }
   if (any) {

@@ -80,6 +80,10 @@ struct RenderWorkspace {
   DevBuf counters;
   DevBuf film;     // staging film of muonx_render_host
   DevBuf samples;  // a launch's samples of the deterministic integrators
+  // Renders without stats return before their work on `counters` and `samples`
+  // is done: while scratch_busy, scratch_done marks the end of the last one's.
+  hipEvent_t scratch_done = nullptr;
+  bool scratch_busy = false;
   // path-tracer engine of muonx_render / muonx_render_batch
   Scheduler *sched = nullptr;
   muonx_tuning sched_tuning{};

@@ -20,6 +20,8 @@ namespace muonx {
 void DestroyWorkspace(RenderWorkspace *ws) {
   if (!ws) return;  // the context never rendered
   DestroyContextScheduler(ws);
+  if (ws->scratch_busy) (void)hipEventSynchronize(ws->scratch_done);
+  if (ws->scratch_done) (void)hipEventDestroy(ws->scratch_done);
   if (ws->ev_in) (void)hipEventDestroy(ws->ev_in);
   if (ws->ev_out) (void)hipEventDestroy(ws->ev_out);
   delete ws;
@@ -376,11 +378,45 @@ constexpr uint32_t kSimpleBlocksPerCu = 12, kWhittedBlocksPerCu = 8;
 // The most memory for a launch's samples.
 constexpr uint64_t kSampleBytes = uint64_t(64) << 20;
 
+// A render's turn at the workspace's counters and samples, which all renders of
+// the context share, on whatever streams they are: its stream waits for the last
+// user, and the next user's for it. Held under the context's lock.
+class ScratchTurn {
+ public:
+  ScratchTurn(RenderWorkspace *ws, hipStream_t stream) : ws_(ws), stream_(stream) {}
+  ~ScratchTurn() {
+    if (!begun_) return;
+    // a render that gave up half-way is ordered like any other
+    if ((ws_->scratch_done || hipEventCreateWithFlags(&ws_->scratch_done, hipEventDisableTiming) == hipSuccess) &&
+        hipEventRecord(ws_->scratch_done, stream_) == hipSuccess) {
+      ws_->scratch_busy = true;
+    } else {
+      (void)hipStreamSynchronize(stream_);
+      ws_->scratch_busy = false;
+    }
+  }
+  int Begin() {
+    if (ws_->scratch_busy) MX_HIP(hipStreamWaitEvent(stream_, ws_->scratch_done, 0));
+    begun_ = true;
+    return MUONX_OK;
+  }
+  // The host has waited for the stream, and so for every user up to this one.
+  void Finished() {
+    ws_->scratch_busy = false;
+    begun_ = false;
+  }
+
+ private:
+  RenderWorkspace *ws_;
+  hipStream_t stream_;
+  bool begun_ = false;
+};
+
 // Runs one of the deterministic integrators; `counters` holds the trace
 // counters and the (cleared) claim counters. Without claim counters the launches
 // use no other buffer of the context either: one sample each, added directly.
 int RenderDeterministic(muonx_scene *scene, const muonx_render_params &p, float *accum, const RenderCounters &counters,
-                        DevBuf &samples, hipStream_t stream) {
+                        RenderWorkspace *ws, hipStream_t stream) {
   const DevSceneView &s = scene->view;
   if (s.bvh_depth > 96) {
     SetError("BVH too deep for the traversal stack");
@@ -393,8 +429,13 @@ int RenderDeterministic(muonx_scene *scene, const muonx_render_params &p, float 
   const uint64_t film = uint64_t(p.width) * uint64_t(p.height) * 3 * sizeof(float);
   const int batch =
       counters.claims ? int(std::max<uint64_t>(1, std::min<uint64_t>(uint64_t(p.spp), kSampleBytes / film))) : 1;
-  if (batch > 1) MX_HIP(samples.Reserve(film * uint64_t(batch)));
-  ImageItems it{uint32_t(p.width), uint32_t(p.height), (uint32_t(p.width) + 7u) >> 3, 0, 0, 0, samples.as<float>()};
+  if (batch > 1) {
+    const size_t bytes = film * uint64_t(batch);
+    if (bytes > ws->samples.bytes && ws->scratch_busy) MX_HIP(hipEventSynchronize(ws->scratch_done));  // it moves
+    MX_HIP(ws->samples.Reserve(bytes));
+  }
+  ImageItems it{uint32_t(p.width), uint32_t(p.height), (uint32_t(p.width) + 7u) >> 3, 0, 0, 0,
+                ws->samples.as<float>()};
   unsigned long long *ctr = counters.trace;
   uint32_t *next = counters.claims;
   // muon/integration.cc:29-33
@@ -470,8 +511,12 @@ extern "C" int muonx_render(muonx_scene *scene, const muonx_render_params *param
   int rc = IsCapturing(stream, &capturing);
   if (rc != MUONX_OK) return rc;
   RenderWorkspace *ws = GetWorkspace(ctx);
-  MX_HIP(ws->counters.Reserve(kRenderCounterBytes + kTraceCounterBytes));
-  if (!capturing) MX_HIP(hipMemsetAsync(ws->counters.ptr, 0, kRenderCounterBytes, stream));
+  MX_HIP(ws->counters.Reserve(kRenderCounterBytes + kTraceCounterBytes));  // allocated once, never moved
+  ScratchTurn turn(ws, stream);
+  if (p.integrator != MUONX_INTEGRATOR_PATHTRACER && !capturing) {
+    if ((rc = turn.Begin()) != MUONX_OK) return rc;
+    MX_HIP(hipMemsetAsync(ws->counters.ptr, 0, kRenderCounterBytes, stream));
+  }
   hipEvent_t e0, e1;
   MX_HIP(hipEventCreate(&e0));
   MX_HIP(hipEventCreate(&e1));
@@ -487,7 +532,7 @@ extern "C" int muonx_render(muonx_scene *scene, const muonx_render_params *param
     case MUONX_INTEGRATOR_DEPTH:
     case MUONX_INTEGRATOR_RAYTRACER:
     case MUONX_INTEGRATOR_ANALYTICDIRECT:
-      rc = RenderDeterministic(scene, p, accum, ctr, ws->samples, stream);
+      rc = RenderDeterministic(scene, p, accum, ctr, ws, stream);
       break;
     case MUONX_INTEGRATOR_PATHTRACER:
       rc = RenderPathTracer(scene, p, accum, stream, rays);
@@ -513,6 +558,7 @@ extern "C" int muonx_render(muonx_scene *scene, const muonx_render_params *param
         for (int c = 0; c < kNumCounters; ++c) h[c] += slots[size_t(k) * kCounterSlotStride + size_t(c)];
     }
     MX_HIP(hipStreamSynchronize(stream));
+    if (!host_rays) turn.Finished();
     float ms = 0.0f;
     MX_HIP(hipEventElapsedTime(&ms, e0, e1));
     stats->primary_rays = host_rays ? rays[0] : h[kCtrPrimary];

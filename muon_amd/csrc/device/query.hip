@@ -109,16 +109,31 @@ __global__ void __launch_bounds__(kQueryBlock) __attribute__((amdgpu_waves_per_e
 // incoherent rays on the level-6 icosphere 361 -> 259 us, 10^6 on 10,000
 // spheres 1154 -> 391 us together with the reciprocal quotients. Refilling
 // at 16, 32 or 48 idle lanes measured the same.
+// Without PRIVATE the whole stack is in LDS (three wavefronts per SIMD at most):
+// for calls that may not take private memory from the runtime.
 constexpr int kExactRefill = 32;
-template <int CAP, bool ANY, bool COUNT>
+template <int CAP, bool PRIVATE>
+struct ExactStack {
+  using T = PrivateStack<CAP>;
+  static constexpr int kLds = kPrivateRing, kOld = T::kOld;
+  static __device__ __forceinline__ T make(uint2 *lds, uint2 *old) { return T(lds + threadIdx.x, kQueryBlock, old); }
+};
+template <int CAP>
+struct ExactStack<CAP, false> {
+  using T = LdsStack<CAP>;
+  static constexpr int kLds = CAP, kOld = 1;
+  static __device__ __forceinline__ T make(uint2 *lds, uint2 *) { return T(lds + threadIdx.x, kQueryBlock); }
+};
+template <int CAP, bool PRIVATE, bool ANY, bool COUNT>
 __global__ void __launch_bounds__(kQueryBlock)
     k_query_exact(DevSceneView s, const float *__restrict__ ro, const float *__restrict__ rd,
                   const float *__restrict__ tmax, uint32_t n, int32_t *__restrict__ prim_out,
                   float *__restrict__ t_out, uint8_t *__restrict__ occ_out, unsigned long long *__restrict__ counters,
                   uint32_t *next) {
-  __shared__ uint2 lds[kPrivateRing * kQueryBlock];
-  uint2 old[PrivateStack<CAP>::kOld];
-  PrivateStack<CAP> st(lds + threadIdx.x, kQueryBlock, old);
+  using Stack = ExactStack<CAP, PRIVATE>;
+  __shared__ uint2 lds[Stack::kLds * kQueryBlock];
+  uint2 old[Stack::kOld];
+  auto st = Stack::make(lds, old);
   ExactWalk<COUNT, ANY ? kWalkAny : kWalkClosest> w;
   TraceCounters cnt;
   WaveFetch wf(n, kChunk, next != nullptr);
@@ -264,11 +279,12 @@ static int ClearClaims(muonx_ctx *ctx, hipStream_t stream, bool noalloc, void *s
   return MUONX_OK;
 }
 
-// Exact mode: stacks in LDS and private memory, so the claim counters are
-// the only scratch, and a batch without claims needs none. 6, 8, 12 or 16
-// blocks per CU: 308 / 301 / 260 / 260 us for 300,007 rays on the level-6
-// icosphere.
+// Exact mode: stacks in LDS and private memory (`noalloc`: in LDS alone), so the
+// claim counters are the only scratch, and a batch without claims needs none.
+// 6, 8, 12 or 16 blocks per CU: 308 / 301 / 260 / 260 us for 300,007 rays on the
+// level-6 icosphere; with whole stacks in LDS, as many as its LDS holds.
 constexpr int kExactBlocksPerCu = 12;
+constexpr int kLdsBytes = 160 << 10;  // of a CU
 constexpr uint32_t kExactPart = 1u << 30;  // rays per launch: 3 * index stays below 2^32
 static int LaunchExactQuery(muonx_ctx *ctx, const DevSceneView &s, bool any, const float *ro, const float *rd,
                             const float *tmax, uint32_t n, int32_t *prim, float *t, uint8_t *occ,
@@ -277,10 +293,13 @@ static int LaunchExactQuery(muonx_ctx *ctx, const DevSceneView &s, bool any, con
     SetError("BVH depth " + std::to_string(s.bvh_depth) + " exceeds the exact-mode traversal stack (96)");
     return MUONX_ERR_CAPACITY;
   }
+  const int cap = s.bvh_depth <= 24 ? 24 : s.bvh_depth <= 48 ? 48 : 96;
+  const int per_cu = noalloc ? std::min(kExactBlocksPerCu, kLdsBytes / (cap * kQueryBlock * int(sizeof(uint2))))
+                             : kExactBlocksPerCu;
   for (uint32_t at = 0; at < n; at += std::min(n - at, kExactPart)) {
     const uint32_t m = std::min(n - at, kExactPart);
     const uint64_t cus = uint64_t(ctx->num_cus > 0 ? ctx->num_cus : 256);
-    const uint32_t grid = ClaimBlocks(m, uint32_t(cus) * kExactBlocksPerCu, kWavesPerBlock);
+    const uint32_t grid = ClaimBlocks(m, uint32_t(cus) * uint32_t(per_cu), kWavesPerBlock);
     uint32_t *next = nullptr;
     if (NeedsClaims(m, grid * kWavesPerBlock)) {
       const int rc = ClearClaims(ctx, stream, noalloc, scratch_base, &next);
@@ -290,13 +309,16 @@ static int LaunchExactQuery(muonx_ctx *ctx, const DevSceneView &s, bool any, con
     int32_t *po = prim ? prim + at : nullptr;
     float *to = t ? t + at : nullptr;
     uint8_t *oo = occ ? occ + at : nullptr;
-#define MX_QX(CAP, A, C) \
-  hipLaunchKernelGGL((k_query_exact<CAP, A, C>), dim3(grid), dim3(kQueryBlock), 0, stream, s, o, d, tm, m, po, to, oo, \
-                     counters, next)
+#define MX_QX(CAP, P, A, C) \
+  hipLaunchKernelGGL((k_query_exact<CAP, P, A, C>), dim3(grid), dim3(kQueryBlock), 0, stream, s, o, d, tm, m, po, to, \
+                     oo, counters, next)
+#define MX_QXP(CAP, A, C) \
+  if (noalloc) MX_QX(CAP, false, A, C); \
+  else MX_QX(CAP, true, A, C)
 #define MX_QXC(A, C) \
-  if (s.bvh_depth <= 24) MX_QX(24, A, C); \
-  else if (s.bvh_depth <= 48) MX_QX(48, A, C); \
-  else MX_QX(96, A, C)
+  if (cap == 24) { MX_QXP(24, A, C); } \
+  else if (cap == 48) { MX_QXP(48, A, C); } \
+  else { MX_QXP(96, A, C); }
     if (any) {
       MX_QXC(true, false);
     } else if (counters) {
@@ -305,6 +327,7 @@ static int LaunchExactQuery(muonx_ctx *ctx, const DevSceneView &s, bool any, con
       MX_QXC(false, false);
     }
 #undef MX_QXC
+#undef MX_QXP
 #undef MX_QX
     MX_HIP(hipGetLastError());
     if (next && !noalloc) MX_HIP(hipEventRecord(ctx->spill_done, stream));
@@ -313,9 +336,9 @@ static int LaunchExactQuery(muonx_ctx *ctx, const DevSceneView &s, bool any, con
 }
 
 // Launches the query kernels. With `noalloc` the spill region and the claim
-// counter come from the static scratch (the grid is capped so that the spill
-// fits), the counter is cleared by a kernel rather than a memset node, and
-// no event or buffer is created.
+// counters come from the static scratch (the grid is capped so that the spill
+// fits), the counters are cleared by a kernel rather than a memset node, no
+// stack is in private memory, and no event or buffer is created.
 int LaunchQuery(muonx_ctx *ctx, const DevSceneView &s, bool any, bool exact, const float *ro, const float *rd,
                 const float *tmax, uint32_t n, int32_t *prim, float *t, uint8_t *occ, unsigned long long *counters,
                 hipStream_t stream, bool noalloc) {
@@ -332,7 +355,7 @@ int LaunchQuery(muonx_ctx *ctx, const DevSceneView &s, bool any, bool exact, con
   }
   if (exact) return LaunchExactQuery(ctx, s, any, ro, rd, tmax, n, prim, t, occ, counters, stream, noalloc, sbase);
   if (noalloc) {
-    rc = PlanTraverseShape(ctx->tuning, ctx->num_cus, s.bvh_depth, s.wstack, n, kQueryBlock, cfg);
+    rc = PlanTraverseShape(ctx->tuning, ctx->num_cus, s.bvh_depth, s.wstack, n, kQueryBlock, cfg, false);
     if (rc != MUONX_OK) return rc;
     if (cfg.gcap > 0) {
       const size_t per_block = size_t(kQueryBlock) * size_t(cfg.gcap) * sizeof(uint2);

@@ -65,9 +65,11 @@ __device__ __forceinline__ typename StackOf<KIND>::T make_stack(uint2 *lds, int 
 // Resolves the variant for a scene (binary depth, wide-stack bound): node
 // format, grid, stack kind and the spill entries per thread (cfg.gcap; the
 // spill region then needs cfg.threads * cfg.gcap uint2, not yet assigned).
-// Allocates nothing.
+// Without `private_stacks` no kind is chosen whose stack lives in private
+// memory, which the runtime provides for every resident wavefront of the card
+// at a kernel's first dispatch (264 MiB for kind 8). Allocates nothing.
 inline int PlanTraverseShape(const muonx_tuning &t, int num_cus, uint32_t bvh_depth, uint32_t wstack,
-                             uint64_t work_items, int block, TraverseCfg &cfg) {
+                             uint64_t work_items, int block, TraverseCfg &cfg, bool private_stacks = true) {
   const int cus = num_cus > 0 ? num_cus : 256;
   cfg.width = t.bvh_width != 4 ? kNodesBinary : (t.node_bits == 8 ? kNodesWideQ : kNodesWide);
   const int bpc = std::max(1, t.blocks_per_cu);
@@ -79,7 +81,7 @@ inline int PlanTraverseShape(const muonx_tuning &t, int num_cus, uint32_t bvh_de
   // binary: entries never exceed depth - 1; wide: the collapse's bound
   const int need = int(cfg.width != kNodesBinary ? std::max<uint32_t>(wstack, 1) : bvh_depth);
   const bool ring = t.stack_entries == 8 || t.stack_entries == 16;
-  if (ring && need <= (t.stack_entries == 8 ? kPrivateCap : 8)) {
+  if (ring && private_stacks && need <= (t.stack_entries == 8 ? kPrivateCap : 8)) {
     cfg.kind = 8;
     return MUONX_OK;
   }

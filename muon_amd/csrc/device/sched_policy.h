@@ -145,6 +145,33 @@ inline void RecordPick(std::vector<SliceCandidate> &running, SliceChoice choice,
   if (choice == SliceChoice::kRunning) running[index].passes = 0;
 }
 
+// How many engine iterations to launch before the next look at the done
+// counters. `bound`: how many end the longest of the open paths, 0 when that is not
+// known; `launched`: those launched since. `last`: the paths are all done then, and
+// the iterations are waited for at once; other looks come one group late, while the
+// next group runs.
+//
+// An iteration of empty kernels costs 20-30 us on the GPU, a look 10 to 20. A
+// closed scene needs every iteration up to the bound, an open one whose paths leave
+// early does not, so up to kLaunchAhead go out without a look, up to kKnownAhead in
+// groups of 8 and 4, and beyond in the groups of unbounded paths. Three spheres
+// without walls, every iteration up to the bound / groups of 2 / as here: 64x64, 4
+// spp, bound 14 420-433 / 329-388 / 384-451 us, 16 (NEE) 625-662 / 484-565 / 514;
+// 256x256, 16 spp, bound 14 534-554 / 531-598 / 548-554, 16 572-591 / 583-589 / 602.
+// Bound 11 in one go or in groups of 2: 374-386 and 380-433, 473-503 and 512-536.
+constexpr uint64_t kLaunchAhead = 12, kKnownAhead = 16;
+struct PollPlan {
+  uint64_t iterations;
+  bool last;
+};
+constexpr PollPlan PlanPoll(uint64_t bound, uint64_t launched, uint32_t per_poll) {
+  if (bound <= launched) return {per_poll, false};
+  const uint64_t left = bound - launched;
+  const uint64_t known = bound <= kLaunchAhead ? bound : bound <= kKnownAhead ? (launched ? 4 : 8) : 0;
+  const uint64_t group = known > per_poll ? known : per_poll;
+  return {group < left ? group : left, group >= left};
+}
+
 }  // namespace muonx
 
 #endif

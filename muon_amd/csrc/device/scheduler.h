@@ -92,9 +92,9 @@ class Scheduler {
   // requests starves it. Images do not depend on the slicing.
   //
   // `closed`: the caller submits nothing before the submitted jobs are done.
-  // A poll that starts with every one of their samples in the path queue and
-  // with bounded paths then launches the iterations that those paths need, no
-  // more, and waits for them (LastIteration).
+  // With every one of their samples in the path queue and bounded paths, no
+  // iteration is then launched after the one that ends the longest of them, which
+  // is waited for (PathBound, PlanPoll).
   int Step(std::vector<SchedJob> *finished, bool closed = false);
   bool Idle() const { return pending_.empty() && jobs_.empty(); }
   size_t pending() const { return pending_.size(); }
@@ -111,7 +111,7 @@ class Scheduler {
   int AdmitWork();
   int AdmitSlice(SchedJob &j);
   int Harvest(int b);
-  uint64_t LastIteration() const;
+  uint64_t PathBound() const;
   int FinishResolves(std::vector<SchedJob> *finished, bool wait_all);
   void AdvanceWindow();
 
@@ -130,6 +130,8 @@ class Scheduler {
   uint64_t snap_id_[2] = {0, 0};
   uint64_t snap_count_ = 0;
   uint64_t iterations_ = 0;
+  uint64_t first_iter_ = 0;     // iterations when the open paths were primed
+  uint64_t path_bound_ = 0;     // and how many of them end the longest path, 0 when not known
   uint64_t progress_iter_ = 0;  // iteration count when a sample last finished
   unsigned long long rays_[kRayCounters] = {};
 };

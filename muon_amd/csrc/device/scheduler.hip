@@ -307,13 +307,11 @@ int Scheduler::FinishResolves(std::vector<SchedJob> *finished, bool wait_all) {
   return MUONX_OK;
 }
 
-// The iteration that ends the last path of the open slices, right after Prime:
+// How many iterations end the longest path of the open slices, right after Prime:
 // with every sample of every submitted job in the path queue, a path of
 // depth cutoff c is retired by iteration c + 1. 0 when samples are left to
-// generate, a job's paths end by Russian roulette alone, or more than
-// kMostKnownIterations remain (most paths may end much earlier).
-uint64_t Scheduler::LastIteration() const {
-  constexpr int64_t kMostKnownIterations = 16;
+// generate or a job's paths end by Russian roulette alone.
+uint64_t Scheduler::PathBound() const {
   if (!pending_.empty() || open_items_ > cfg_.path_slots) return 0;
   int64_t most = 1;
   for (const auto &kv : jobs_) {
@@ -323,7 +321,7 @@ uint64_t Scheduler::LastIteration() const {
     if (j.next_sample < uint32_t(p.spp) || p.max_depth == -1) return 0;
     most = std::max<int64_t>(most, int64_t(p.max_depth) + (p.nee != MUONX_NEE_OFF ? 0 : 1));
   }
-  return most <= kMostKnownIterations ? iterations_ + uint64_t(most) : 0;
+  return uint64_t(most);
 }
 
 int Scheduler::Step(std::vector<SchedJob> *finished, bool closed) {
@@ -333,9 +331,12 @@ int Scheduler::Step(std::vector<SchedJob> *finished, bool closed) {
   const bool primed = idle && !slices_.empty();
   if (primed && (rc = eng_->Prime()) != MUONX_OK) return rc;
   if (!slices_.empty()) {
-    const uint64_t last = primed && closed ? LastIteration() : 0;
-    const uint64_t n = last ? last - iterations_ : cfg_.iterations_per_poll;
-    for (uint64_t i = 0; i < n; ++i) {
+    if (primed) {
+      first_iter_ = iterations_;
+      path_bound_ = closed ? PathBound() : 0;
+    }
+    const PollPlan plan = PlanPoll(path_bound_, iterations_ - first_iter_, cfg_.iterations_per_poll);
+    for (uint64_t i = 0; i < plan.iterations; ++i) {
       if ((rc = eng_->Iterate()) != MUONX_OK) return rc;
       ++iterations_;
     }
@@ -344,7 +345,7 @@ int Scheduler::Step(std::vector<SchedJob> *finished, bool closed) {
     snap_id_[b] = snap_count_++;
     snap_pending_[b] = true;
     snap_ ^= 1;
-    if (last) {  // everything is done: read these counters now (an older snapshot holds less)
+    if (plan.last) {  // everything is done: read these counters now (an older snapshot holds less)
       if ((rc = eng_->WaitDone(b)) != MUONX_OK) return rc;
       snap_pending_[0] = snap_pending_[1] = false;
       if ((rc = Harvest(b)) != MUONX_OK) return rc;

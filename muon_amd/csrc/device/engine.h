@@ -126,12 +126,6 @@ struct PathState {
   float4 *rad;    // radiance, pixel; moved by retire, not by shade
 };
 
-// nidx: the path's position in the next queue, or kPathEnds, and which of
-// the iteration's terms retire has to look for. Positions fit the 30 bits:
-// 2^30 paths would take 300 GB.
-constexpr uint32_t kPathNextMask = 0x3fffffffu, kPathEnds = kPathNextMask;
-constexpr uint32_t kPathHasMis = 0x40000000u, kPathHasShadow = 0x80000000u;
-
 struct EngArgs {
   const DevSceneView *scenes;
   const JobDev *jobs;

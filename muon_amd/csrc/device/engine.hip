@@ -880,8 +880,8 @@ int Engine::Create(muonx_ctx *ctx, const muonx_tuning &tuning, uint32_t capacity
     SetError("engine: max_jobs must be at most 65536");
     return MUONX_ERR_INVALID;
   }
-  if (capacity > (1u << 30) || uint64_t(capacity) * uint64_t(kmax) > kMaxShadowSlots) {
-    SetError("engine: paths in flight x shadow rays per vertex must stay below 2^31");
+  if (!EngineCapacityOk(capacity, uint64_t(kmax))) {
+    SetError("engine: paths in flight must stay below 2^30, times the shadow rays per vertex below 2^31");
     return MUONX_ERR_INVALID;
   }
   Engine *e = new Engine();

@@ -56,10 +56,21 @@ constexpr ItemPos ItemPosition(unsigned long long local, uint32_t npix, uint32_t
 }
 
 // Index of shadow ray k of path i (the shadow arrays hold kmax rays per path
-// in k-major order). Engine::Create keeps capacity * kmax <= 2^31, so the
-// index and the queue entries that store it fit 32 bits.
+// in k-major order). Engine::Create keeps capacity * kmax <= 2^31
+// (EngineCapacityOk), so the index and the queue entries that store it fit 32 bits.
 constexpr uint32_t ShadowSlot(uint32_t k, uint32_t capacity, uint32_t i) { return k * capacity + i; }
 constexpr unsigned long long kMaxShadowSlots = 1ull << 31;
+
+// nidx: the path's position in the next queue, or kPathEnds, and which of
+// the iteration's terms retire has to look for.
+constexpr uint32_t kPathNextMask = 0x3fffffffu, kPathEnds = kPathNextMask;
+constexpr uint32_t kPathHasMis = 0x40000000u, kPathHasShadow = 0x80000000u;
+
+// Whether an engine can hold `capacity` paths of `kmax` shadow rays per vertex:
+// every queue position lies below kPathEnds and every shadow slot below 2^31.
+constexpr bool EngineCapacityOk(uint64_t capacity, uint64_t kmax) {
+  return capacity <= kPathEnds && capacity * kmax <= kMaxShadowSlots;
+}
 
 // Byte layout of the engine's buffers: arrays of `per_path` elements of
 // `elem_bytes` per path (per path and shadow ray for the shadow buffer), in

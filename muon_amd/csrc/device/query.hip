@@ -2,6 +2,7 @@
 // (muonx_intersect_closest / muonx_intersect_any).
 #include "exact_trace.h"
 #include "query.h"
+#include "query_parts.h"
 #include "runtime.h"
 #include "trace.h"
 #include "traverse_launch.h"
@@ -178,11 +179,8 @@ template <bool ANY, bool COUNT>
 struct QueryDynLaunch {
   const TraverseCfg &cfg;
   const DevSceneView &s;
-  const float *ro, *rd, *tmax;
+  const QueryArrays &q;
   uint32_t n;
-  int32_t *prim;
-  float *t;
-  uint8_t *occ;
   unsigned long long *counters;
   uint32_t *next;
   int fetch_min;
@@ -191,7 +189,7 @@ struct QueryDynLaunch {
   void run() const {
     const StackArgs sa{cfg.spill, cfg.gcap};
     hipLaunchKernelGGL((k_query_dyn<KIND, WIDTH, ANY, COUNT>), dim3(cfg.grid), dim3(kQueryBlock), 0, stream, s, sa,
-                       ro, rd, tmax, n, prim, t, occ, counters, next, fetch_min);
+                       q.o, q.d, q.tmax, n, q.prim, q.t, q.occ, counters, next, fetch_min);
   }
 };
 
@@ -199,18 +197,15 @@ template <bool ANY, bool COUNT>
 struct QueryLaunch {
   const TraverseCfg &cfg;
   const DevSceneView &s;
-  const float *ro, *rd, *tmax;
+  const QueryArrays &q;
   uint32_t n;
-  int32_t *prim;
-  float *t;
-  uint8_t *occ;
   unsigned long long *counters;
   hipStream_t stream;
   template <int KIND, bool WW, int WIDTH>
   void run() const {
     const StackArgs sa{cfg.spill, cfg.gcap};
     hipLaunchKernelGGL((k_query<KIND, WW, WIDTH, ANY, COUNT>), dim3(cfg.grid), dim3(kQueryBlock), 0, stream,
-                       s, sa, ro, rd, tmax, n, prim, t, occ, counters);
+                       s, sa, q.o, q.d, q.tmax, n, q.prim, q.t, q.occ, counters);
   }
 };
 }  // namespace
@@ -285,9 +280,7 @@ static int ClearClaims(muonx_ctx *ctx, hipStream_t stream, bool noalloc, void *s
 // level-6 icosphere; with whole stacks in LDS, as many as its LDS holds.
 constexpr int kExactBlocksPerCu = 12;
 constexpr int kLdsBytes = 160 << 10;  // of a CU
-constexpr uint32_t kExactPart = 1u << 30;  // rays per launch: 3 * index stays below 2^32
-static int LaunchExactQuery(muonx_ctx *ctx, const DevSceneView &s, bool any, const float *ro, const float *rd,
-                            const float *tmax, uint32_t n, int32_t *prim, float *t, uint8_t *occ,
+static int LaunchExactQuery(muonx_ctx *ctx, const DevSceneView &s, bool any, const QueryArrays &q, uint32_t n,
                             unsigned long long *counters, hipStream_t stream, bool noalloc, void *scratch_base) {
   if (s.bvh_depth > 96) {
     SetError("BVH depth " + std::to_string(s.bvh_depth) + " exceeds the exact-mode traversal stack (96)");
@@ -296,22 +289,16 @@ static int LaunchExactQuery(muonx_ctx *ctx, const DevSceneView &s, bool any, con
   const int cap = s.bvh_depth <= 24 ? 24 : s.bvh_depth <= 48 ? 48 : 96;
   const int per_cu = noalloc ? std::min(kExactBlocksPerCu, kLdsBytes / (cap * kQueryBlock * int(sizeof(uint2))))
                              : kExactBlocksPerCu;
-  for (uint32_t at = 0; at < n; at += std::min(n - at, kExactPart)) {
-    const uint32_t m = std::min(n - at, kExactPart);
-    const uint64_t cus = uint64_t(ctx->num_cus > 0 ? ctx->num_cus : 256);
-    const uint32_t grid = ClaimBlocks(m, uint32_t(cus) * uint32_t(per_cu), kWavesPerBlock);
-    uint32_t *next = nullptr;
-    if (NeedsClaims(m, grid * kWavesPerBlock)) {
-      const int rc = ClearClaims(ctx, stream, noalloc, scratch_base, &next);
-      if (rc != MUONX_OK) return rc;
-    }
-    const float *o = ro + 3 * size_t(at), *d = rd + 3 * size_t(at), *tm = tmax ? tmax + at : nullptr;
-    int32_t *po = prim ? prim + at : nullptr;
-    float *to = t ? t + at : nullptr;
-    uint8_t *oo = occ ? occ + at : nullptr;
+  const uint32_t cus = uint32_t(ctx->num_cus > 0 ? ctx->num_cus : 256);
+  const uint32_t grid = ClaimBlocks(n, cus * uint32_t(per_cu), kWavesPerBlock);
+  uint32_t *next = nullptr;
+  if (NeedsClaims(n, grid * kWavesPerBlock)) {
+    const int rc = ClearClaims(ctx, stream, noalloc, scratch_base, &next);
+    if (rc != MUONX_OK) return rc;
+  }
 #define MX_QX(CAP, P, A, C) \
-  hipLaunchKernelGGL((k_query_exact<CAP, P, A, C>), dim3(grid), dim3(kQueryBlock), 0, stream, s, o, d, tm, m, po, to, \
-                     oo, counters, next)
+  hipLaunchKernelGGL((k_query_exact<CAP, P, A, C>), dim3(grid), dim3(kQueryBlock), 0, stream, s, q.o, q.d, q.tmax, n, \
+                     q.prim, q.t, q.occ, counters, next)
 #define MX_QXP(CAP, A, C) \
   if (noalloc) MX_QX(CAP, false, A, C); \
   else MX_QX(CAP, true, A, C)
@@ -319,30 +306,27 @@ static int LaunchExactQuery(muonx_ctx *ctx, const DevSceneView &s, bool any, con
   if (cap == 24) { MX_QXP(24, A, C); } \
   else if (cap == 48) { MX_QXP(48, A, C); } \
   else { MX_QXP(96, A, C); }
-    if (any) {
-      MX_QXC(true, false);
-    } else if (counters) {
-      MX_QXC(false, true);
-    } else {
-      MX_QXC(false, false);
-    }
+  if (any) {
+    MX_QXC(true, false);
+  } else if (counters) {
+    MX_QXC(false, true);
+  } else {
+    MX_QXC(false, false);
+  }
 #undef MX_QXC
 #undef MX_QXP
 #undef MX_QX
-    MX_HIP(hipGetLastError());
-    if (next && !noalloc) MX_HIP(hipEventRecord(ctx->spill_done, stream));
-  }
+  MX_HIP(hipGetLastError());
+  if (next && !noalloc) MX_HIP(hipEventRecord(ctx->spill_done, stream));
   return MUONX_OK;
 }
 
-// Launches the query kernels. With `noalloc` the spill region and the claim
+// Launches the query kernels for up to kQueryPart rays. With `noalloc` the spill region and the claim
 // counters come from the static scratch (the grid is capped so that the spill
 // fits), the counters are cleared by a kernel rather than a memset node, no
 // stack is in private memory, and no event or buffer is created.
-int LaunchQuery(muonx_ctx *ctx, const DevSceneView &s, bool any, bool exact, const float *ro, const float *rd,
-                const float *tmax, uint32_t n, int32_t *prim, float *t, uint8_t *occ, unsigned long long *counters,
-                hipStream_t stream, bool noalloc) {
-  if (n == 0) return MUONX_OK;
+static int LaunchPart(muonx_ctx *ctx, const DevSceneView &s, bool any, bool exact, const QueryArrays &q, uint32_t n,
+                      unsigned long long *counters, hipStream_t stream, bool noalloc) {
   TraverseCfg cfg;
   unsigned char *sbase = nullptr;
   int rc;
@@ -353,7 +337,7 @@ int LaunchQuery(muonx_ctx *ctx, const DevSceneView &s, bool any, bool exact, con
       return MUONX_ERR_STATE;
     }
   }
-  if (exact) return LaunchExactQuery(ctx, s, any, ro, rd, tmax, n, prim, t, occ, counters, stream, noalloc, sbase);
+  if (exact) return LaunchExactQuery(ctx, s, any, q, n, counters, stream, noalloc, sbase);
   if (noalloc) {
     rc = PlanTraverseShape(ctx->tuning, ctx->num_cus, s.bvh_depth, s.wstack, n, kQueryBlock, cfg, false);
     if (rc != MUONX_OK) return rc;
@@ -375,16 +359,15 @@ int LaunchQuery(muonx_ctx *ctx, const DevSceneView &s, bool any, bool exact, con
     if (rc != MUONX_OK) return rc;
     if ((rc = BeginSpill(ctx, cfg, stream)) != MUONX_OK) return rc;
   }
-#define MX_Q(A, C) DispatchTraverse(cfg, QueryLaunch<A, C>{cfg, s, ro, rd, tmax, n, prim, t, occ, counters, stream})
+#define MX_Q(A, C) DispatchTraverse(cfg, QueryLaunch<A, C>{cfg, s, q, n, counters, stream})
   const bool cnt = counters != nullptr;
   const int fetch = ctx->tuning.ray_fetch;
-  if (fetch > 0 && n <= (1u << 31)) {  // claimed indices stay below 2^32
-    // per-lane ray fetch
+  if (fetch > 0) {  // per-lane ray fetch
     uint32_t *next = nullptr;
     if (NeedsClaims(n, uint32_t(cfg.grid) * kWavesPerBlock) &&
         (rc = ClearClaims(ctx, stream, noalloc, sbase, &next)) != MUONX_OK)
       return rc;
-#define MX_QD(A, C) DispatchTraverse(cfg, QueryDynLaunch<A, C>{cfg, s, ro, rd, tmax, n, prim, t, occ, counters, next, fetch, stream})
+#define MX_QD(A, C) DispatchTraverse(cfg, QueryDynLaunch<A, C>{cfg, s, q, n, counters, next, fetch, stream})
     if (any) {
       if (cnt) MX_QD(true, true);
       else MX_QD(true, false);
@@ -407,6 +390,14 @@ int LaunchQuery(muonx_ctx *ctx, const DevSceneView &s, bool any, bool exact, con
 #undef MX_Q
   MX_HIP(hipGetLastError());
   return noalloc ? MUONX_OK : EndSpill(ctx, cfg, stream);
+}
+
+int LaunchQuery(muonx_ctx *ctx, const DevSceneView &s, bool any, bool exact, const float *ro, const float *rd,
+                const float *tmax, uint32_t n, int32_t *prim, float *t, uint8_t *occ, unsigned long long *counters,
+                hipStream_t stream, bool noalloc) {
+  return ForEachPart(QueryArrays{ro, rd, tmax, prim, t, occ}, n, kQueryPart, [&](const QueryArrays &q, uint32_t m) {
+    return LaunchPart(ctx, s, any, exact, q, m, counters, stream, noalloc);
+  });
 }
 
 }  // namespace muonx

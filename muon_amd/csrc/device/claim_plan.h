@@ -18,8 +18,8 @@ namespace muonx {
 //    wavefront) from one of up to kClaimGroups counters, each handing out
 //    every 16th chunk. Groups are made of eight consecutive blocks,
 //    one on each XCD, so that a slower XCD takes fewer chunks of every group.
-//    A launch without counters (a captured one, whose replays no clear or
-//    order between streams would cover) takes every waves-th chunk here too.
+// A captured launch, whose replays no clear or order between streams would
+// cover, stays within UnclaimedItems.
 // Atomics on one address take 11.3 ns each here however few wavefronts are
 // left (1.8 ns spread over 8 addresses, 0.24 over 64), so one counter bounds
 // a launch by its chunks: 3,000,017 any-hit rays on 10,000 spheres take 677 us
@@ -40,7 +40,9 @@ constexpr uint32_t kClaimStride = 64;  // counters on 256-byte lines of their ow
 constexpr size_t kClaimBytes = size_t(kClaimGroups) * kClaimStride * sizeof(uint32_t);
 constexpr uint32_t kSpreadWaves = 2048, kSpreadMin = 2;
 
-constexpr bool NeedsClaims(uint32_t items, uint32_t waves) { return items > uint64_t(waves) * kChunk * kStaticRounds; }
+// The most items that `waves` wavefronts take without a counter.
+constexpr uint64_t UnclaimedItems(uint32_t waves) { return uint64_t(waves) * kChunk * kStaticRounds; }
+constexpr bool NeedsClaims(uint32_t items, uint32_t waves) { return items > UnclaimedItems(waves); }
 // Items in a wavefront's first chunk.
 constexpr uint32_t FirstChunk(uint32_t items, uint32_t waves) {
   const uint32_t each = items / (waves < kSpreadWaves ? waves : kSpreadWaves) + 1u;
@@ -65,9 +67,9 @@ struct ClaimPlan {
   uint32_t group, groups;      // claimed chunks: the counter and their number, 0 for none,
   uint32_t chunk;              // the items of each
   constexpr ClaimPlan(uint32_t items, uint32_t blocks, uint32_t waves, uint32_t wave, uint32_t block,
-                      uint32_t max_chunk, bool counters = true)
+                      uint32_t max_chunk)
       : cbase(0), cend(0), snext(0), send(0), step(0), group(0), groups(0), chunk(kChunk) {
-    if (counters && NeedsClaims(items, waves)) {
+    if (NeedsClaims(items, waves)) {
       groups = (blocks + 7u) / 8u < kClaimGroups ? (blocks + 7u) / 8u : kClaimGroups;  // none without blocks
       group = (block >> 3) % groups;
       const uint32_t c = (items / (4u * waves)) & ~63u;

@@ -66,7 +66,7 @@ __global__ void __launch_bounds__(kQueryBlock) __attribute__((amdgpu_waves_per_e
   auto st = make_stack<KIND>(lds, kQueryBlock, sa, old);
   LaneTrace<WIDTH, ANY, COUNT> lt;
   uint32_t idx = 0;
-  WaveFetch wf(n, kChunk, next != nullptr);
+  WaveFetch wf(n, kChunk);
   bool walking = false, have = false, drained = false;
   while (true) {
     const uint64_t needm = __builtin_amdgcn_ballot_w64(!have && !drained);
@@ -137,7 +137,7 @@ __global__ void __launch_bounds__(kQueryBlock)
   auto st = Stack::make(lds, old);
   ExactWalk<COUNT, ANY ? kWalkAny : kWalkClosest> w;
   TraceCounters cnt;
-  WaveFetch wf(n, kChunk, next != nullptr);
+  WaveFetch wf(n, kChunk);
   uint32_t idx = 0;
   bool walking = false, have = false, drained = false;
   while (true) {
@@ -251,16 +251,7 @@ int InitStaticScratch(int device) {
 // The claim counters of the per-lane fetch kernels, cleared on `stream`: in
 // the static scratch with `noalloc` (by a kernel rather than a memset node),
 // else in the context, ordered after its previous user like the spill region.
-// None under capture: on replays after the first the recorded memset has left
-// the counters as they were, and no replay waits for the context's other calls.
 static int ClearClaims(muonx_ctx *ctx, hipStream_t stream, bool noalloc, void *scratch_base, uint32_t **next) {
-  bool capturing = false;
-  if (!noalloc) {
-    const int rc = IsCapturing(stream, &capturing);
-    if (rc != MUONX_OK) return rc;
-  }
-  *next = nullptr;
-  if (capturing) return MUONX_OK;
   if (noalloc) {
     *next = static_cast<uint32_t *>(scratch_base);
     hipLaunchKernelGGL(k_clear_claims, dim3(1), dim3(kClaimGroups), 0, stream, *next);
@@ -271,6 +262,32 @@ static int ClearClaims(muonx_ctx *ctx, hipStream_t stream, bool noalloc, void *s
   MX_HIP(hipStreamWaitEvent(stream, ctx->spill_done, 0));
   MX_HIP(hipMemsetAsync(ctx->fetch_ctr.ptr, 0, kClaimBytes, stream));
   *next = ctx->fetch_ctr.as<uint32_t>();
+  return MUONX_OK;
+}
+
+// Calls launch(arrays, rays, counters) for n rays on `waves` wavefronts, with
+// cleared claim counters (else null) where they need them; `counted` says whether
+// the context's were used. Under capture the rays go out in parts that need none:
+// on replays after the first a recorded memset has left the counters as they
+// were, and no replay waits for the context's other calls.
+template <class F>
+static int LaunchClaiming(muonx_ctx *ctx, const QueryArrays &q, uint32_t n, uint32_t waves, hipStream_t stream,
+                          bool noalloc, void *scratch_base, bool *counted, F &&launch) {
+  *counted = false;
+  uint32_t *next = nullptr;
+  if (NeedsClaims(n, waves)) {
+    bool capturing = false;
+    int rc = noalloc ? MUONX_OK : IsCapturing(stream, &capturing);
+    if (rc != MUONX_OK) return rc;
+    if (capturing)
+      return ForEachPart(q, n, uint32_t(UnclaimedItems(waves)), [&](const QueryArrays &part, uint32_t m) {
+        launch(part, m, next);
+        return MUONX_OK;
+      });
+    if ((rc = ClearClaims(ctx, stream, noalloc, scratch_base, &next)) != MUONX_OK) return rc;
+    *counted = !noalloc;
+  }
+  launch(q, n, next);
   return MUONX_OK;
 }
 
@@ -291,13 +308,9 @@ static int LaunchExactQuery(muonx_ctx *ctx, const DevSceneView &s, bool any, con
                              : kExactBlocksPerCu;
   const uint32_t cus = uint32_t(ctx->num_cus > 0 ? ctx->num_cus : 256);
   const uint32_t grid = ClaimBlocks(n, cus * uint32_t(per_cu), kWavesPerBlock);
-  uint32_t *next = nullptr;
-  if (NeedsClaims(n, grid * kWavesPerBlock)) {
-    const int rc = ClearClaims(ctx, stream, noalloc, scratch_base, &next);
-    if (rc != MUONX_OK) return rc;
-  }
+  const auto launch = [&](const QueryArrays &q, uint32_t m, uint32_t *next) {
 #define MX_QX(CAP, P, A, C) \
-  hipLaunchKernelGGL((k_query_exact<CAP, P, A, C>), dim3(grid), dim3(kQueryBlock), 0, stream, s, q.o, q.d, q.tmax, n, \
+  hipLaunchKernelGGL((k_query_exact<CAP, P, A, C>), dim3(grid), dim3(kQueryBlock), 0, stream, s, q.o, q.d, q.tmax, m, \
                      q.prim, q.t, q.occ, counters, next)
 #define MX_QXP(CAP, A, C) \
   if (noalloc) MX_QX(CAP, false, A, C); \
@@ -306,18 +319,22 @@ static int LaunchExactQuery(muonx_ctx *ctx, const DevSceneView &s, bool any, con
   if (cap == 24) { MX_QXP(24, A, C); } \
   else if (cap == 48) { MX_QXP(48, A, C); } \
   else { MX_QXP(96, A, C); }
-  if (any) {
-    MX_QXC(true, false);
-  } else if (counters) {
-    MX_QXC(false, true);
-  } else {
-    MX_QXC(false, false);
-  }
+    if (any) {
+      MX_QXC(true, false);
+    } else if (counters) {
+      MX_QXC(false, true);
+    } else {
+      MX_QXC(false, false);
+    }
 #undef MX_QXC
 #undef MX_QXP
 #undef MX_QX
+  };
+  bool counted;
+  const int rc = LaunchClaiming(ctx, q, n, grid * kWavesPerBlock, stream, noalloc, scratch_base, &counted, launch);
+  if (rc != MUONX_OK) return rc;
   MX_HIP(hipGetLastError());
-  if (next && !noalloc) MX_HIP(hipEventRecord(ctx->spill_done, stream));
+  if (counted) MX_HIP(hipEventRecord(ctx->spill_done, stream));
   return MUONX_OK;
 }
 
@@ -363,21 +380,22 @@ static int LaunchPart(muonx_ctx *ctx, const DevSceneView &s, bool any, bool exac
   const bool cnt = counters != nullptr;
   const int fetch = ctx->tuning.ray_fetch;
   if (fetch > 0) {  // per-lane ray fetch
-    uint32_t *next = nullptr;
-    if (NeedsClaims(n, uint32_t(cfg.grid) * kWavesPerBlock) &&
-        (rc = ClearClaims(ctx, stream, noalloc, sbase, &next)) != MUONX_OK)
-      return rc;
-#define MX_QD(A, C) DispatchTraverse(cfg, QueryDynLaunch<A, C>{cfg, s, q, n, counters, next, fetch, stream})
-    if (any) {
-      if (cnt) MX_QD(true, true);
-      else MX_QD(true, false);
-    } else {
-      if (cnt) MX_QD(false, true);
-      else MX_QD(false, false);
-    }
+    const auto launch = [&](const QueryArrays &q, uint32_t m, uint32_t *next) {
+#define MX_QD(A, C) DispatchTraverse(cfg, QueryDynLaunch<A, C>{cfg, s, q, m, counters, next, fetch, stream})
+      if (any) {
+        if (cnt) MX_QD(true, true);
+        else MX_QD(true, false);
+      } else {
+        if (cnt) MX_QD(false, true);
+        else MX_QD(false, false);
+      }
 #undef MX_QD
+    };
+    bool counted;
+    rc = LaunchClaiming(ctx, q, n, uint32_t(cfg.grid) * kWavesPerBlock, stream, noalloc, sbase, &counted, launch);
+    if (rc != MUONX_OK) return rc;
     MX_HIP(hipGetLastError());
-    if (!noalloc && (next || cfg.spill)) MX_HIP(hipEventRecord(ctx->spill_done, stream));
+    if (counted || (cfg.spill && !noalloc)) MX_HIP(hipEventRecord(ctx->spill_done, stream));
     return MUONX_OK;
   }
   if (any) {

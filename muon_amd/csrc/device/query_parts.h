@@ -8,7 +8,7 @@
 
 namespace muonx {
 
-// Rays per launch: the kernels index the rays' coordinates (3 * ray + axis) and
+// The most rays of a launch: the kernels index the rays' coordinates (3 * ray + axis) and
 // step over rays in 32 bits.
 constexpr uint32_t kQueryPart = 1u << 30;
 

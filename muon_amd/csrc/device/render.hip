@@ -128,7 +128,7 @@ __global__ void __launch_bounds__(kSimpleBlock) __attribute__((amdgpu_waves_per_
   PrivateStack<CAP> st(lds + threadIdx.x, kSimpleBlock, old);
   ExactWalk<true, kWalkClosest> w;
   TraceCounters cnt;
-  WaveFetch wf(items, kChunk, next != nullptr);
+  WaveFetch wf(items, kChunk);
   uint32_t traced = 0;
   ImageItem i;
   bool walking = false, have = false, drained = false;
@@ -227,7 +227,7 @@ __global__ void __launch_bounds__(kSimpleBlock) __attribute__((amdgpu_waves_per_
   PrivateStack<CAP> st(lds + threadIdx.x, kSimpleBlock, old);
   ExactWalk<true, kWalkEither> w;
   TraceCounters cnt;
-  WaveFetch wf(items, kChunk, next != nullptr);
+  WaveFetch wf(items, kChunk);
   uint32_t n_primary = 0, n_secondary = 0, n_shadow = 0;
   ImageItem i;
   int nb = 0;  // bounces with a hit (the depth of the next)
@@ -414,7 +414,8 @@ class ScratchTurn {
 
 // Runs one of the deterministic integrators; `counters` holds the trace
 // counters and the (cleared) claim counters. Without claim counters the launches
-// use no other buffer of the context either: one sample each, added directly.
+// use no other buffer of the context either: one sample each, added directly, of
+// as many pixels as their wavefronts take without.
 int RenderDeterministic(muonx_scene *scene, const muonx_render_params &p, float *accum, const RenderCounters &counters,
                         RenderWorkspace *ws, hipStream_t stream) {
   const DevSceneView &s = scene->view;
@@ -441,14 +442,16 @@ int RenderDeterministic(muonx_scene *scene, const muonx_render_params &p, float 
   // muon/integration.cc:29-33
   const int cutoff = p.max_depth == -1 ? INT_MAX : (p.nee != MUONX_NEE_OFF ? p.max_depth - 1 : p.max_depth);
   const bool whitted = p.integrator == MUONX_INTEGRATOR_RAYTRACER || p.integrator == MUONX_INTEGRATOR_ANALYTICDIRECT;
+  const uint32_t max_blocks = cus * (whitted ? kWhittedBlocksPerCu : kSimpleBlocksPerCu);
   bool cleared = true;  // the claim counters
   for (it.first = 0; it.first < p.spp; it.first += it.count) {
     it.count = std::min(batch, p.spp - it.first);
-    const uint64_t part = std::max<uint64_t>(1, (1u << 24) / uint64_t(it.count));  // tiles per launch: below 2^31 items
+    uint64_t part = std::max<uint64_t>(1, (1u << 24) / uint64_t(it.count));  // tiles per launch: below 2^31 items
+    if (!next) part = std::min(part, UnclaimedItems(max_blocks * (kSimpleBlock / 64)) / 64);
     for (it.tile0 = 0; it.tile0 < tiles; it.tile0 += part) {
       const uint32_t items = uint32_t(std::min(tiles - it.tile0, part)) * uint32_t(it.count) * 64u;
-      const uint32_t blocks = ClaimBlocks(items, cus * (whitted ? kWhittedBlocksPerCu : kSimpleBlocksPerCu), kSimpleBlock / 64);
-      if (next && NeedsClaims(items, blocks * (kSimpleBlock / 64))) {
+      const uint32_t blocks = ClaimBlocks(items, max_blocks, kSimpleBlock / 64);
+      if (NeedsClaims(items, blocks * (kSimpleBlock / 64))) {
         if (!cleared) MX_HIP(hipMemsetAsync(next, 0, kClaimBytes, stream));
         cleared = false;
       }

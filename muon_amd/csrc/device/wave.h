@@ -154,10 +154,10 @@ __device__ __forceinline__ void wave_count(uint32_t n, unsigned long long *ctr) 
 // in every lane.
 struct WaveFetch {
   ClaimPlan p;
-  __device__ __forceinline__ explicit WaveFetch(uint32_t items, uint32_t max_chunk = 256, bool counters = true)
+  __device__ __forceinline__ explicit WaveFetch(uint32_t items, uint32_t max_chunk = 256)
       : p(items, gridDim.x, gridDim.x * (blockDim.x >> 6),
           uint32_t(__builtin_amdgcn_readfirstlane(int(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)))),
-          blockIdx.x, max_chunk, counters) {}
+          blockIdx.x, max_chunk) {}
   // Called by every lane of the wavefront with the ballot of `need`; returns
   // the index claimed for this lane (meaningful where `need` is set; an
   // index >= the item count means none is left).

@@ -10,7 +10,7 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
-@pytest.mark.parametrize("name", ["static_claims_check", "poll_plan_check", "path_capacity_check",
+@pytest.mark.parametrize("name", ["poll_plan_check", "path_capacity_check",
                                   "query_parts_check"])
 def test_cpu_check(name, tmp_path):
     if shutil.which("g++") is None:

@@ -486,13 +486,10 @@ int RenderDeterministic(muonx_scene *scene, const muonx_render_params &p, float 
 
 using namespace muonx;
 
-extern "C" int muonx_render(muonx_scene *scene, const muonx_render_params *params, float *accum,
-                            muonx_trace_stats *stats, void *stream_) {
-  if (!scene || !params || !accum) {
-    SetError("muonx_render: null argument");
-    return MUONX_ERR_INVALID;
-  }
-  const muonx_render_params &p = *params;
+namespace {
+// muonx_render with the context's lock held.
+int RenderLocked(muonx_scene *scene, const muonx_render_params &p, float *accum, muonx_trace_stats *stats,
+                 hipStream_t stream) {
   if (p.width <= 0 || p.height <= 0 || p.spp <= 0) {
     SetError("muonx_render: width, height and spp must be positive");
     return MUONX_ERR_INVALID;
@@ -507,9 +504,7 @@ extern "C" int muonx_render(muonx_scene *scene, const muonx_render_params *param
     return MUONX_ERR_STATE;
   }
   muonx_ctx *ctx = scene->ctx;
-  std::lock_guard<std::mutex> lock(ctx->mu);
   MX_HIP(hipSetDevice(ctx->device));
-  hipStream_t stream = static_cast<hipStream_t>(stream_);
   bool capturing = false;
   int rc = IsCapturing(stream, &capturing);
   if (rc != MUONX_OK) return rc;
@@ -579,6 +574,17 @@ extern "C" int muonx_render(muonx_scene *scene, const muonx_render_params *param
   (void)hipEventDestroy(e1);
   return MUONX_OK;
 }
+}  // namespace
+
+extern "C" int muonx_render(muonx_scene *scene, const muonx_render_params *params, float *accum,
+                            muonx_trace_stats *stats, void *stream) {
+  if (!scene || !params || !accum) {
+    SetError("muonx_render: null argument");
+    return MUONX_ERR_INVALID;
+  }
+  std::lock_guard<std::mutex> lock(scene->ctx->mu);
+  return RenderLocked(scene, *params, accum, stats, static_cast<hipStream_t>(stream));
+}
 
 extern "C" int muonx_render_host(muonx_scene *scene, const muonx_render_params *params, float *accum_host,
                                  muonx_trace_stats *stats) {
@@ -591,15 +597,13 @@ extern "C" int muonx_render_host(muonx_scene *scene, const muonx_render_params *
     return MUONX_ERR_INVALID;
   }
   const size_t bytes = size_t(params->width) * size_t(params->height) * 3 * sizeof(float);
-  float *dev = nullptr;
-  {
-    std::lock_guard<std::mutex> lock(scene->ctx->mu);
-    MX_HIP(hipSetDevice(scene->ctx->device));
-    RenderWorkspace *ws = GetWorkspace(scene->ctx);
-    MX_HIP(ws->film.Reserve(bytes));
-    dev = ws->film.as<float>();
-  }
-  const int rc = muonx_render(scene, params, dev, stats, nullptr);
+  // one call at a time from the film's allocation to its copy: the next may move it
+  std::lock_guard<std::mutex> lock(scene->ctx->mu);
+  MX_HIP(hipSetDevice(scene->ctx->device));
+  RenderWorkspace *ws = GetWorkspace(scene->ctx);
+  MX_HIP(ws->film.Reserve(bytes));
+  float *dev = ws->film.as<float>();
+  const int rc = RenderLocked(scene, *params, dev, stats, nullptr);
   if (rc != MUONX_OK) return rc;
   MX_HIP(hipMemcpy(accum_host, dev, bytes, hipMemcpyDeviceToHost));
   return MUONX_OK;

@@ -1,5 +1,6 @@
-// Wavefront-level helpers (64 lanes): queue appends with one atomic per
-// wavefront and counter reductions.
+// Helpers of wavefronts (64 lanes) and blocks: queue appends with one atomic per
+// block, exchange through LDS within a wavefront, counter reductions and the
+// claiming of work.
 #ifndef MUONX_DEVICE_WAVE_H_
 #define MUONX_DEVICE_WAVE_H_
 
@@ -11,65 +12,10 @@
 
 namespace muonx {
 
-// Appends the lanes with `want` to a queue: returns each such lane's index
-// (lane order within the wavefront).
-__device__ __forceinline__ uint32_t wave_append(bool want, uint32_t *counter) {
-  const uint64_t active = __ballot(1);
-  const uint64_t mask = __ballot(want);
-  const uint32_t lane = __lane_id();
-  const uint32_t leader = uint32_t(__ffsll((unsigned long long)active) - 1);
-  uint32_t base = 0;
-  if (lane == leader && mask) base = atomicAdd(counter, uint32_t(__popcll(mask)));
-  base = uint32_t(__shfl(int(base), int(leader)));
-  return base + uint32_t(__popcll(mask & ((1ull << lane) - 1ull)));
-}
-
-// Reserves `cnt` consecutive entries per lane with one atomic per wavefront
-// (exclusive prefix sum over the lanes); all 64 lanes must be active.
-__device__ __forceinline__ uint32_t wave_append_n(uint32_t cnt, uint32_t *counter) {
-  const int lane = int(__lane_id());
-  uint32_t incl = cnt;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const uint32_t v = uint32_t(__shfl_up(int(incl), off));
-    if (lane >= off) incl += v;
-  }
-  const uint32_t total = uint32_t(__shfl(int(incl), 63));
-  uint32_t base = 0;
-  if (lane == 63 && total) base = atomicAdd(counter, total);
-  base = uint32_t(__shfl(int(base), 63));
-  return base + incl - cnt;
-}
-
-// Block-wide versions: NW wavefronts (blockDim.x = 64 * NW) reserve their
-// entries with one atomic per block, in block order. Every thread of the
-// block must call them (they synchronise the block); `sh` is NW + 1 words of
-// shared memory.
-template <int NW>
-__device__ __forceinline__ uint32_t block_append_n(uint32_t cnt, uint32_t *counter, uint32_t *sh) {
-  const int lane = int(__lane_id());
-  const int w = int(threadIdx.x) >> 6;
-  uint32_t incl = cnt;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const uint32_t v = uint32_t(__shfl_up(int(incl), off));
-    if (lane >= off) incl += v;
-  }
-  if (lane == 63) sh[w] = incl;  // the wavefront's total
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    uint32_t tot = 0;
-#pragma unroll
-    for (int k = 0; k < NW; ++k) tot += sh[k];
-    sh[NW] = tot ? atomicAdd(counter, tot) : 0u;
-  }
-  __syncthreads();
-  uint32_t base = sh[NW];
-  for (int k = 0; k < w; ++k) base += sh[k];
-  __syncthreads();  // sh is reused by the next call
-  return base + incl - cnt;
-}
-
+// Appends a block's lanes with `want` to a queue: returns each such lane's index.
+// NW wavefronts (blockDim.x = 64 * NW) reserve their entries with one atomic per
+// block, in block order. Every thread of the block must call it (it synchronises
+// the block); `sh` is NW + 1 words of shared memory.
 template <int NW>
 __device__ __forceinline__ uint32_t block_append(bool want, uint32_t *counter, uint32_t *sh) {
   const uint64_t m = __ballot(want);

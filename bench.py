@@ -18,7 +18,10 @@ set against the MALL read rate measured in the run by a streaming-read
 probe (mall_frac; read_measured_gbs holds its L2, MALL and HBM rates).
 `traffic` is the kernel's measured traffic past L2 per launch (rocprofv3
 FETCH_SIZE / WRITE_SIZE scaled by a copy of known size, from
-profiles/traffic_closest_icosphere.json). reference_equivalent gives the
+profiles/traffic_closest_icosphere.json). `bound` names the resource that the
+fractions are of, not the limit: most of these bytes hit caches, and what the
+kernel waits for is VALU issue at about 40 % lane use and dependent fetches
+(profiles/closest_icosphere.md). reference_equivalent gives the
 bytes the reference's binary SAH tree would move for the same rays,
 32 + 16 + 32 per bounds test + 36 per object test (its counters measured by
 the CPU restatement on a sample of the rays).

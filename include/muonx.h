@@ -210,8 +210,9 @@ void muonx_ctx_destroy(muonx_ctx *ctx);
  * from the BVH depth); 8 or 16 = LDS ring of that many entries per lane (more
  * waves per CU) with older entries in the lane's private memory (8, up to 72
  * entries) or spilled to a per-thread HBM region (16, or deeper trees).
- * while_while: lanes walk internal nodes until each holds a leaf, then test
- * leaves together. blocks_per_cu: persistent grid size. path_budget_mb:
+ * while_while (with ray_fetch 0): lanes walk internal nodes until each holds a
+ * leaf, then test leaves together; with ray fetch, while half of the wavefront's
+ * walking lanes are at a node. blocks_per_cu: persistent grid size. path_budget_mb:
  * HBM for the path tracer's per-path state and queues. bvh_width: node
  * width of the fast traversal mode (the exact mode always walks the
  * reference's binary tree). */

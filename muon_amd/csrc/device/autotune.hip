@@ -92,7 +92,7 @@ extern "C" int muonx_autotune(muonx_scene *scene, const muonx_render_params *job
         for (int ww : {1, 0})
           for (int bpc : {8, 16, 24})
             for (int fetch : {0, 16, 32}) {
-              if (fetch > 0 && ww == 0) continue;  // the fetch kernels always walk while-while
+              if (fetch > 0 && ww == 0) continue;  // the fetch kernels have one loop form (run_walks)
               if (width == 2 && bits == 8) continue;  // quantized boxes exist for 4-wide nodes
               muonx_tuning c = base;
               c.bvh_width = width;

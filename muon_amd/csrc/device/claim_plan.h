@@ -27,7 +27,8 @@ namespace muonx {
 // on the Cornell box 224 us with one and 76 us static, 2^24 on the level-7
 // icosphere 2.59 and 2.54 ms (all static 3.03 ms: XCDs differ).
 //
-// Fewer items than lanes are spread over two wavefronts per SIMD before a
+// Fewer items than lanes are spread over two wavefronts per SIMD of the whole
+// card's 256 CUs (on fewer CUs over all of the grid's wavefronts) before a
 // wavefront gets all of its lanes an item: a wavefront takes as long as the
 // longest of its lanes at every step, and idle SIMDs cost nothing. 10,000
 // exact closest hits on the level-5 icosphere take 95 us against 128 us with

@@ -572,8 +572,9 @@ constexpr uint32_t kDoneTable = 64;  // per-block done-count entries (a power of
 // The film sums of a wavefront's finished paths go through LDS, so that an
 // atomic instruction covers consecutive words: neighbouring paths hold
 // neighbouring pixels, and with one instruction per colour component each
-// touched every line of the wavefront's pixels (level-7 icosphere, 512x512,
-// 64 spp: 27.75 -> 26.94 ms; Cornell box, 256x256, 16 spp: 1268 -> 1226 us).
+// touched every line of the wavefront's pixels (level-7 icosphere from one random
+// pose, 512x512, 64 spp: 27.75 -> 26.94 ms; Cornell box, 256x256, 16 spp: 1268 ->
+// 1226 us).
 __global__ void __launch_bounds__(kRetireBlock) k_eng_retire(EngArgs a, int cur) {
   const uint32_t n = a.c->qcount[cur].v;
   const PathState &ps = a.st[cur];
@@ -831,7 +832,7 @@ struct IterLaunch {
   int cur;
   int fetch;   // per-lane fetch threshold, 0 = grid-stride kernels
   bool count;  // traversal kernels count their box and primitive tests
-  bool plain;  // no admitted job has NEE on: one shade kernel, no shadow / MIS rays
+  bool plain;  // no admitted job has NEE on: no shadow / MIS rays, and none of their kernels
   hipStream_t st;
   template <int KIND, bool WW, int WIDTH>
   void run() const {

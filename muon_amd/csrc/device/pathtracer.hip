@@ -89,7 +89,7 @@ int RunInline(Scheduler *s, const muonx_job *jobs, uint32_t n, muonx_job_result 
   for (uint32_t i = 0; i < n; ++i)
     if ((rc = s->Validate(jobs[i])) != MUONX_OK) return rc;
   // Jobs without NEE first (in their order), then the others: while only the
-  // former are admitted the engine runs its single-shade-kernel iterations.
+  // former are admitted the engine's iterations have no shadow and MIS kernels.
   // A job's image does not depend on the order.
   for (int with_nee = 0; with_nee < 2; ++with_nee)
     for (uint32_t i = 0; i < n; ++i)

@@ -280,8 +280,9 @@ struct RingStack {
 // the lane's private memory `private_old` (CAP - kPrivateRing entries, an
 // array of the kernel): as little LDS as a RingStack of 8, with no region to
 // reserve or to order between launches, and without that region's addresses
-// in registers (the closest-hit query kernel then fits eight wavefronts per
-// SIMD without register spills).
+// in registers (at eight wavefronts per SIMD the closest-hit query kernel spills
+// one register, with the region four). The runtime keeps this memory for every
+// wavefront that the card can hold: 264 MiB for 64 old entries.
 constexpr int kPrivateRing = 8;
 template <int CAP>
 struct PrivateStack {

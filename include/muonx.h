@@ -317,7 +317,9 @@ int muonx_intersect_noalloc(muonx_scene *scene, const muonx_query *q, void *stre
  * Replaces the tile loop of muon::Renderer::Render (muon/renderer.cc:40-76):
  * Camera::CastRay + Integrator::Trace per sample + Film::SetPixel.
  * accum_rgb: device pointer to H*W*3 floats, row-major, receives the
- * unnormalised sum over samples (zeroed by the call). stats may be NULL. */
+ * unnormalised sum over samples (zeroed by the call). stats may be NULL: the
+ * deterministic integrators then return with their work enqueued on `stream`,
+ * and may be captured into a graph (after one call outside of capture). */
 int muonx_render(muonx_scene *scene, const muonx_render_params *params, float *accum_rgb,
                  muonx_trace_stats *stats, void *stream);
 

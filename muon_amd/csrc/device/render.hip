@@ -508,6 +508,11 @@ int RenderLocked(muonx_scene *scene, const muonx_render_params &p, float *accum,
   bool capturing = false;
   int rc = IsCapturing(stream, &capturing);
   if (rc != MUONX_OK) return rc;
+  if (capturing && p.integrator == MUONX_INTEGRATOR_PATHTRACER) {
+    // the host polls the engine's counters: nothing may reach its stream, whose work the graph would take in
+    SetError("muonx_render: the path tracer cannot be captured into a graph");
+    return MUONX_ERR_STATE;
+  }
   RenderWorkspace *ws = GetWorkspace(ctx);
   MX_HIP(ws->counters.Reserve(kRenderCounterBytes + kTraceCounterBytes));  // allocated once, never moved
   ScratchTurn turn(ws, stream);

@@ -13,7 +13,7 @@ from muon_amd import _lib  # noqa: E402
 from muon_amd.renderer import render_device  # noqa: E402
 
 
-NORMALS, RAYTRACER = 0, 3  # MUONX_INTEGRATOR_*
+NORMALS, RAYTRACER, PATHTRACER = 0, 3, 5  # MUONX_INTEGRATOR_*
 
 
 def _scene(ctx, integrator, w, h, spp):
@@ -51,4 +51,25 @@ def test_captured_render_replays(integrator, w, h, spp):
         torch.cuda.synchronize()
         assert torch.equal(acc, want), k
     again, _ = render_device(ds, p)  # and the context renders on as before
+    assert torch.equal(again, want)
+
+
+def test_captured_path_tracer_is_refused():
+    """Its loop runs on the host. The context renders on after the refusal, to the same bits."""
+    ctx = Context(0)
+    ds, p = _scene(ctx, PATHTRACER, 64, 48, 2)
+    want, _ = render_device(ds, p)
+    want = want.clone()
+    acc = torch.zeros_like(want)
+    marker = torch.zeros(1, device="cuda:0")
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        marker.add_(1.0)
+        rc = _lib.lib.muonx_render(ds.h, C.byref(p), acc.data_ptr(), None, torch.cuda.current_stream().cuda_stream)
+    assert rc == -5 and b"captured" in _lib.lib.muonx_last_error()
+    g.replay()
+    torch.cuda.synchronize()
+    assert marker.item() == 1.0 and not acc.any()
+    again, _ = render_device(ds, p)
     assert torch.equal(again, want)
